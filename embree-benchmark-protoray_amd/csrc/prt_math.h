@@ -346,19 +346,6 @@ PRT_HD bool plane_t(f3 p0, f3 p1, f3 p2, f3 o, f3 d, float& t_out)
     return true;
 }
 
-// Candidate intersection.  The watertight test decides whether the ray's line
-// crosses the triangle (fp32 edge functions, a zero one recomputed in
-// double); the hit distance is the plane distance of plane_t.  Returns false
-// for a miss, a plane parallel to the ray or a distance outside [tmin, tmax];
-// (V, W, det) are kept so that the caller computes u = V/det, v = W/det only
-// for accepted hits.  Ordering candidates by this t rather than by the fp32
-// T/det makes the choice of the nearest triangle follow the true distances,
-// and keeps the traversal's conservative box culling (slack relative to the
-// box distances) consistent with every candidate's t.
-struct TriCandidate {
-    float t, v_num, w_num, det;
-};
-
 // Scaled barycentrics U, V, W of p0, p1, p2 (the edge functions in the
 // ray's shear space); a zero one sends all three to double.
 PRT_HD void tri_edges(const WatertightRay& w, f3 org, f3 p0, f3 p1, f3 p2, float& U, float& V, float& W)
@@ -374,34 +361,40 @@ PRT_HD void tri_edges(const WatertightRay& w, f3 org, f3 p0, f3 p1, f3 p2, float
     U = cx * by - cy * bx;
     V = ax * cy - ay * cx;
     W = bx * ay - by * ax;
-    if (U == 0.0f || V == 0.0f || W == 0.0f) {
+    if (fminf(fminf(fabsf(U), fabsf(V)), fabsf(W)) == 0.0f) {
         U = (float)((double)cx * (double)by - (double)cy * (double)bx);
         V = (float)((double)ax * (double)cy - (double)ay * (double)cx);
         W = (float)((double)bx * (double)ay - (double)by * (double)ax);
     }
 }
 
+// Candidate intersection.  The watertight test decides whether the ray's line
+// crosses the triangle (fp32 edge functions, a zero one recomputed in
+// double); the hit distance is the plane distance of plane_t.  Returns false
+// for a miss, a plane parallel to the ray or a distance outside [tmin, tmax].
+// Ordering candidates by this t rather than by the fp32 T/det makes the choice
+// of the nearest triangle follow the true distances, and keeps the
+// traversal's conservative box culling (slack relative to the box distances)
+// consistent with every candidate's t.
 PRT_HD bool tri_test(const WatertightRay& w, f3 org, f3 dir, f3 p0, f3 p1, f3 p2, float tmin, float tmax,
-                     TriCandidate& c)
+                     float& t_out)
 {
     float U, V, W;
     tri_edges(w, org, p0, p1, p2, U, V, W);
-    if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
-    float det = (U + V) + W;
-    if (det == 0.0f) return false;
+    // signs differ (fminf and fmaxf pass over a NaN, as comparisons do)
+    const int mixed = (int)(fminf(fminf(U, V), W) < 0.0f) & (int)(fmaxf(fmaxf(U, V), W) > 0.0f);
+    const float det = (U + V) + W;
+    if (mixed | (int)(det == 0.0f)) return false;
     float t;
     if (!plane_t(p0, p1, p2, org, dir, t)) return false;
     if (!(t >= tmin && t <= tmax)) return false;
-    c.t = t;
-    c.v_num = V;
-    c.w_num = W;
-    c.det = det;
+    t_out = t;
     return true;
 }
 
 // Hit coordinates (u, v) = (V/det, W/det) of a triangle that tri_test
-// accepted for this ray, recomputed from the same edge functions (so equal to
-// what tri_test's caller derives from the candidate).
+// accepted for this ray, from the same edge functions: computed once for the
+// winner instead of for every accepted candidate.
 PRT_HD void tri_barycentrics(const WatertightRay& w, f3 org, f3 p0, f3 p1, f3 p2, float& u, float& v)
 {
     float U, V, W;
