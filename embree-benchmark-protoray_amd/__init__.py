@@ -362,8 +362,8 @@ class HipDevice:
                 "drainWaveSteps": st.drain_wave_steps, "drainLaneSteps": st.drain_lane_steps, "drainMs": st.drain_ms}
 
     def set_tail(self, mode: str = "cooperative") -> None:
-        """Tail of the fused diffuse frame: 'cooperative' (a wave with at most 8
-        paths left spreads each over 8 lanes) or 'lanes'."""
+        """Tail of the persistent launches: 'cooperative' (a wave with at most 8
+        rays or paths left spreads each over 8 lanes) or 'lanes'."""
         ids = {"lanes": 0, "cooperative": 1}
         if mode not in ids:
             raise ValueError("mode must be 'cooperative' or 'lanes'")

@@ -430,7 +430,7 @@ int prt_hip_intersect_closest_device_noalloc(prt_hip_ctx* ctx, const prt_ray* d_
         return set_error(ctx, "intersect_noalloc: a BVH of depth " + std::to_string(ctx->scene.bvh_depth) +
                                   " needs " + std::to_string(per_block) + " bytes of stack per workgroup, more than the " +
                                   std::to_string((size_t)PRT_HIP_NOALLOC_SCRATCH_BYTES) + "-byte scratch holds");
-    int grid = ctx->trace_per_cu * ctx->num_cus;
+    int grid = query_grid(ctx, n);
     if ((size_t)grid > blocks_fit) grid = (int)blocks_fit;
     uint32_t* hdr = static_cast<uint32_t*>(ctx->d_scratch);
     PRT_TRY(ctx, launch_zero_u32(hdr, 2, ctx->stream));  // a kernel, not a memset: safe under graph capture
@@ -729,7 +729,7 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
         key.height = ctx->height;
         key.max_depth = last;
         key.pass = ctx->pass;
-        key.grid = ctx->diffuse_grid;
+        key.grid = diffuse_grid(ctx, entries);
         std::memcpy(&key.albedo_bits, &albedo, sizeof(float));
     }
     const bool look_run = look_on && ctx->look_prev_on && look_follows(ctx->look_prev, key);
@@ -757,7 +757,6 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
         p.depth_rays = ctx->d_stats + 16;
         p.stats = ctx->d_stats;
         p.fast = fast;
-        p.coop = ctx->tail_coop;
         if (look_run) {
             // a call that keeps no earlier work skips kLookLevels tags, so no
             // side sample left by an earlier chain of calls carries its tag

@@ -191,8 +191,7 @@ struct prt_hip_ctx {
     // traversal spill stack (global part of the short stack)
     uint2* d_spill = nullptr;
     int64_t spill_bytes = 0;
-    int trace_grid = 0;        // persistent workgroups per trace launch
-    int diffuse_grid = 0;      // persistent workgroups per diffuse render launch (for the current scene)
+    int trace_grid = 0;        // most persistent workgroups of a trace launch
     int trace_per_cu = 0;      // occupancy limit of the persistent trace kernel, workgroups per CU
     int stack_entries = 0;     // max stack depth per lane (LDS + spill); only grows
     uint64_t spill_gen = 0;    // bumped whenever d_spill or stack_entries change
@@ -231,7 +230,7 @@ struct prt_hip_ctx {
     int64_t rgb_planes_cap = 0;      // ... in float4
     hipEvent_t kev[4 * 16] = {};    // per-launch timing events (trace/shade x begin/end)
 
-    // cooperative tail of the fused diffuse frame (prt_hip_set_tail)
+    // cooperative tail of the persistent launches (prt_hip_set_tail)
     int tail_coop = 1;
 
     // frame lookahead of the fused diffuse frame (prt_hip_set_lookahead)
@@ -331,8 +330,8 @@ struct PathLaunch {
     // the "Fast" renderers: frame of the geometric normal whatever attributes
     // the mesh has, and each pass overwrites the accumulator
     bool fast;
-    // diffuse frames: a wave with at most 8 paths left traces them
-    // cooperatively (0: never)
+    // a wave with at most 8 rays or paths left traces them cooperatively (0:
+    // never)
     int coop;
     // diffuse frames: frame lookahead (nullptr: off)
     LookState* look;
@@ -344,6 +343,10 @@ struct PathLaunch {
     uint32_t* look_flags; // per block (kLookFlagStride apart): look_gen once this frame is finished
 };
 int ensure_trace_resources(prt_hip_ctx* ctx);
+// persistent workgroups of a diffuse frame of `entries` path slots, and of a
+// closest-hit query of `rays` rays
+int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries);
+int query_grid(const prt_hip_ctx* ctx, int64_t rays);
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented);
 // closest-hit launch over `grid` persistent workgroups whose stack spill
 // (stack_entries per lane) and error flag the caller provides

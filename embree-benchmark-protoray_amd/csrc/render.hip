@@ -388,7 +388,7 @@ hipError_t launch_look_call_begin(prt_hip_ctx* ctx, bool valid, uint32_t entries
     const int grid = valid ? (n + kBlock - 1) / kBlock : 1;
     k_look_call_begin<<<grid, kBlock, 0, ctx->stream>>>(
         ctx->d_counters, entries, ctx->d_stats, ctx->d_look, entries, valid ? 1 : 0, ctx->look_q_cap,
-        (uint32_t)ctx->diffuse_grid * (uint32_t)(kTraceBlock / 64), ctx->d_look_side, ctx->d_accum, n,
+        (uint32_t)diffuse_grid(ctx, entries) * (uint32_t)(kTraceBlock / 64), ctx->d_look_side, ctx->d_accum, n,
         ctx->look_gen);
     return hipGetLastError();
 }

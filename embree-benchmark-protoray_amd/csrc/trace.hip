@@ -43,6 +43,9 @@
 // that the watertight test says the ray crosses with tnear <= t <= tfar, t
 // being the plane distance computed in double -- the same answer as testing
 // every triangle, whatever the visiting order.
+#include <algorithm>
+#include <type_traits>
+
 #include "prt_internal.h"
 
 namespace prt {
@@ -56,18 +59,48 @@ enum {
     kModeDiffuse2 = 6, kModeOccluded = 7
 };
 
-__device__ __forceinline__ float byte_f(uint32_t w, int k)
-{
-    return (float)((w >> (8 * k)) & 0xffu);
-}
-
 __device__ __forceinline__ float as_f(uint32_t u) { return __uint_as_float(u); }
 
-// kLook: the fused diffuse frame with the frame lookahead compiled in (and the
-// cooperative tail, which it never uses, left out); the plain variant is the
-// other way round, so each carries only the code it runs.
+// Minimum over the 8 lanes of an aligned group, in every lane of it: three
+// DPP steps (lane ^ 1, lane ^ 2, then the mirror of the 8 lanes, whose halves
+// hold one value each by then) instead of three trips through the LDS crossbar.
+__device__ __forceinline__ uint32_t dpp8(uint32_t v, int step)
+{
+    const int x = (int)v;
+    return (uint32_t)(step == 0 ? __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, true)
+                      : step == 1 ? __builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, true)
+                                  : __builtin_amdgcn_update_dpp(x, x, 0x141, 0xF, 0xF, true));
+}
+__device__ __forceinline__ uint32_t min8(uint32_t v)
+{
+    v = min(v, dpp8(v, 0));
+    v = min(v, dpp8(v, 1));
+    return min(v, dpp8(v, 2));
+}
+__device__ __forceinline__ uint32_t or8(uint32_t v)
+{
+    v |= dpp8(v, 0);
+    v |= dpp8(v, 1);
+    return v | dpp8(v, 2);
+}
+
+// Position of the r-th (from 0) set bit of m, which has more than r.
+__device__ __forceinline__ uint32_t nth_bit(uint32_t m, uint32_t r)
+{
+    uint32_t pos = 0;
+#pragma unroll
+    for (int w = 16; w >= 1; w >>= 1) {
+        const uint32_t c = (uint32_t)__popc((m >> pos) & ((1u << w) - 1u));
+        const bool up = r >= c;
+        pos += up ? (uint32_t)w : 0u;
+        r -= up ? c : 0u;
+    }
+    return pos;
+}
+
+// kLook: the fused diffuse frame with the frame lookahead compiled in.
 template <bool kCount, int kMode, int kBlock = kTraceBlock, int kStack = kStackLds, bool kLook = false>
-__global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl, PathLaunch pl, BatchLaunch bl,
+__global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoint ? 4 : 1) void k_trace(SceneDevice sc, TraceLaunch tl, PathLaunch pl, BatchLaunch bl,
                                                   uint2* spill, int stack_entries, int refill, uint32_t* err)
 {
     static_assert((kStack & (kStack - 1)) == 0, "LDS stack depth must be a power of two");
@@ -143,7 +176,6 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
     float gw_r = 0.0f, gw_g = 0.0f, gw_b = 0.0f;
     bool replay = false;
     int path_pass = 0;
-    int path_x = 0, path_y = 0;
     // diffuse2: the current ray is a shadow ray; the path's next ray waits in
     // (eo, ed); radiance gathered so far
     bool shadow = false;
@@ -154,12 +186,15 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
     unsigned long long n_dwsteps = 0, n_dlsteps = 0;              // ... after the work ran out
     unsigned long long t_exhausted = 0;                           // wall clock when it ran out
     bool exhausted = false;  // wave-uniform: the work counter has run past count
-    // Tail of a diffuse frame (kModeDiffuse): once out of work with at most
-    // 8 paths left, the wave traces them cooperatively, 8 lanes per path
-    // (see the cooperative phase after the main loop)
-    constexpr bool kCoop = kMode == kModeDiffuse && !kLook;
+    // Cooperative traversal of a wave's last paths (see coop_traverse below)
+    constexpr bool kCoop = !kLook;
     const bool coop_on = kCoop && pl.coop != 0;
-    bool cont = false;  // the path's next ray waits in (o, d) for the cooperative phase
+    uint64_t coop_paths = 0;                 // lanes whose paths the wave goes on with in groups
+    const int gj = lane & 7;                 // this lane's place in its group
+    const int gbase = lane & ~7;             // first lane of the group
+    constexpr int kGStack = 8 * kStack;      // a group's stack: its lanes' LDS rings joined
+    uint2* const g_spill = spill + ((size_t)blockIdx.x * kBlock + (tid & ~7)) * (size_t)stack_entries;
+    auto group_slot = [&](int q) -> int { return ((q >> 3) & (kStack - 1)) * kBlock + (tid & ~7) + (q & 7); };
 
     // Frame lookahead (kModeDiffuse, LookState); a path of frame pass + l is
     // at level l.  This frame's space, from LookState::counter: [0, F) are
@@ -178,7 +213,6 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
     //  - After the stop no more items are taken, and paths of later frames
     //    leave for the queue of their level: at a bounce, or in the middle
     //    of a ray, which the next call then traces again from its origin.
-    //  - The cooperative tail is off under the lookahead.
     constexpr bool kLookMode = kMode == kModeDiffuse && kLook;
     LookState* const look = kLookMode ? pl.look : nullptr;
     uint32_t lk_F = 0, lk_fresh_end = 0, lk_target = 0;
@@ -264,6 +298,471 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
         return make_frame(face_normal(p0, p1, p2, d));
     };
 
+    // Shades the lanes whose ray has finished (active, not tracing).  lead: the
+    // lane counts and writes for its path (in a cooperative wave, a group's
+    // first lane).
+    auto shade = [&](bool lead) __attribute__((always_inline)) {
+        if (kCount && __ballot(active && !tracing) != 0 && lane == 0) ++n_wshade;
+        if (active && !tracing) do {
+            if (kMode == kModeOccluded) {
+                if (lead) tl.any_t[ray_idx] = best_prim >= 0 ? tbest : -1.0f;
+                active = false;
+                break;
+            }
+            if (kMode == kModeDiffuse2 && shadow) {
+                // shadow ray done: light from the sky unless blocked (MIS weight 1/2)
+                if constexpr (kCount) { if (lead) atomicAdd(&depth_hist[min(depth, kMaxQueueDepth - 1)], 1u); }
+                n_rays += lead ? 1u : 0u;
+                if (best_prim < 0) lsum += lw * 0.5f;
+                shadow = false;
+                start_ray(eo, ed, 0.0f, 3.402823466e38f);
+                break;
+            }
+            float t = -1.0f;
+            f3 p0{}, p1{}, p2{};
+            if (best_prim >= 0) {
+                const PRT_GLOBAL float* tp = tris + 9 * (size_t)best_rec;
+                p0 = mk3(tp[0], tp[1], tp[2]);
+                p1 = mk3(tp[3], tp[4], tp[5]);
+                p2 = mk3(tp[6], tp[7], tp[8]);
+                t = tbest;  // plane distance of the winner (tri_test)
+            }
+            if (kMode == kModeTrace) {
+                float bu = 0.0f, bv = 0.0f;
+                if (best_prim >= 0) tri_barycentrics(wr, o, p0, p1, p2, bu, bv);
+                if (lead)
+                    tl.hits[ray_idx] = best_prim >= 0
+                                           ? make_float4(t, __int_as_float(best_prim), bu, bv)
+                                           : make_float4(-1.0f, __int_as_float(-1), 0.0f, 0.0f);
+                active = false;
+                break;
+            }
+            if constexpr (kCount && kMode != kModeBatch) { if (lead) atomicAdd(&depth_hist[min(depth, kMaxQueueDepth - 1)], 1u); }
+            if (kLookMode && level > 0) {
+#pragma unroll
+                for (int l = 1; l <= kLookLevels; ++l)
+                    if (level == l && lead) ++n_ahead[l - 1];
+            } else {
+                n_rays += lead ? 1u : 0u;
+            }
+            float4* acc = kMode == kModeBatch ? nullptr : pl.accum + pixel;
+            if (kMode == kModeDiffuse2) {
+                // extension ray done (render/diffuse2_integrator_single.h:52-85)
+                bool done = false;
+                if (best_prim < 0) {
+                    lsum += lw * (depth > 0 ? 0.5f : 1.0f);
+                    done = true;
+                } else if (depth == max_depth) {
+                    done = true;
+                }
+                if (done) {
+                    const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
+                    if (lead) *acc = make_float4(a.x + lsum, a.y + lsum, a.z + lsum, a.w + 1.0f);
+                    active = false;
+                    break;
+                }
+                lw *= albedo;
+                const Frame fr = hit_frame(p0, p1, p2);
+                const float s1 = sampler_next(rng);
+                const float s2 = sampler_next(rng);
+                const float s3 = sampler_next(rng);
+                const float s4 = sampler_next(rng);
+                f3 so, sd;
+                diffuse_bounce(o, d, t, fr, s1, s2, so, sd);
+                diffuse_bounce(o, d, t, fr, s3, s4, eo, ed);
+                ++depth;
+                shadow = true;
+                start_ray(so, sd, 0.0f, 3.402823466e38f);
+                break;
+            }
+            if (kMode == kModePrimary) {
+                f3 c = mk3(0.05f, 0.05f, 0.05f);
+                if (best_prim >= 0) {
+                    const f3 n = hit_frame(p0, p1, p2).n;
+                    c = mk3((n.x + 1.0f) * 0.5f, (n.y + 1.0f) * 0.5f, (n.z + 1.0f) * 0.5f);
+                }
+                const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
+                if (lead) *acc = make_float4(a.x + c.x, a.y + c.y, a.z + c.z, a.w + 1.0f);
+                active = false;
+                break;
+            }
+            if (best_prim < 0 || depth == max_depth) {
+                if (kMode == kModeAdjoint) {
+                    if (!replay && best_prim < 0) {
+                        // the path escaped: replay it from its seed to
+                        // hand each hit its share of the gradient
+                        replay = true;
+                        rng = sampler_seed(path_pass, pixel);
+                        const float u1 = sampler_next(rng);
+                        const float u2 = sampler_next(rng);
+                        const float l1 = sampler_next(rng);
+                        const float l2 = sampler_next(rng);
+                        f3 org, dir;
+                        const int y = pixel / pl.width, x = pixel - y * pl.width;
+                        camera_ray(pl.cam, ((float)x + u1) * pl.inv_w, ((float)y + u2) * pl.inv_h, l1, l2, org, dir);
+                        depth = 0;
+                        start_ray(org, dir, 0.0f, 3.402823466e38f);
+                        continue;
+                    }
+                    active = false;
+                    break;
+                }
+                const float c = best_prim < 0 ? lw : 0.0f;
+                if (kMode == kModeBatch) {
+                    if (lead) *sample_out = c;
+                } else if (kMode == kModeRgb) {
+                    const float cg = best_prim < 0 ? lg : 0.0f, cb = best_prim < 0 ? lb : 0.0f;
+                    if (pl.rgb_planes) {
+                        // one plane per sample; they are added in pass order afterwards
+                        if (lead)
+                            pl.rgb_planes[(size_t)(path_pass - pl.pass) * (size_t)(pl.width * pl.height) + pixel] =
+                                make_float4(c, cg, cb, 0.0f);
+                    } else {
+                        const float4 a = *acc;
+                        if (lead) *acc = make_float4(a.x + c, a.y + cg, a.z + cb, a.w + 1.0f);
+                    }
+                } else if (kLookMode && level > 0) {
+                    // a later frame's sample, for the call whose tag it carries
+                    const uint32_t tag = pl.look_gen + (uint32_t)level;
+                    if (lead)
+                        pl.side[(size_t)(tag % (uint32_t)kLookLevels) * (size_t)(pl.width * pl.height) + pixel] =
+                            make_uint2(__float_as_uint(c), tag);
+                } else {
+                    const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
+                    if (lead) *acc = make_float4(a.x + c, a.y + c, a.z + c, a.w + 1.0f);
+                }
+                active = false;
+                break;
+            }
+            // diffuse bounce: the next ray of this path
+            if (kMode == kModeRgb || kMode == kModeAdjoint) {
+                const float* a = pl.albedo_rgb + 3 * (size_t)best_prim;
+                const float ar = a[0], ag = a[1], ab = a[2];
+                if (kMode == kModeAdjoint) {
+                    if (!replay) {
+                        // primal: products of the nonzero albedos, zero counts
+                        if (ar != 0.0f) pr *= ar; else zeros += 1u;
+                        if (ag != 0.0f) pg *= ag; else zeros += 1u << 8;
+                        if (ab != 0.0f) pb *= ab; else zeros += 1u << 16;
+                    } else {
+                        // dL_c/da_c(t) = product of the path's other albedos
+                        float* g = pl.grad + 3 * (size_t)best_prim;
+                        const uint32_t zr = zeros & 0xffu, zg = (zeros >> 8) & 0xffu, zb = zeros >> 16;
+                        const float dr = zr == 0 ? pr / ar : (zr == 1 && ar == 0.0f ? pr : 0.0f);
+                        const float dg = zg == 0 ? pg / ag : (zg == 1 && ag == 0.0f ? pg : 0.0f);
+                        const float db = zb == 0 ? pb / ab : (zb == 1 && ab == 0.0f ? pb : 0.0f);
+                        if (lead && gw_r * dr != 0.0f) atomicAdd(g + 0, gw_r * dr);
+                        if (lead && gw_g * dg != 0.0f) atomicAdd(g + 1, gw_g * dg);
+                        if (lead && gw_b * db != 0.0f) atomicAdd(g + 2, gw_b * db);
+                    }
+                } else {
+                    lw *= ar;
+                    lg *= ag;
+                    lb *= ab;
+                }
+            } else {
+                lw *= albedo;
+            }
+            const Frame fr = hit_frame(p0, p1, p2);
+            const float s1 = sampler_next(rng);
+            const float s2 = sampler_next(rng);
+            f3 no, nd;
+            diffuse_bounce(o, d, t, fr, s1, s2, no, nd);
+            ++depth;
+            if (kLookMode && level > 0 && stop) {
+                o = no;
+                d = nd;
+                suspend = true;
+                active = false;
+                break;
+            }
+            start_ray(no, nd, 0.0f, 3.402823466e38f);
+        } while (0);
+    };
+
+    // ---- cooperative traversal.  A wave out of work that holds at most 8
+    // paths moves each, in the middle of its ray or between rays, to a group
+    // of 8 lanes that hold its state alike.  Per step, lane j of a group tests
+    // one of up to 8 pending triangles, then child j of the group's node; the
+    // nearest children and the closest hit come from DPP minima inside the
+    // group (no trip through the LDS crossbar).  A step then issues about a
+    // third of the lane-by-lane instructions and tests up to 8 triangles at
+    // once, so the dependent steps of the last paths, which set a launch's
+    // end, follow each other faster.  The closest hit is the same (t, primId)
+    // minimum in any order, so hits and images do not change.  8 lanes: a
+    // group's lanes are the node's children.  Plain frames with it and lane by
+    // lane: 1080p spheres 1.199 / 1.285 ms, 720p of 0.4 M triangles 1.146 /
+    // 1.283 ms, next-event frames of 717x405 0.937 / 0.986 ms (4 workgroups
+    // per CU on all).
+    auto to_groups = [&](uint64_t paths) {
+        const int npaths = __popcll(paths);
+        const int grp = lane >> 3;
+        uint64_t mm = paths;
+        for (int k = 0; k < grp; ++k) mm &= mm - 1;
+        const int src = mm ? __ffsll((unsigned long long)mm) - 1 : 0;
+        auto mv_u = [&](uint32_t v) -> uint32_t { return (uint32_t)__shfl((int)v, src, 64); };
+        auto mv_i = [&](int& v) { v = __shfl(v, src, 64); };
+        auto mv_w = [&](uint32_t& v) { v = mv_u(v); };
+        auto mv_f = [&](float& v) { v = __shfl(v, src, 64); };
+        auto mv_3 = [&](f3& v) { mv_f(v.x); mv_f(v.y); mv_f(v.z); };
+        auto mv_b = [&](bool& v) { v = __shfl(v ? 1 : 0, src, 64) != 0; };
+        auto mv_p = [&](auto& v) {
+            uint64_t u = (uint64_t)v;
+            u = (uint64_t)mv_u((uint32_t)u) | ((uint64_t)mv_u((uint32_t)(u >> 32)) << 32);
+            v = (std::remove_reference_t<decltype(v)>)u;
+        };
+        mv_i(sp);
+        // the ray's stack (all in LDS: bottom is 0, so at most kStack entries):
+        // read by the group's lanes, then written in the joined order
+        const int stid = (tid & ~63) + src;
+        uint32_t en[kStack / 8], et[kStack / 8];
+#pragma unroll
+        for (int r = 0; r < kStack / 8; ++r) {
+            const int at = (8 * r + gj) * kBlock + stid;
+            en[r] = st_node[at];
+            et[r] = __float_as_uint(st_t[at]);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < kStack / 8; ++r) {
+            st_node[group_slot(8 * r + gj)] = en[r];
+            st_t[group_slot(8 * r + gj)] = as_f(et[r]);
+        }
+        mv_b(active);
+        mv_b(tracing);
+        mv_3(o);
+        mv_3(d);
+        mv_f(tmin);
+        mv_f(tbest);
+        mv_f(inv_x);
+        mv_f(inv_y);
+        mv_f(inv_z);
+        neg_x = inv_x < 0.0f;
+        neg_y = inv_y < 0.0f;
+        neg_z = inv_z < 0.0f;
+        mv_i(wr.kx);
+        mv_i(wr.ky);
+        mv_i(wr.kz);
+        mv_f(wr.sx);
+        mv_f(wr.sy);
+        mv_f(wr.sz);
+        mv_i(best_prim);
+        mv_w(best_rec);
+        mv_i(node);
+        mv_f(node_t);
+        mv_w(pend);
+        mv_w(pend_base);
+        mv_w(pend2);
+        mv_w(pend2_base);
+        if constexpr (kRayQuery) {
+            mv_w(ray_idx);
+        } else {
+            mv_i(pixel);
+            mv_w(rng);
+            mv_i(depth);
+            mv_f(lw);
+        }
+        if constexpr (kLookMode) mv_i(level);
+        if constexpr (kMode == kModeBatch) {
+            mv_i(max_depth);
+            mv_f(albedo);
+            mv_i(scene_id);
+            mv_p(nodes);
+            mv_p(tris);
+            mv_p(prim_ids);
+            mv_p(sample_out);
+        }
+        if constexpr (kMode == kModeRgb || kMode == kModeAdjoint) {
+            mv_f(lg);
+            mv_f(lb);
+            mv_i(path_pass);
+        }
+        if constexpr (kMode == kModeAdjoint) {
+            mv_f(pr);
+            mv_f(pg);
+            mv_f(pb);
+            mv_w(zeros);
+            mv_f(gw_r);
+            mv_f(gw_g);
+            mv_f(gw_b);
+            mv_b(replay);
+        }
+        if constexpr (kMode == kModeDiffuse2) {
+            mv_b(shadow);
+            mv_3(eo);
+            mv_3(ed);
+            mv_f(lsum);
+        }
+        if (grp >= npaths) active = tracing = false;
+    };
+
+    // Traverses the groups' rays until half of the `groups` with a path wait
+    // for shading.
+    auto coop_traverse = [&](int groups) {
+        const int keep = groups - max(1, groups >> 1);
+        for (;;) {
+            const int left = __popcll(__ballot(tracing)) >> 3;
+            if (left <= keep) break;
+            if (kCount) {
+                if (tracing) {
+                    ++n_lsteps;
+                    ++n_dlsteps;
+                }
+                if (lane == 0) {
+                    ++n_wsteps;
+                    ++n_dwsteps;
+                }
+            }
+            if (tracing && pend != 0) {
+                // up to 8 pending triangles, one per lane
+                const int np = __popc(pend);
+                uint32_t cp = ~0u, crec = 0;
+                float hit_t = __builtin_inff();
+                if (gj < np) {
+                    const uint32_t rec = pend_base + nth_bit(pend, (uint32_t)gj);
+                    const PRT_GLOBAL float* tp = tris + 9 * (size_t)rec;
+                    const f3 p0 = mk3(tp[0], tp[1], tp[2]);
+                    const f3 p1 = mk3(tp[3], tp[4], tp[5]);
+                    const f3 p2 = mk3(tp[6], tp[7], tp[8]);
+                    if (kCount) ++n_tris;
+                    if (tri_test(wr, o, d, p0, p1, p2, tmin, tbest, hit_t)) {
+                        cp = (uint32_t)prim_ids[rec];
+                        crec = rec;
+                    }
+                }
+                if (np <= 8) {
+                    pend = pend2;
+                    pend_base = pend2_base;
+                    pend2 = 0;
+                } else {
+                    pend &= ~0u << nth_bit(pend, 8);
+                }
+                if (__ballot(cp != ~0u) != 0) {
+                    // the smallest (t, primId): floats ordered as unsigned
+                    // integers (t is negative only where tnear is; -0 as +0)
+                    const uint32_t tb = __float_as_uint(hit_t + 0.0f);
+                    const uint32_t ct = cp != ~0u ? tb ^ (tb >> 31 ? 0xffffffffu : 0x80000000u) : ~0u;
+                    const uint32_t mt = min8(ct);
+                    const uint32_t mp = min8(ct == mt ? cp : ~0u);
+                    if (mp != ~0u) {
+                        const bool won = ct == mt && cp == mp;
+                        const float t = __uint_as_float(or8(won ? __float_as_uint(hit_t) : 0u));
+                        const uint32_t mr = or8(won ? crec : 0u);
+                        if (kMode == kModeOccluded || (kMode == kModeDiffuse2 && shadow)) {
+                            // any hit ends the query
+                            tbest = t;
+                            best_prim = 0;
+                            sp = bottom = 0;
+                            pend = pend2 = 0;
+                            node = -1;
+                        } else if (t < tbest || best_prim < 0 || (int32_t)mp < best_prim) {
+                            tbest = t;
+                            best_prim = (int32_t)mp;
+                            best_rec = mr;
+                        }
+                    }
+                }
+            }
+            if (tracing && pend == 0) {
+                if (node >= 0 && node_t > tbest) node = -1;
+                while (node < 0 && sp > 0) {
+                    // the 8 youngest entries at once: the topmost that can
+                    // still hold a closer hit
+                    const int q = sp - 1 - gj;
+                    uint32_t nid = 0;
+                    float nt = __builtin_inff();
+                    if (q >= bottom) {
+                        const int slot = group_slot(q);
+                        nid = st_node[slot];
+                        nt = st_t[slot];
+                    } else if (q >= 0) {
+                        const uint2 e = g_spill[q];
+                        nid = e.x;
+                        nt = as_f(e.y);
+                    }
+                    const uint32_t ok = (uint32_t)(__ballot(q >= 0 && nt <= tbest) >> gbase) & 0xffu;
+                    if (ok == 0) {
+                        sp = max(sp - 8, 0);
+                    } else {
+                        const int f = __builtin_ctz(ok);
+                        node = __shfl((int)nid, gbase + f, 64);
+                        node_t = __shfl(nt, gbase + f, 64);
+                        sp -= f + 1;
+                    }
+                    bottom = min(bottom, sp);
+                }
+                if (node < 0) tracing = false;
+            }
+            if (tracing && pend == 0) {
+                // ---- child gj of the group's node
+                const PRT_GLOBAL uint8_t* nb = reinterpret_cast<const PRT_GLOBAL uint8_t*>(nodes + node);
+                const PRT_GLOBAL uint4* np = reinterpret_cast<const PRT_GLOBAL uint4*>(nb);
+                const uint4 w0 = np[0];
+                const uint2 base = reinterpret_cast<const PRT_GLOBAL uint2*>(nb)[2];
+                const uint32_t mb = nb[24 + gj];
+                const PRT_GLOBAL uint8_t* qb = nb + 32 + gj;
+                const float qnx = (float)qb[neg_x ? 24 : 0], qfx = (float)qb[neg_x ? 0 : 24];
+                const float qny = (float)qb[neg_y ? 32 : 8], qfy = (float)qb[neg_y ? 8 : 32];
+                const float qnz = (float)qb[neg_z ? 40 : 16], qfz = (float)qb[neg_z ? 16 : 40];
+                if (kCount && gj == 0) ++n_nodes;
+                const float ax = __builtin_amdgcn_ldexpf(inv_x, (int)(int8_t)(w0.w & 0xffu));
+                const float ay = __builtin_amdgcn_ldexpf(inv_y, (int)(int8_t)((w0.w >> 8) & 0xffu));
+                const float az = __builtin_amdgcn_ldexpf(inv_z, (int)(int8_t)((w0.w >> 16) & 0xffu));
+                const uint32_t imask = w0.w >> 24;
+                const float bx = (as_f(w0.x) - o.x) * inv_x;
+                const float by = (as_f(w0.y) - o.y) * inv_y;
+                const float bz = (as_f(w0.z) - o.z) * inv_z;
+                // slack 2^-21 (255 |a| + |b|): the roundings of b, b -/+ slack
+                // and the fma, the reciprocal's ulp and the hit distance's
+                // rounding sum to at most 2^-21 (128 |a| + |b|)
+                const float slx = 0x1p-21f * __builtin_fmaf(255.0f, fabsf(ax), fabsf(bx));
+                const float sly = 0x1p-21f * __builtin_fmaf(255.0f, fabsf(ay), fabsf(by));
+                const float slz = 0x1p-21f * __builtin_fmaf(255.0f, fabsf(az), fabsf(bz));
+                const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(qnx, ax, bx - slx), __builtin_fmaf(qny, ay, by - sly)),
+                                             __builtin_fmaf(qnz, az, bz - slz)), tmin);
+                const float tf = fminf(fminf(fminf(__builtin_fmaf(qfx, ax, bx + slx), __builtin_fmaf(qfy, ay, by + sly)),
+                                             __builtin_fmaf(qfz, az, bz + slz)), tbest);
+                const bool hit = tn <= tf;
+                const bool inner = ((imask >> gj) & 1u) != 0;
+                // leaf slots: one pending mask over the node's records
+                pend = or8(hit && !inner ? ((1u << (mb >> 5)) - 1u) << (mb & 31u) : 0u);
+                pend_base = base.y;
+                // nearest internal child next, the others pushed by slot with
+                // the second nearest on top (keys as lane by lane)
+                const uint32_t key = hit && inner ? (__float_as_uint(tn) & 0x7ffffff8u) | (uint32_t)gj : ~0u;
+                const uint32_t m1 = min8(key);
+                const uint32_t m2 = min8(key == m1 ? ~0u : key);
+                node = -1;
+                if (m1 != ~0u) {
+                    node = (int32_t)(base.x + __popc(imask & ((1u << (m1 & 7u)) - 1u)));
+                    node_t = __uint_as_float(m1 & ~7u);
+                    const bool push = key != ~0u && key != m1;
+                    const uint32_t pm = (uint32_t)(__ballot(push && key != m2) >> gbase) & 0xffu;
+                    if (m2 != ~0u) {
+                        const int npush = __popc(pm) + 1;
+                        bool room = true;
+                        while (sp + npush - bottom > kGStack) {
+                            if (bottom >= spill_cap) { if (gj == 0) atomicOr(err, 1u); room = false; break; }
+                            const int bs = group_slot(bottom);
+                            g_spill[bottom] = make_uint2(st_node[bs], __float_as_uint(st_t[bs]));
+                            ++bottom;
+                            if (kCount && gj == 0) ++n_spill;
+                        }
+                        if (room) {
+                            if (push) {
+                                const int at = sp + (key == m2 ? npush - 1 : __popc(pm & ((1u << gj) - 1u)));
+                                const int slot = group_slot(at);
+                                st_node[slot] = base.x + __popc(imask & ((1u << gj) - 1u));
+                                st_t[slot] = tn;
+                            }
+                            sp += npush;
+                        }
+                    }
+                }
+            }
+        }
+    };
+
     for (;;) {
         // lookahead: a wave that holds paths of this frame takes no items of
         // later frames once this frame's are handed out, and issues ahead of
@@ -289,196 +788,10 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
             if (hold) __builtin_amdgcn_s_setprio(3);
             else __builtin_amdgcn_s_setprio(0);
         }
-        // the wave goes cooperative once out of work, with at most 8 paths
-        // left and all of them between rays
-        bool go_coop = false;
-        if (coop_on && exhausted) {
-            const uint64_t a = __ballot(active);
-            go_coop = a != 0 && __popcll(a) <= 8 && __ballot(active && tracing) == 0;
-        }
-        // ---- shade the lanes whose ray has finished.  The traversal loop
-        // hands them over in groups, so this code runs for many lanes at once
-        // instead of stalling every traversal step of the wave for one lane.
-        if (kCount && __ballot(active && !tracing) != 0 && lane == 0) ++n_wshade;
-        if (active && !tracing) do {
-            if (kMode == kModeOccluded) {
-                tl.any_t[ray_idx] = best_prim >= 0 ? tbest : -1.0f;
-                active = false;
-                break;
-            }
-            if (kMode == kModeDiffuse2 && shadow) {
-                // shadow ray done: light from the sky unless blocked (MIS weight 1/2)
-                if constexpr (kCount) atomicAdd(&depth_hist[min(depth, kMaxQueueDepth - 1)], 1u);
-                ++n_rays;
-                if (best_prim < 0) lsum += lw * 0.5f;
-                shadow = false;
-                start_ray(eo, ed, 0.0f, 3.402823466e38f);
-                break;
-            }
-            float t = -1.0f;
-            f3 p0{}, p1{}, p2{};
-            if (best_prim >= 0) {
-                const PRT_GLOBAL float* tp = tris + 9 * (size_t)best_rec;
-                p0 = mk3(tp[0], tp[1], tp[2]);
-                p1 = mk3(tp[3], tp[4], tp[5]);
-                p2 = mk3(tp[6], tp[7], tp[8]);
-                t = tbest;  // plane distance of the winner (tri_test)
-            }
-            if (kMode == kModeTrace) {
-                float bu = 0.0f, bv = 0.0f;
-                if (best_prim >= 0) tri_barycentrics(wr, o, p0, p1, p2, bu, bv);
-                tl.hits[ray_idx] = best_prim >= 0
-                                       ? make_float4(t, __int_as_float(best_prim), bu, bv)
-                                       : make_float4(-1.0f, __int_as_float(-1), 0.0f, 0.0f);
-                active = false;
-                break;
-            }
-            if constexpr (kCount && kMode != kModeBatch) atomicAdd(&depth_hist[min(depth, kMaxQueueDepth - 1)], 1u);
-            if (kLookMode && level > 0) {
-#pragma unroll
-                for (int l = 1; l <= kLookLevels; ++l)
-                    if (level == l) ++n_ahead[l - 1];
-            } else {
-                ++n_rays;
-            }
-            float4* acc = kMode == kModeBatch ? nullptr : pl.accum + pixel;
-            if (kMode == kModeDiffuse2) {
-                // extension ray done (render/diffuse2_integrator_single.h:52-85)
-                bool done = false;
-                if (best_prim < 0) {
-                    lsum += lw * (depth > 0 ? 0.5f : 1.0f);
-                    done = true;
-                } else if (depth == max_depth) {
-                    done = true;
-                }
-                if (done) {
-                    const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
-                    *acc = make_float4(a.x + lsum, a.y + lsum, a.z + lsum, a.w + 1.0f);
-                    active = false;
-                    break;
-                }
-                lw *= albedo;
-                const Frame fr = hit_frame(p0, p1, p2);
-                const float s1 = sampler_next(rng);
-                const float s2 = sampler_next(rng);
-                const float s3 = sampler_next(rng);
-                const float s4 = sampler_next(rng);
-                f3 so, sd;
-                diffuse_bounce(o, d, t, fr, s1, s2, so, sd);
-                diffuse_bounce(o, d, t, fr, s3, s4, eo, ed);
-                ++depth;
-                shadow = true;
-                start_ray(so, sd, 0.0f, 3.402823466e38f);
-                break;
-            }
-            if (kMode == kModePrimary) {
-                f3 c = mk3(0.05f, 0.05f, 0.05f);
-                if (best_prim >= 0) {
-                    const f3 n = hit_frame(p0, p1, p2).n;
-                    c = mk3((n.x + 1.0f) * 0.5f, (n.y + 1.0f) * 0.5f, (n.z + 1.0f) * 0.5f);
-                }
-                const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
-                *acc = make_float4(a.x + c.x, a.y + c.y, a.z + c.z, a.w + 1.0f);
-                active = false;
-                break;
-            }
-            if (best_prim < 0 || depth == max_depth) {
-                if (kMode == kModeAdjoint) {
-                    if (!replay && best_prim < 0) {
-                        // the path escaped: replay it from its seed to
-                        // hand each hit its share of the gradient
-                        replay = true;
-                        rng = sampler_seed(path_pass, pixel);
-                        const float u1 = sampler_next(rng);
-                        const float u2 = sampler_next(rng);
-                        const float l1 = sampler_next(rng);
-                        const float l2 = sampler_next(rng);
-                        f3 org, dir;
-                        camera_ray(pl.cam, ((float)path_x + u1) * pl.inv_w, ((float)path_y + u2) * pl.inv_h,
-                                   l1, l2, org, dir);
-                        depth = 0;
-                        start_ray(org, dir, 0.0f, 3.402823466e38f);
-                        continue;
-                    }
-                    active = false;
-                    break;
-                }
-                const float c = best_prim < 0 ? lw : 0.0f;
-                if (kMode == kModeBatch) {
-                    *sample_out = c;
-                } else if (kMode == kModeRgb) {
-                    const float cg = best_prim < 0 ? lg : 0.0f, cb = best_prim < 0 ? lb : 0.0f;
-                    if (pl.rgb_planes) {
-                        // one plane per sample; they are added in pass order afterwards
-                        pl.rgb_planes[(size_t)(path_pass - pl.pass) * (size_t)(pl.width * pl.height) + pixel] =
-                            make_float4(c, cg, cb, 0.0f);
-                    } else {
-                        const float4 a = *acc;
-                        *acc = make_float4(a.x + c, a.y + cg, a.z + cb, a.w + 1.0f);
-                    }
-                } else if (kLookMode && level > 0) {
-                    // a later frame's sample, for the call whose tag it carries
-                    const uint32_t tag = pl.look_gen + (uint32_t)level;
-                    pl.side[(size_t)(tag % (uint32_t)kLookLevels) * (size_t)(pl.width * pl.height) + pixel] =
-                        make_uint2(__float_as_uint(c), tag);
-                } else {
-                    const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
-                    *acc = make_float4(a.x + c, a.y + c, a.z + c, a.w + 1.0f);
-                }
-                active = false;
-                break;
-            }
-            // diffuse bounce: the next ray of this path
-            if (kMode == kModeRgb || kMode == kModeAdjoint) {
-                const float* a = pl.albedo_rgb + 3 * (size_t)best_prim;
-                const float ar = a[0], ag = a[1], ab = a[2];
-                if (kMode == kModeAdjoint) {
-                    if (!replay) {
-                        // primal: products of the nonzero albedos, zero counts
-                        if (ar != 0.0f) pr *= ar; else zeros += 1u;
-                        if (ag != 0.0f) pg *= ag; else zeros += 1u << 8;
-                        if (ab != 0.0f) pb *= ab; else zeros += 1u << 16;
-                    } else {
-                        // dL_c/da_c(t) = product of the path's other albedos
-                        float* g = pl.grad + 3 * (size_t)best_prim;
-                        const uint32_t zr = zeros & 0xffu, zg = (zeros >> 8) & 0xffu, zb = zeros >> 16;
-                        const float dr = zr == 0 ? pr / ar : (zr == 1 && ar == 0.0f ? pr : 0.0f);
-                        const float dg = zg == 0 ? pg / ag : (zg == 1 && ag == 0.0f ? pg : 0.0f);
-                        const float db = zb == 0 ? pb / ab : (zb == 1 && ab == 0.0f ? pb : 0.0f);
-                        if (gw_r * dr != 0.0f) atomicAdd(g + 0, gw_r * dr);
-                        if (gw_g * dg != 0.0f) atomicAdd(g + 1, gw_g * dg);
-                        if (gw_b * db != 0.0f) atomicAdd(g + 2, gw_b * db);
-                    }
-                } else {
-                    lw *= ar;
-                    lg *= ag;
-                    lb *= ab;
-                }
-            } else {
-                lw *= albedo;
-            }
-            const Frame fr = hit_frame(p0, p1, p2);
-            const float s1 = sampler_next(rng);
-            const float s2 = sampler_next(rng);
-            f3 no, nd;
-            diffuse_bounce(o, d, t, fr, s1, s2, no, nd);
-            ++depth;
-            if (kLookMode && level > 0 && stop) {
-                o = no;
-                d = nd;
-                suspend = true;
-                active = false;
-                break;
-            }
-            if (kCoop && go_coop) {
-                o = no;
-                d = nd;
-                cont = true;
-                break;
-            }
-            start_ray(no, nd, 0.0f, 3.402823466e38f);
-        } while (0);
-        if (kCoop && go_coop) break;
+        // ---- shade the lanes whose ray has finished: the traversal loop hands
+        // them over in groups, so this code runs for many lanes at once
+        // instead of stalling every traversal step of the wave for one lane
+        shade(true);
 
         // ---- lookahead: queue the later frames' paths that stopped, by level
         if (kLookMode && look && __ballot(suspend) != 0) {
@@ -624,8 +937,6 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
                         const int y = (int)(tile / (uint32_t)pl.tiles_x) * 8 + my_;
                         if (x < pl.width && y < pl.height) {
                             pixel = x + y * pl.width;
-                            path_x = x;
-                            path_y = y;
                             rng = sampler_seed(path_pass, pixel);
                             const float u1 = sampler_next(rng);
                             const float u2 = sampler_next(rng);
@@ -669,13 +980,17 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
             if (exhausted) break;
             continue;
         }
+        if (kCoop && coop_on && exhausted && __popcll(busy) <= 8 && __ballot(active && bottom != 0) == 0) {
+            coop_paths = busy;
+            break;
+        }
 
         // ---- traverse until enough lanes wait for shading or for new work:
         // refill lanes once no more than 64 - refill trace; after the work
         // counter ran out, shade once half of the remaining lanes wait
         const int n_act = __popcll(busy);
         const int keep = !(exhausted || hold) ? 64 - refill
-                                    : (coop_on && n_act <= 8 ? 0 : n_act - max(1, min(refill, n_act >> 1)));
+                                    : n_act - max(1, min(refill, n_act >> 1));
         while (tracing) {
             if (kCount) {
                 const bool lead = lane == __ffsll((unsigned long long)__ballot(1)) - 1;
@@ -943,273 +1258,12 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
 
     if (kLookMode && look && live) look_leave();
 
-    // ---- cooperative tail (kModeDiffuse).  Each of the wave's remaining
-    // paths (at most 8) moves to a group of G = 8 lanes that hold its ray
-    // state alike.  Per step, lane j of a group tests child j of the visited
-    // node, or one of G pending triangles, and the group's choices (nearest children, closest hit) come
-    // from shuffles inside the group.  The closest hit is the same (t, primId)
-    // minimum as lane by lane, whatever the order of the tests, so images do
-    // not change; a path's tail of dependent steps gets shorter.  The group's
-    // stack is its lanes' LDS rings joined (G x kStack entries), spilling to
-    // its first lane's slice.
     if constexpr (kCoop) {
-        const uint64_t cm = __ballot(cont);
-        if (coop_on && cm != 0) {
-            const int npaths = __popcll(cm);
-            constexpr int lg = 3;                 // log2 G: 8 lanes per path
-            constexpr int G = 1 << lg;
-            const int gj = lane & (G - 1);        // this lane's slot in its group
-            const int gbase = lane & ~(G - 1);    // first lane of the group
-            const int grp = lane >> lg;
-            constexpr uint32_t gmask = (1u << G) - 1u;
-            constexpr int kGStack = G * kStack;
-            uint64_t mm = cm;
-            for (int k = 0; k < grp; ++k) mm &= mm - 1;
-            const int src = mm ? __ffsll((unsigned long long)mm) - 1 : 0;
-            const bool gact = grp < npaths;
-            o = mk3(__shfl(o.x, src, 64), __shfl(o.y, src, 64), __shfl(o.z, src, 64));
-            d = mk3(__shfl(d.x, src, 64), __shfl(d.y, src, 64), __shfl(d.z, src, 64));
-            pixel = __shfl(pixel, src, 64);
-            rng = __shfl(rng, src, 64);
-            depth = __shfl(depth, src, 64);
-            lw = __shfl(lw, src, 64);
-            cont = false;
-            active = gact;
-            tracing = false;
-            if (gact) start_ray(o, d, 0.0f, 3.402823466e38f);
-            uint2* g_spill = spill + ((size_t)blockIdx.x * kBlock + (tid & ~(G - 1))) * (size_t)stack_entries;
-            auto gslot = [&](int q) { return ((q >> lg) & (kStack - 1)) * kBlock + (tid & ~(G - 1)) + (q & (G - 1)); };
+        if (coop_paths != 0) {
+            to_groups(coop_paths);
             for (;;) {
-                while (__ballot(tracing) != 0) {
-                    if (kCount) {
-                        const bool lead = lane == __ffsll((unsigned long long)__ballot(1)) - 1;
-                        if (tracing) {
-                            ++n_lsteps;
-                            ++n_dlsteps;
-                        }
-                        if (lead) {
-                            ++n_wsteps;
-                            ++n_dwsteps;
-                        }
-                    }
-                    if (tracing && pend == 0) {
-                        if (node >= 0 && node_t > tbest) node = -1;
-                        if (node < 0) {
-                            while (sp > 0) {
-                                --sp;
-                                uint32_t nid;
-                                float nt;
-                                if (sp < bottom) {
-                                    const uint2 e = g_spill[sp];
-                                    bottom = sp;
-                                    nid = e.x;
-                                    nt = as_f(e.y);
-                                } else {
-                                    const int slot = gslot(sp & (kGStack - 1));
-                                    nid = st_node[slot];
-                                    nt = st_t[slot];
-                                }
-                                if (nt <= tbest) { node = (int32_t)nid; break; }
-                            }
-                            if (node < 0) tracing = false;
-                        }
-                    }
-                    const bool node_step = tracing && pend == 0;
-                    // this lane's children: slots gj + c G, c < 8 / G
-                    float tkc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                    bool hitc[4] = {false, false, false, false};
-                    uint4 w0{}, w1{};
-                    if (node_step) {
-                        const PRT_GLOBAL uint4* np = reinterpret_cast<const PRT_GLOBAL uint4*>(nodes + node);
-                        w0 = np[0];
-                        w1 = np[1];
-                        const uint4 w2 = np[2], w3 = np[3], w4 = np[4];
-                        if (kCount && gj == 0) ++n_nodes;
-                        const int ex = (int)(int8_t)(w0.w & 0xffu);
-                        const int ey = (int)(int8_t)((w0.w >> 8) & 0xffu);
-                        const int ez = (int)(int8_t)((w0.w >> 16) & 0xffu);
-                        const float ax = __uint_as_float((uint32_t)(ex + 127) << 23) * inv_x;
-                        const float ay = __uint_as_float((uint32_t)(ey + 127) << 23) * inv_y;
-                        const float az = __uint_as_float((uint32_t)(ez + 127) << 23) * inv_z;
-                        const float bx = (as_f(w0.x) - o.x) * inv_x;
-                        const float by = (as_f(w0.y) - o.y) * inv_y;
-                        const float bz = (as_f(w0.z) - o.z) * inv_z;
-                        const float slx = 4.76837158203125e-7f * (255.0f * fabsf(ax) + fabsf(bx));
-                        const float sly = 4.76837158203125e-7f * (255.0f * fabsf(ay) + fabsf(by));
-                        const float slz = 4.76837158203125e-7f * (255.0f * fabsf(az) + fabsf(bz));
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            const int k = gj + (c << lg);
-                            if (k < 8) {
-                                // child k: byte k & 3 of the words of its half of the node
-                                const bool hi = k >= 4;
-                                const int kb = k & 3;
-                                const uint32_t qlx = hi ? w2.y : w2.x, qhx = hi ? w3.w : w3.z;
-                                const uint32_t qly = hi ? w2.w : w2.z, qhy = hi ? w4.y : w4.x;
-                                const uint32_t qlz = hi ? w3.y : w3.x, qhz = hi ? w4.w : w4.z;
-                                const float lox = byte_f(qlx, kb), hix = byte_f(qhx, kb);
-                                const float loy = byte_f(qly, kb), hiy = byte_f(qhy, kb);
-                                const float loz = byte_f(qlz, kb), hiz = byte_f(qhz, kb);
-                                const float tnx = __builtin_fmaf(neg_x ? hix : lox, ax, bx - slx);
-                                const float tny = __builtin_fmaf(neg_y ? hiy : loy, ay, by - sly);
-                                const float tnz = __builtin_fmaf(neg_z ? hiz : loz, az, bz - slz);
-                                const float tfx = __builtin_fmaf(neg_x ? lox : hix, ax, bx + slx);
-                                const float tfy = __builtin_fmaf(neg_y ? loy : hiy, ay, by + sly);
-                                const float tfz = __builtin_fmaf(neg_z ? loz : hiz, az, bz + slz);
-                                tkc[c] = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), tmin);
-                                const float tf = fminf(fminf(fminf(tfx, tfy), tfz), tbest);
-                                hitc[c] = tkc[c] <= tf;
-                            }
-                        }
-                    }
-                    uint32_t ghits = 0;
-#pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                        ghits |= ((uint32_t)(__ballot(hitc[c]) >> gbase) & gmask) << (c << lg);
-                    ghits &= 0xffu;
-                    if (node_step) {
-                        const uint32_t imask = w0.w >> 24;
-                        const uint32_t hit_int = ghits & imask;
-                        uint32_t hit_leaf = ghits & ~imask;
-                        while (hit_leaf) {
-                            const int k = __builtin_ctz(hit_leaf);
-                            hit_leaf &= hit_leaf - 1;
-                            const uint32_t mb = ((k < 4 ? w1.z : w1.w) >> (8 * (k & 3))) & 0xffu;
-                            pend |= ((1u << (mb >> 5)) - 1u) << (mb & 31u);
-                        }
-                        pend_base = w1.y;
-                        node = -1;
-                        if (hit_int) {
-                            // nearest and second nearest internal child over the group
-                            float t1 = __builtin_inff(), t2 = __builtin_inff();
-                            int k1 = 8, k2 = 8;
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) {
-                                const int k = gj + (c << lg);
-                                if (k < 8 && ((hit_int >> k) & 1u) && (tkc[c] < t1 || (tkc[c] == t1 && k < k1))) {
-                                    t1 = tkc[c];
-                                    k1 = k;
-                                }
-                            }
-                            for (int x = 1; x < G; x <<= 1) {
-                                const float ot = __shfl_xor(t1, x, 64);
-                                const int ok = __shfl_xor(k1, x, 64);
-                                if (ot < t1 || (ot == t1 && ok < k1)) { t1 = ot; k1 = ok; }
-                            }
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) {
-                                const int k = gj + (c << lg);
-                                if (k < 8 && k != k1 && ((hit_int >> k) & 1u) &&
-                                    (tkc[c] < t2 || (tkc[c] == t2 && k < k2))) {
-                                    t2 = tkc[c];
-                                    k2 = k;
-                                }
-                            }
-                            for (int x = 1; x < G; x <<= 1) {
-                                const float ot = __shfl_xor(t2, x, 64);
-                                const int ok = __shfl_xor(k2, x, 64);
-                                if (ot < t2 || (ot == t2 && ok < k2)) { t2 = ot; k2 = ok; }
-                            }
-                            const uint32_t child_base = w1.x;
-                            node = (int32_t)(child_base + __popc(imask & ((1u << k1) - 1u)));
-                            node_t = t1;
-                            const uint32_t pushm = hit_int & ~(1u << k1);
-                            if (pushm) {
-                                const int npush = __popc(pushm);
-                                bool ok = true;
-                                while (sp + npush - bottom > kGStack) {
-                                    if (bottom >= spill_cap) { atomicOr(err, 1u); ok = false; break; }
-                                    const int bslot = gslot(bottom & (kGStack - 1));
-                                    g_spill[bottom] = make_uint2(st_node[bslot], __float_as_uint(st_t[bslot]));
-                                    ++bottom;
-                                    if (kCount && gj == 0) ++n_spill;
-                                }
-                                if (ok) {
-                                    const int klast = 31 - __builtin_clz(pushm);
-                                    if (k2 > 7 || !((pushm >> k2) & 1u)) k2 = klast;
-                                    const int pos_k2 = __popc(pushm & ((1u << k2) - 1u));
-#pragma unroll
-                                    for (int c = 0; c < 4; ++c) {
-                                        const int k = gj + (c << lg);
-                                        if (k < 8 && ((pushm >> k) & 1u)) {
-                                            int pos = __popc(pushm & ((1u << k) - 1u));
-                                            pos = k == k2 ? npush - 1 : (k == klast ? pos_k2 : pos);
-                                            const int slot = gslot((sp + pos) & (kGStack - 1));
-                                            st_node[slot] = child_base + __popc(imask & ((1u << k) - 1u));
-                                            st_t[slot] = tkc[c];
-                                        }
-                                    }
-                                    sp += npush;
-                                }
-                            }
-                        }
-                    }
-                    if (tracing && pend != 0 && !node_step) {
-                        // up to G pending triangles at once: lane j takes the
-                        // j-th lowest pending record
-                        uint32_t mj = pend;
-                        for (int k = 0; k < gj; ++k) mj &= mj - 1;
-                        for (int k = 0; k < G; ++k) pend &= pend - 1;
-                        float ct = __builtin_inff();
-                        int32_t cp = INT32_MAX;
-                        uint32_t crec = 0;
-                        if (mj != 0) {
-                            const uint32_t rec = pend_base + (uint32_t)__builtin_ctz(mj);
-                            const PRT_GLOBAL float* tp = tris + 9 * (size_t)rec;
-                            const f3 p0 = mk3(tp[0], tp[1], tp[2]);
-                            const f3 p1 = mk3(tp[3], tp[4], tp[5]);
-                            const f3 p2 = mk3(tp[6], tp[7], tp[8]);
-                            if (kCount) ++n_tris;
-                            float t;
-                            if (tri_test(wr, o, d, p0, p1, p2, tmin, tbest, t)) {
-                                ct = t;
-                                cp = prim_ids[rec];
-                                crec = rec;
-                            }
-                        }
-                        for (int x = 1; x < G; x <<= 1) {
-                            const float ot = __shfl_xor(ct, x, 64);
-                            const int32_t op = __shfl_xor(cp, x, 64);
-                            const uint32_t orr = __shfl_xor(crec, x, 64);
-                            if (ot < ct || (ot == ct && op < cp)) { ct = ot; cp = op; crec = orr; }
-                        }
-                        if (cp != INT32_MAX && (ct < tbest || best_prim < 0 || cp < best_prim)) {
-                            tbest = ct;
-                            best_prim = cp;
-                            best_rec = crec;
-                        }
-                    }
-                }
-                // ---- shade each group's finished ray (the same in its G lanes;
-                // its first lane counts the ray and writes the pixel)
-                if (active) {
-                    if constexpr (kCount) {
-                        if (gj == 0) atomicAdd(&depth_hist[min(depth, kMaxQueueDepth - 1)], 1u);
-                    }
-                    if (gj == 0) ++n_rays;
-                    float4* acc = pl.accum + pixel;
-                    if (best_prim < 0 || depth == max_depth) {
-                        const float c = best_prim < 0 ? lw : 0.0f;
-                        if (gj == 0) {
-                            const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
-                            *acc = make_float4(a.x + c, a.y + c, a.z + c, a.w + 1.0f);
-                        }
-                        active = false;
-                    } else {
-                        const PRT_GLOBAL float* tp = tris + 9 * (size_t)best_rec;
-                        const f3 p0 = mk3(tp[0], tp[1], tp[2]);
-                        const f3 p1 = mk3(tp[3], tp[4], tp[5]);
-                        const f3 p2 = mk3(tp[6], tp[7], tp[8]);
-                        lw *= albedo;
-                        const Frame fr = hit_frame(p0, p1, p2);
-                        const float s1 = sampler_next(rng);
-                        const float s2 = sampler_next(rng);
-                        f3 no, nd;
-                        diffuse_bounce(o, d, tbest, fr, s1, s2, no, nd);
-                        ++depth;
-                        start_ray(no, nd, 0.0f, 3.402823466e38f);
-                    }
-                }
+                coop_traverse(__popcll(__ballot(active)) >> 3);
+                shade(gj == 0);
                 if (__ballot(active) == 0) break;
             }
         }
@@ -1263,13 +1317,56 @@ __global__ __launch_bounds__(kBlock) void k_trace(SceneDevice sc, TraceLaunch tl
     }
 }
 
+// Persistent workgroups of a launch over `items` rays or paths.  Each wave pays
+// for the drain of its own last items (about 50 steps at a few active lanes),
+// so a launch that has few items per lane gains more from fewer waves than it
+// loses in latency hiding.  Measured per frame or launch with 1 / 2 / 3 / 4
+// workgroups per CU (256 CUs of 256 lanes each), ms:
+//   diffuse   24 k paths 0.248 0.246 0.263 0.283; 140 k 0.618 0.631 0.606 0.623;
+//             262 k 0.457 0.320 0.337 0.377; 518 k 0.806 0.717 0.769 0.810;
+//             0.92 M 1.392 0.979 0.995 1.120; 1.05 M 1.476 0.919 0.792 0.768;
+//             2.07 M 2.260 1.389 1.182 1.167
+//   ray query 60 k 0.098 0.112 0.124 0.132; 200 k 0.314 0.268 0.264 0.274;
+//             1 M 1.071 0.628 0.500 0.481
+//   diffuse2  290 k 0.690 0.770 0.846 0.796; 1.35 M 1.585 1.124 1.115 1.224:
+//             two rays a hit make its drain twice as long, so it counts half
+//   primary   262 k 0.088 0.093 0.106 0.118; 8.3 M 1.737 1.729 1.743 1.766:
+//             coherent rays fill the issue slots with 2
+// On scenes whose nodes and triangles outgrow the memory-side cache (256 MiB)
+// diffuse launches run at most one below the occupancy limit: their paths take
+// long, so does the drain; the albedo and query launches are faster with all.
+int grid_for(const prt_hip_ctx* ctx, int mode, uint64_t items)
+{
+    if (mode == kModeDiffuse2) items /= 2;
+    int per_cu = items <= (128u << 10) ? 1 : (items <= (640u << 10) ? 2 : (items <= (1000u << 10) ? 3 : 4));
+    if (mode == kModePrimary) per_cu = std::min(per_cu, 2);
+    int limit = ctx->trace_per_cu;
+    if (mode == kModeDiffuse && limit > 1) {
+        const SceneBuffers& s = ctx->scene;
+        const int64_t scene_bytes =
+            s.node_count * (int64_t)sizeof(Bvh8Node) + s.tri_count * (int64_t)(9 * sizeof(float) + sizeof(int32_t));
+        if (scene_bytes > kLargeSceneBytes) limit -= 1;
+    }
+    return std::min(per_cu, limit) * ctx->num_cus;
+}
+
+// Work items of a launch; ~0 where only the device knows.
+uint64_t launch_items(int mode, const TraceLaunch& t, const PathLaunch& p)
+{
+    if (mode == kModeTrace || mode == kModeOccluded) return t.count_ptr ? ~0ull : t.count;
+    if (mode == kModeAdjoint || (mode == kModeRgb && p.rgb_planes)) return (uint64_t)p.entries * (uint64_t)p.spp;
+    return p.entries;
+}
+
 template <int kMode>
-hipError_t launch_mode(prt_hip_ctx* ctx, const TraceLaunch& t, const PathLaunch& p, bool instrumented)
+hipError_t launch_mode(prt_hip_ctx* ctx, const TraceLaunch& t, const PathLaunch& paths, bool instrumented)
 {
     const SceneDevice sc = ctx->scene.device();
     uint32_t* err = ctx->d_counters + 32;
     const BatchLaunch bl{};
-    const int grid = kMode == kModeDiffuse ? ctx->diffuse_grid : ctx->trace_grid;
+    const int grid = grid_for(ctx, kMode, launch_items(kMode, t, paths));
+    PathLaunch p = paths;
+    p.coop = ctx->tail_coop;
     if (instrumented) {
         k_trace<true, kMode><<<grid, kTraceBlock, 0, ctx->stream>>>(
             sc, t, p, bl, ctx->d_spill, ctx->stack_entries, kRefill, err);
@@ -1303,7 +1400,8 @@ hipError_t launch_batch_variant(prt_hip_ctx* ctx, const BatchLaunch& bl, int blo
     uint32_t* err = ctx->d_counters + 32;
     const SceneDevice sc{};
     const TraceLaunch t{};
-    const PathLaunch p{};
+    PathLaunch p{};
+    p.coop = ctx->tail_coop;
     if (instrumented)
         k_trace<true, kModeBatch, kBlock, kStack><<<grid, kBlock, 0, ctx->stream>>>(
             sc, t, p, bl, ctx->d_spill, ctx->stack_entries, refill, err);
@@ -1332,18 +1430,6 @@ int ensure_trace_resources(prt_hip_ctx* ctx)
         ctx->trace_per_cu = per_cu;
     }
     ctx->trace_grid = ctx->trace_per_cu * ctx->num_cus;
-    // Diffuse render launches on a scene whose nodes and triangles outgrow the
-    // memory-side cache (256 MiB) run one workgroup per CU fewer.  Paths on such
-    // a scene take long, so a frame's tail (its last paths, in sparse waves)
-    // is long, and fewer resident waves shorten it by more than they slow the
-    // rest; the albedo and trace launches keep the full occupancy, which is
-    // faster for them
-    const SceneBuffers& s = ctx->scene;
-    const int64_t scene_bytes =
-        s.node_count * (int64_t)sizeof(Bvh8Node) + s.tri_count * (int64_t)(9 * sizeof(float) + sizeof(int32_t));
-    int per_cu = ctx->trace_per_cu;
-    if (scene_bytes > kLargeSceneBytes && per_cu > 1) per_cu -= 1;
-    ctx->diffuse_grid = per_cu * ctx->num_cus;
     // worst case stack: 7 pushes per level of the tree, plus slack; sized for
     // the deepest scene and for every lane a CU can hold (2048), so any
     // persistent launch shape fits
@@ -1370,6 +1456,10 @@ int ensure_trace_resources(prt_hip_ctx* ctx)
     return 0;
 }
 
+int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries) { return grid_for(ctx, kModeDiffuse, entries); }
+
+int query_grid(const prt_hip_ctx* ctx, int64_t rays) { return grid_for(ctx, kModeTrace, (uint64_t)rays); }
+
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented)
 {
     return launch_mode<kModeTrace>(ctx, t, PathLaunch{}, instrumented);
@@ -1378,9 +1468,10 @@ hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumente
 hipError_t launch_trace_scratch(prt_hip_ctx* ctx, const TraceLaunch& t, uint2* spill, int stack_entries,
                                 uint32_t* err, int grid)
 {
-    k_trace<false, kModeTrace><<<grid, kTraceBlock, 0, ctx->stream>>>(ctx->scene.device(), t, PathLaunch{},
-                                                                     BatchLaunch{}, spill, stack_entries, kRefill,
-                                                                     err);
+    PathLaunch p{};
+    p.coop = ctx->tail_coop;
+    k_trace<false, kModeTrace><<<grid, kTraceBlock, 0, ctx->stream>>>(ctx->scene.device(), t, p, BatchLaunch{}, spill,
+                                                                     stack_entries, kRefill, err);
     return hipGetLastError();
 }
 
