@@ -303,7 +303,7 @@ int prt_hip_destroy(prt_hip_ctx* ctx)
     void* ptrs[] = {ctx->d_spill,
                     ctx->d_accum, ctx->d_bgr8, ctx->d_rays[0], ctx->d_rays[1], ctx->d_hits,
                     ctx->d_pix[0], ctx->d_pix[1], ctx->d_rng[0], ctx->d_rng[1], ctx->d_counters,
-                    ctx->d_io_rays, ctx->d_io_hits, ctx->d_look, ctx->d_look_side, ctx->d_look_flags};
+                    ctx->d_io_rays, ctx->d_io_hits, ctx->d_look, ctx->d_look_side, ctx->d_look_flags, ctx->d_build};
     for (void* p : ptrs) free_ptr(p);
     for (auto& level : ctx->d_look_q)
         for (uint4* q : level) free_ptr(q);

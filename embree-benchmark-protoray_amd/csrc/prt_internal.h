@@ -33,6 +33,7 @@ static_assert(sizeof(Bvh8Node) == 80, "BVH8 node must be 80 bytes");
 constexpr int kLeafMax = 3;           // triangles per leaf slot
 constexpr int kTraceBlock = 256;      // threads per trace workgroup
 constexpr int64_t kLargeSceneBytes = int64_t(256) << 20;  // nodes + triangles beyond MI355X's 256 MiB Infinity Cache
+constexpr size_t kBuildKeepBytes = size_t(512) << 20;  // build scratch a context keeps (about 150 B per triangle)
 constexpr int kMaxQueueDepth = 16;    // per-depth ray statistics bins; the last bin holds depths >= 15
 constexpr int kMaxDepth = 1024;       // largest max_depth accepted (an R^k throughput below 1 is 0 in fp32 long before)
 
@@ -255,6 +256,10 @@ struct prt_hip_ctx {
     // device address of the library's fixed scratch array on this context's
     // GPU (prt_hip_intersect_closest_device_noalloc)
     void* d_scratch = nullptr;
+
+    // scratch of the last builds (kept up to kBuildKeepBytes)
+    void* d_build = nullptr;
+    size_t build_bytes = 0;
 
     // BVH8 collapse (prt_hip_set_bvh_collapse)
     int bvh_collapse = PRT_COLLAPSE_SAH;
