@@ -430,7 +430,7 @@ int prt_hip_intersect_closest_device_noalloc(prt_hip_ctx* ctx, const prt_ray* d_
         return set_error(ctx, "intersect_noalloc: a BVH of depth " + std::to_string(ctx->scene.bvh_depth) +
                                   " needs " + std::to_string(per_block) + " bytes of stack per workgroup, more than the " +
                                   std::to_string((size_t)PRT_HIP_NOALLOC_SCRATCH_BYTES) + "-byte scratch holds");
-    int grid = query_grid(ctx, n);
+    int grid = ctx->trace_grid;
     if ((size_t)grid > blocks_fit) grid = (int)blocks_fit;
     uint32_t* hdr = static_cast<uint32_t*>(ctx->d_scratch);
     PRT_TRY(ctx, launch_zero_u32(hdr, 2, ctx->stream));  // a kernel, not a memset: safe under graph capture
@@ -720,6 +720,7 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
     // camera that moves every frame renders each frame exactly as without
     // it; the work is kept only if that previous call ran the lookahead too.
     const bool look_on = fused && renderer == PRT_RENDERER_DIFFUSE && !fast && !counting && ctx->lookahead != 0 &&
+                         lookahead_pays(ctx, entries) &&
                          ctx->pass < INT32_MAX - kLookLevels;  // the passes started ahead must not overflow
     prt_hip_ctx::LookKey key{};
     if (look_on) {

@@ -281,6 +281,9 @@ struct TraceLaunch {
     uint32_t* fetch_ptr;        // device fetch counter, zero before launch
     unsigned long long* stats;  // nullptr unless instrumented
 };
+// PathLaunch::coop: a wave's last rays or paths on 8 lanes each (0: never), or
+// a small launch spread over the waves that way from its start
+constexpr int kCoopTail = 1, kCoopSpread = 2;
 // Fused path launch (one frame, one sample per pixel)
 // Frame lookahead of the fused diffuse renderer: device state that one render
 // call hands to the next.  A call renders frame p; a path of frame p + l is
@@ -335,8 +338,7 @@ struct PathLaunch {
     // the "Fast" renderers: frame of the geometric normal whatever attributes
     // the mesh has, and each pass overwrites the accumulator
     bool fast;
-    // a wave with at most 8 rays or paths left traces them cooperatively (0:
-    // never)
+    // cooperative tracing (kCoopTail, kCoopSpread or 0); set by the launch
     int coop;
     // diffuse frames: frame lookahead (nullptr: off)
     LookState* look;
@@ -348,15 +350,16 @@ struct PathLaunch {
     uint32_t* look_flags; // per block (kLookFlagStride apart): look_gen once this frame is finished
 };
 int ensure_trace_resources(prt_hip_ctx* ctx);
-// persistent workgroups of a diffuse frame of `entries` path slots, and of a
-// closest-hit query of `rays` rays
+// persistent workgroups of a diffuse frame of `entries` path slots under the
+// lookahead
 int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries);
-int query_grid(const prt_hip_ctx* ctx, int64_t rays);
+// frames of so many path slots are faster with the lookahead
+bool lookahead_pays(const prt_hip_ctx* ctx, uint32_t entries);
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented);
-// closest-hit launch over `grid` persistent workgroups whose stack spill
-// (stack_entries per lane) and error flag the caller provides
+// closest-hit launch over at most max_grid persistent workgroups whose stack
+// spill (stack_entries per lane) and error flag the caller provides
 hipError_t launch_trace_scratch(prt_hip_ctx* ctx, const TraceLaunch& t, uint2* spill, int stack_entries,
-                                uint32_t* err, int grid);
+                                uint32_t* err, int max_grid);
 hipError_t launch_occluded(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented);
 // renderer: PRT_RENDERER_PRIMARY, _DIFFUSE or _DIFFUSE2
 hipError_t launch_paths(prt_hip_ctx* ctx, const PathLaunch& p, int renderer, bool instrumented);

@@ -100,7 +100,7 @@ __device__ __forceinline__ uint32_t nth_bit(uint32_t m, uint32_t r)
 
 // kLook: the fused diffuse frame with the frame lookahead compiled in.
 template <bool kCount, int kMode, int kBlock = kTraceBlock, int kStack = kStackLds, bool kLook = false>
-__global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoint ? 4 : 1) void k_trace(SceneDevice sc, TraceLaunch tl, PathLaunch pl, BatchLaunch bl,
+__global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoint || kMode == kModeDiffuse2 ? 4 : 1) void k_trace(SceneDevice sc, TraceLaunch tl, PathLaunch pl, BatchLaunch bl,
                                                   uint2* spill, int stack_entries, int refill, uint32_t* err)
 {
     static_assert((kStack & (kStack - 1)) == 0, "LDS stack depth must be a power of two");
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     auto look_leave = [&]() {
         uint32_t old = 0;
         if (lane == 0) old = atomicSub(&look->live, 1u);
-        old = __shfl(old, 0, 64);
+        old = (uint32_t)__builtin_amdgcn_readfirstlane((int)old);
         if (old == 1u)
             for (uint32_t b = (uint32_t)lane; b < gridDim.x; b += 64u)
                 __hip_atomic_store(pl.look_flags + (size_t)b * kLookFlagStride, pl.look_gen, __ATOMIC_RELAXED,
@@ -296,6 +296,138 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
             return attribute_frame(aidx, an, at, best_prim, p0, p1, p2, d, hu, hv);
         }
         return make_frame(face_normal(p0, p1, p2, d));
+    };
+
+    // Starts work item `my` (a ray, or a path's camera ray) in this lane.
+    // spec_claim: an item of a later frame (lookahead).
+    auto start_item = [&](uint32_t my, bool spec_claim) __attribute__((always_inline)) {
+        if (kRayQuery) {
+            ray_idx = my;
+            const float4 r0 = tl.rays[2 * (size_t)my];
+            const float4 r1 = tl.rays[2 * (size_t)my + 1];
+            if (r1.w < 0.0f) {
+                if (kMode == kModeOccluded) tl.any_t[my] = -1.0f;
+                else tl.hits[my] = make_float4(-1.0f, __int_as_float(-1), 0.0f, 0.0f);
+            } else {
+                start_ray(mk3(r0.x, r0.y, r0.z), mk3(r1.x, r1.y, r1.z), r0.w, r1.w);
+                active = true;
+            }
+        } else if (kMode == kModeBatch) {
+            // work item -> job (binary search over the job prefix),
+            // then sample and path inside the job
+            int lo = 0, hi = bl.n_jobs;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (bl.work_begin[mid] <= my) lo = mid; else hi = mid;
+            }
+            const BatchJobDevice& job = bl.jobs[lo];
+            const uint32_t local = my - bl.work_begin[lo];
+            const uint32_t sample = local / job.entries;
+            const uint32_t path = local - sample * job.entries;
+            const uint32_t tile = path >> 6, tl_lane = path & 63u;
+            const int mx = (tl_lane & 1) | ((tl_lane >> 1) & 2) | ((tl_lane >> 2) & 4);
+            const int my_ = ((tl_lane >> 1) & 1) | ((tl_lane >> 2) & 2) | ((tl_lane >> 3) & 4);
+            const int x = (int)(tile % (uint32_t)job.tiles_x) * 8 + mx;
+            const int y = (int)(tile / (uint32_t)job.tiles_x) * 8 + my_;
+            if (x < job.width && y < job.height) {
+                pixel = x + y * job.width;
+                const SceneDevice jsc = bl.scenes[job.scene];
+                scene_id = job.scene;
+                nodes = global_view(jsc.nodes);
+                tris = global_view(jsc.tris);
+                prim_ids = global_view(jsc.prim_ids);
+                sample_out = bl.samples + job.sample_base +
+                             (size_t)sample * (size_t)(job.width * job.height) + pixel;
+                max_depth = job.max_depth;
+                albedo = job.albedo;
+                rng = sampler_seed(job.pass0 + (int)sample, pixel);
+                const float u1 = sampler_next(rng);
+                const float u2 = sampler_next(rng);
+                const float l1 = sampler_next(rng);  // lens 2D
+                const float l2 = sampler_next(rng);
+                f3 org, dir;
+                camera_ray(job.cam, ((float)x + u1) * job.inv_w, ((float)y + u2) * job.inv_h, l1, l2,
+                           org, dir);
+                start_ray(org, dir, 0.0f, 3.402823466e38f);
+                depth = 0;
+                lw = 1.0f;
+                active = true;
+            }
+        } else if (kLookMode && look && !spec_claim && my >= lk_F) {
+            // a path that the previous call stopped at a bounce
+            // (or in the middle of a ray): its next ray
+            const uint4* q = pl.q_in[0] + 3 * (size_t)(my - lk_res[0]);
+            level = 0;
+#pragma unroll
+            for (int l = 1; l < kLookLevels; ++l)
+                if (my >= lk_res[l]) {
+                    q = pl.q_in[l] + 3 * (size_t)(my - lk_res[l]);
+                    level = l;
+                }
+            const uint4 e0 = q[0], e1 = q[1], e2 = q[2];
+            pixel = (int32_t)e0.w;
+            rng = e1.w;
+            depth = (int)e2.x;
+            lw = __uint_as_float(e2.y);
+            start_ray(mk3(as_f(e0.x), as_f(e0.y), as_f(e0.z)), mk3(as_f(e1.x), as_f(e1.y), as_f(e1.z)),
+                      0.0f, 3.402823466e38f);
+            active = true;
+        } else {
+            // camera ray of path `my`: 8x8 tiles, Morton order inside
+            // a tile (image/morton.cpp:22), as the wavefront raygen
+            uint32_t path = my;
+            path_pass = pl.pass;
+            if (kLookMode && look) {
+                level = 0;
+                path = lk_S[0] + my;
+                if (spec_claim) {
+#pragma unroll
+                    for (int l = 1; l <= kLookLevels; ++l)
+                        if (my >= lk_spec[l]) {
+                            level = l;
+                            path = lk_S[l] + (my - lk_spec[l]);
+                        }
+                }
+                path_pass = pl.pass + level;
+            }
+            if (kMode == kModeAdjoint || (kMode == kModeRgb && pl.rgb_planes)) {
+                const uint32_t sample = my / pl.entries;
+                path = my - sample * pl.entries;
+                path_pass = pl.pass + (int)sample;
+            }
+            const uint32_t tile = path >> 6, tl_lane = path & 63u;
+            const int mx = (tl_lane & 1) | ((tl_lane >> 1) & 2) | ((tl_lane >> 2) & 4);
+            const int my_ = ((tl_lane >> 1) & 1) | ((tl_lane >> 2) & 2) | ((tl_lane >> 3) & 4);
+            const int x = (int)(tile % (uint32_t)pl.tiles_x) * 8 + mx;
+            const int y = (int)(tile / (uint32_t)pl.tiles_x) * 8 + my_;
+            if (x < pl.width && y < pl.height) {
+                pixel = x + y * pl.width;
+                rng = sampler_seed(path_pass, pixel);
+                const float u1 = sampler_next(rng);
+                const float u2 = sampler_next(rng);
+                const float l1 = sampler_next(rng);  // lens 2D
+                const float l2 = sampler_next(rng);
+                f3 org, dir;
+                camera_ray(pl.cam, ((float)x + u1) * pl.inv_w, ((float)y + u2) * pl.inv_h, l1, l2, org,
+                           dir);
+                start_ray(org, dir, 0.0f, 3.402823466e38f);
+                depth = 0;
+                lw = lg = lb = 1.0f;
+                lsum = 0.0f;
+                shadow = false;
+                active = true;
+                if (kMode == kModeAdjoint) {
+                    replay = false;
+                    pr = pg = pb = 1.0f;
+                    zeros = 0;
+                    const float* g = pl.dldi + 3 * (size_t)pixel;
+                    gw_r = g[0] * pl.inv_spp;
+                    gw_g = g[1] * pl.inv_spp;
+                    gw_b = g[2] * pl.inv_spp;
+                    if (gw_r == 0.0f && gw_g == 0.0f && gw_b == 0.0f) active = tracing = false;
+                }
+            }
+        }
     };
 
     // Shades the lanes whose ray has finished (active, not tracing).  lead: the
@@ -599,7 +731,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     // Traverses the groups' rays until half of the `groups` with a path wait
     // for shading.
     auto coop_traverse = [&](int groups) {
-        const int keep = groups - max(1, groups >> 1);
+        const int keep = max(0, groups - max(1, groups >> 1));  // no groups: nothing to trace
         for (;;) {
             const int left = __popcll(__ballot(tracing)) >> 3;
             if (left <= keep) break;
@@ -763,7 +895,10 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         }
     };
 
-    for (;;) {
+    uint32_t* const work_counter = kRayQuery ? tl.fetch_ptr : (kMode == kModeBatch ? bl.work_counter : pl.path_counter);
+    // a small launch is traced in groups from its start (wave-uniform)
+    const bool spread = kCoop && pl.coop == kCoopSpread;
+    while (!spread) {
         // lookahead: a wave that holds paths of this frame takes no items of
         // later frames once this frame's are handed out, and issues ahead of
         // the waves that run later frames' paths, so the frame's last paths
@@ -803,7 +938,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
                 const int leader = __ffsll((unsigned long long)sm) - 1;
                 uint32_t qb = 0;
                 if (lane == leader) qb = atomicAdd(&look->resume_out[l], (uint32_t)__popcll(sm));
-                qb = __shfl(qb, leader, 64);
+                qb = (uint32_t)__builtin_amdgcn_readlane((int)qb, leader);
                 if (mine) {
                     const uint32_t slot = qb + (uint32_t)__popcll(sm & lane_lt);
                     if (slot < pl.q_cap) {
@@ -825,144 +960,18 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         const int n_idle = __popcll(idle);
         if (!exhausted && !hold && n_idle >= refill) {
             const int leader = __ffsll((unsigned long long)idle) - 1;
-            uint32_t* ctr = kRayQuery ? tl.fetch_ptr : (kMode == kModeBatch ? bl.work_counter : pl.path_counter);
+            uint32_t* ctr = work_counter;
             uint32_t lim = count;
             const bool spec_claim = kLookMode && look && fresh_out;  // items of later frames
             if (kLookMode && look) lim = spec_claim ? lk_spec[kLookLevels + 1] : lk_fresh_end;
             if (spec_claim) ctr = &look->spec_counter;
             uint32_t base = 0;
             if (lane == leader) base = atomicAdd(ctr, (uint32_t)n_idle);
-            base = __shfl(base, leader, 64);
+            base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);  // wave-uniform
             if (!active) {
                 const uint32_t my = base + (uint32_t)__popcll(idle & lane_lt);
                 if (my < lim) {
-                    if (kRayQuery) {
-                        ray_idx = my;
-                        const float4 r0 = tl.rays[2 * (size_t)my];
-                        const float4 r1 = tl.rays[2 * (size_t)my + 1];
-                        if (r1.w < 0.0f) {
-                            if (kMode == kModeOccluded) tl.any_t[my] = -1.0f;
-                            else tl.hits[my] = make_float4(-1.0f, __int_as_float(-1), 0.0f, 0.0f);
-                        } else {
-                            start_ray(mk3(r0.x, r0.y, r0.z), mk3(r1.x, r1.y, r1.z), r0.w, r1.w);
-                            active = true;
-                        }
-                    } else if (kMode == kModeBatch) {
-                        // work item -> job (binary search over the job prefix),
-                        // then sample and path inside the job
-                        int lo = 0, hi = bl.n_jobs;
-                        while (hi - lo > 1) {
-                            const int mid = (lo + hi) >> 1;
-                            if (bl.work_begin[mid] <= my) lo = mid; else hi = mid;
-                        }
-                        const BatchJobDevice& job = bl.jobs[lo];
-                        const uint32_t local = my - bl.work_begin[lo];
-                        const uint32_t sample = local / job.entries;
-                        const uint32_t path = local - sample * job.entries;
-                        const uint32_t tile = path >> 6, tl_lane = path & 63u;
-                        const int mx = (tl_lane & 1) | ((tl_lane >> 1) & 2) | ((tl_lane >> 2) & 4);
-                        const int my_ = ((tl_lane >> 1) & 1) | ((tl_lane >> 2) & 2) | ((tl_lane >> 3) & 4);
-                        const int x = (int)(tile % (uint32_t)job.tiles_x) * 8 + mx;
-                        const int y = (int)(tile / (uint32_t)job.tiles_x) * 8 + my_;
-                        if (x < job.width && y < job.height) {
-                            pixel = x + y * job.width;
-                            const SceneDevice jsc = bl.scenes[job.scene];
-                            scene_id = job.scene;
-                            nodes = global_view(jsc.nodes);
-                            tris = global_view(jsc.tris);
-                            prim_ids = global_view(jsc.prim_ids);
-                            sample_out = bl.samples + job.sample_base +
-                                         (size_t)sample * (size_t)(job.width * job.height) + pixel;
-                            max_depth = job.max_depth;
-                            albedo = job.albedo;
-                            rng = sampler_seed(job.pass0 + (int)sample, pixel);
-                            const float u1 = sampler_next(rng);
-                            const float u2 = sampler_next(rng);
-                            const float l1 = sampler_next(rng);  // lens 2D
-                            const float l2 = sampler_next(rng);
-                            f3 org, dir;
-                            camera_ray(job.cam, ((float)x + u1) * job.inv_w, ((float)y + u2) * job.inv_h, l1, l2,
-                                       org, dir);
-                            start_ray(org, dir, 0.0f, 3.402823466e38f);
-                            depth = 0;
-                            lw = 1.0f;
-                            active = true;
-                        }
-                    } else if (kLookMode && look && !spec_claim && my >= lk_F) {
-                        // a path that the previous call stopped at a bounce
-                        // (or in the middle of a ray): its next ray
-                        const uint4* q = pl.q_in[0] + 3 * (size_t)(my - lk_res[0]);
-                        level = 0;
-#pragma unroll
-                        for (int l = 1; l < kLookLevels; ++l)
-                            if (my >= lk_res[l]) {
-                                q = pl.q_in[l] + 3 * (size_t)(my - lk_res[l]);
-                                level = l;
-                            }
-                        const uint4 e0 = q[0], e1 = q[1], e2 = q[2];
-                        pixel = (int32_t)e0.w;
-                        rng = e1.w;
-                        depth = (int)e2.x;
-                        lw = __uint_as_float(e2.y);
-                        start_ray(mk3(as_f(e0.x), as_f(e0.y), as_f(e0.z)), mk3(as_f(e1.x), as_f(e1.y), as_f(e1.z)),
-                                  0.0f, 3.402823466e38f);
-                        active = true;
-                    } else {
-                        // camera ray of path `my`: 8x8 tiles, Morton order inside
-                        // a tile (image/morton.cpp:22), as the wavefront raygen
-                        uint32_t path = my;
-                        path_pass = pl.pass;
-                        if (kLookMode && look) {
-                            level = 0;
-                            path = lk_S[0] + my;
-                            if (spec_claim) {
-#pragma unroll
-                                for (int l = 1; l <= kLookLevels; ++l)
-                                    if (my >= lk_spec[l]) {
-                                        level = l;
-                                        path = lk_S[l] + (my - lk_spec[l]);
-                                    }
-                            }
-                            path_pass = pl.pass + level;
-                        }
-                        if (kMode == kModeAdjoint || (kMode == kModeRgb && pl.rgb_planes)) {
-                            const uint32_t sample = my / pl.entries;
-                            path = my - sample * pl.entries;
-                            path_pass = pl.pass + (int)sample;
-                        }
-                        const uint32_t tile = path >> 6, tl_lane = path & 63u;
-                        const int mx = (tl_lane & 1) | ((tl_lane >> 1) & 2) | ((tl_lane >> 2) & 4);
-                        const int my_ = ((tl_lane >> 1) & 1) | ((tl_lane >> 2) & 2) | ((tl_lane >> 3) & 4);
-                        const int x = (int)(tile % (uint32_t)pl.tiles_x) * 8 + mx;
-                        const int y = (int)(tile / (uint32_t)pl.tiles_x) * 8 + my_;
-                        if (x < pl.width && y < pl.height) {
-                            pixel = x + y * pl.width;
-                            rng = sampler_seed(path_pass, pixel);
-                            const float u1 = sampler_next(rng);
-                            const float u2 = sampler_next(rng);
-                            const float l1 = sampler_next(rng);  // lens 2D
-                            const float l2 = sampler_next(rng);
-                            f3 org, dir;
-                            camera_ray(pl.cam, ((float)x + u1) * pl.inv_w, ((float)y + u2) * pl.inv_h, l1, l2, org,
-                                       dir);
-                            start_ray(org, dir, 0.0f, 3.402823466e38f);
-                            depth = 0;
-                            lw = lg = lb = 1.0f;
-                            lsum = 0.0f;
-                            shadow = false;
-                            active = true;
-                            if (kMode == kModeAdjoint) {
-                                replay = false;
-                                pr = pg = pb = 1.0f;
-                                zeros = 0;
-                                const float* g = pl.dldi + 3 * (size_t)pixel;
-                                gw_r = g[0] * pl.inv_spp;
-                                gw_g = g[1] * pl.inv_spp;
-                                gw_b = g[2] * pl.inv_spp;
-                                if (gw_r == 0.0f && gw_g == 0.0f && gw_b == 0.0f) active = tracing = false;
-                            }
-                        }
-                    }
+                    start_item(my, spec_claim);
                 }
             }
             if ((uint64_t)base + (uint64_t)n_idle >= lim) {
@@ -1259,13 +1268,29 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     if (kLookMode && look && live) look_leave();
 
     if constexpr (kCoop) {
-        if (coop_paths != 0) {
-            to_groups(coop_paths);
-            for (;;) {
-                coop_traverse(__popcll(__ballot(active)) >> 3);
-                shade(gj == 0);
-                if (__ballot(active) == 0) break;
+        if (coop_paths != 0) to_groups(coop_paths);
+        // spread: every wave starts with its own 8 items, without the counter,
+        // which then hands out those past all waves' shares
+        const uint32_t shares = 8u * gridDim.x * (uint32_t)(kBlock / 64);
+        bool more = spread, first = true;
+        while (more || __ballot(active) != 0) {
+            const uint64_t idle = __ballot(!active);
+            const uint32_t n = (uint32_t)__popcll(idle) >> 3;
+            if (more && n >= 4) {
+                uint32_t base = 8u * (blockIdx.x + gridDim.x * (uint32_t)(tid >> 6));
+                if (!first) {
+                    if (lane == 0) base = shares + atomicAdd(work_counter, n);
+                    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+                }
+                if (!active) {
+                    const uint32_t my = base + ((uint32_t)__popcll(idle & ((1ull << gbase) - 1ull)) >> 3);
+                    if (my < count) start_item(my, false);
+                }
+                more = first ? count > shares : (uint64_t)base + n < count;
+                first = false;
             }
+            coop_traverse(__popcll(__ballot(active)) >> 3);
+            shade(gj == 0);
         }
     }
 
@@ -1358,15 +1383,54 @@ uint64_t launch_items(int mode, const TraceLaunch& t, const PathLaunch& p)
     return p.entries;
 }
 
+// Launches of at most this many items are traced in groups of 8 lanes from
+// their start: with so few, a launch takes as long as its longest path's chain
+// of steps, and a step of a group is shorter.  Above, throughput decides: a
+// group's 8 lanes do the work of one.  Measured lane by lane / in groups, us:
+//   closest hits  512 rays 112 / 73, 8192 144 / 92, 32768 172 / 104,
+//                 49152 174 / 177, 65536 173 / 217
+//   primary       9216 74 / 46, 32256 83 / 82, 64000 107 / 126
+//   diffuse       32256 265 / 172, 64000 324 / 279, 96000 584 / 473, 286 /
+//                 283, 324 / 319 (three scenes), 140000 314 / 356
+//   diffuse2      32256 425 / 317, 64000 467 / 381, 96000 939 / 762, 454 /
+//                 409, 140000 484 / 494
+// The albedo modes trace the same paths as diffuse.
+constexpr uint64_t kSpreadRays = 32768, kSpreadPaths = 96 << 10;
+
+uint64_t spread_limit(int mode)
+{
+    return mode == kModeTrace || mode == kModeOccluded || mode == kModePrimary ? kSpreadRays : kSpreadPaths;
+}
+
+// Workgroups of such a launch: a wave per 8 items, on as many CUs as there are
+// waves, then up to the 4 waves of each.
+int spread_grid(const prt_hip_ctx* ctx, uint64_t items)
+{
+    const int waves = (int)std::min<uint64_t>((items + 7) / 8, 1u << 30);
+    const int most = ctx->trace_grid;
+    return std::min(most, std::max(1, std::max(std::min(waves, ctx->num_cus), (waves + 3) / 4)));
+}
+
+// Tail mode and grid of a launch.
+int launch_shape(const prt_hip_ctx* ctx, int mode, uint64_t items, int& coop)
+{
+    coop = ctx->tail_coop ? kCoopTail : 0;
+    if (coop && items <= spread_limit(mode)) {
+        coop = kCoopSpread;
+        return spread_grid(ctx, items);
+    }
+    return grid_for(ctx, mode, items);
+}
+
 template <int kMode>
 hipError_t launch_mode(prt_hip_ctx* ctx, const TraceLaunch& t, const PathLaunch& paths, bool instrumented)
 {
     const SceneDevice sc = ctx->scene.device();
     uint32_t* err = ctx->d_counters + 32;
     const BatchLaunch bl{};
-    const int grid = grid_for(ctx, kMode, launch_items(kMode, t, paths));
     PathLaunch p = paths;
-    p.coop = ctx->tail_coop;
+    const int grid = p.look ? diffuse_grid(ctx, p.entries)
+                            : launch_shape(ctx, kMode, launch_items(kMode, t, p), p.coop);
     if (instrumented) {
         k_trace<true, kMode><<<grid, kTraceBlock, 0, ctx->stream>>>(
             sc, t, p, bl, ctx->d_spill, ctx->stack_entries, kRefill, err);
@@ -1401,7 +1465,7 @@ hipError_t launch_batch_variant(prt_hip_ctx* ctx, const BatchLaunch& bl, int blo
     const SceneDevice sc{};
     const TraceLaunch t{};
     PathLaunch p{};
-    p.coop = ctx->tail_coop;
+    p.coop = ctx->tail_coop ? kCoopTail : 0;
     if (instrumented)
         k_trace<true, kModeBatch, kBlock, kStack><<<grid, kBlock, 0, ctx->stream>>>(
             sc, t, p, bl, ctx->d_spill, ctx->stack_entries, refill, err);
@@ -1458,7 +1522,10 @@ int ensure_trace_resources(prt_hip_ctx* ctx)
 
 int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries) { return grid_for(ctx, kModeDiffuse, entries); }
 
-int query_grid(const prt_hip_ctx* ctx, int64_t rays) { return grid_for(ctx, kModeTrace, (uint64_t)rays); }
+// Frames that gain more from groups than from the lookahead: us per frame of
+// 13-frame chains, in groups / lookahead: 3072 path slots 161 / 191, 32256 211 /
+// 220, 282 / 311, 227 / 235 (three scenes), 64000 266 / 240, 348 / 328, 298 / 243.
+bool lookahead_pays(const prt_hip_ctx* ctx, uint32_t entries) { return !ctx->tail_coop || entries > 32768; }
 
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented)
 {
@@ -1466,10 +1533,15 @@ hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumente
 }
 
 hipError_t launch_trace_scratch(prt_hip_ctx* ctx, const TraceLaunch& t, uint2* spill, int stack_entries,
-                                uint32_t* err, int grid)
+                                uint32_t* err, int max_grid)
 {
     PathLaunch p{};
-    p.coop = ctx->tail_coop;
+    int grid = launch_shape(ctx, kModeTrace, t.count, p.coop);
+    if (grid > max_grid) {
+        // fewer workgroups than a small launch is spread over: one by one
+        if (p.coop == kCoopSpread) p.coop = kCoopTail;
+        grid = max_grid;
+    }
     k_trace<false, kModeTrace><<<grid, kTraceBlock, 0, ctx->stream>>>(ctx->scene.device(), t, p, BatchLaunch{}, spill,
                                                                      stack_entries, kRefill, err);
     return hipGetLastError();

@@ -273,7 +273,9 @@ int prt_hip_set_tail(prt_hip_ctx* ctx, int mode);
  * first call after any change renders as without the lookahead.  The
  * accumulator after each call and its ray count are those of rendering the
  * frames one by one.  Off for the primary, diffuse2 and Fast renderers, the
- * wavefront pipeline and under PRT_PROFILE_COUNTERS. */
+ * wavefront pipeline, under PRT_PROFILE_COUNTERS, and for frames of at most
+ * 32768 path slots with the cooperative tail, which trace each path on 8 lanes
+ * from the start. */
 int prt_hip_set_lookahead(prt_hip_ctx* ctx, int enable);
 
 /* --- frame buffer read-back -------------------------------------------- */

@@ -1,8 +1,9 @@
 """The cooperative tail of every persistent launch: a wave with at most 8 rays
-or paths left goes on with 8 lanes per path, in the middle of a ray.  Item
-counts around its borders (one path, one group, one wave, launches whose last
-waves hold few rays) in each mode against the lane-by-lane tail, and the
-queries against the oracle."""
+or paths left goes on with 8 lanes per path, in the middle of a ray, and a
+small launch is traced that way from its start.  Item counts around the borders
+(one path, one group, one wave, a share of 8 for every wave, the largest small
+launch of each mode, host queries answered in place) against lane-by-lane
+launches, and the queries against the oracle."""
 import numpy as np
 import pytest
 
@@ -27,7 +28,7 @@ def scene(scenes, orc):
     return mesh, orc.Scene(mesh.idx, mesh.pos)
 
 
-@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 63, 64, 65, 255, 257, 4097, 20011])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 63, 64, 65, 255, 257, 4097, 16384, 16385, 20011, 32768, 32769])
 def test_queries(dev, scene, n):
     mesh, oracle = scene
     dev.upload_scene(mesh.idx, mesh.pos)
@@ -46,7 +47,8 @@ def test_queries(dev, scene, n):
         dev.set_tail("cooperative")
 
 
-@pytest.mark.parametrize("size", [(1, 1), (3, 2), (8, 8), (9, 8), (65, 33), (311, 203)])
+@pytest.mark.parametrize("size", [(1, 1), (3, 2), (8, 8), (9, 8), (65, 33), (256, 128), (256, 136),
+                                  (383, 256), (385, 256)])
 def test_renders(dev, prt, scene, size):
     mesh, _ = scene
     w, h = size
