@@ -300,6 +300,7 @@ int prt_hip_destroy(prt_hip_ctx* ctx)
     prt_hip_batch_reset(ctx);
     free_ptr(ctx->d_albedo_own);
     free_ptr(ctx->d_rgb_planes);
+    free_ptr(ctx->d_path_hits);
     void* ptrs[] = {ctx->d_spill,
                     ctx->d_accum, ctx->d_bgr8, ctx->d_rays[0], ctx->d_rays[1], ctx->d_hits,
                     ctx->d_pix[0], ctx->d_pix[1], ctx->d_rng[0], ctx->d_rng[1], ctx->d_counters,
@@ -1403,6 +1404,20 @@ int prt_hip_adjoint_albedo(prt_hip_ctx* ctx, int pass0, int spp, int max_depth, 
     p.inv_spp = 1.0f / (float)spp;
     p.dldi = d_dldi;
     p.grad = d_grad;
+    if (max_depth <= kPathHitsDepth) {
+        // one column per lane of the largest launch
+        const int64_t lanes = (int64_t)ctx->trace_grid * kTraceBlock;
+        const int64_t need = lanes * std::max(1, max_depth);
+        if (need > ctx->path_hits_cap) {
+            free_ptr(ctx->d_path_hits);
+            ctx->d_path_hits = nullptr;
+            ctx->path_hits_cap = 0;
+            PRT_TRY(ctx, hipMalloc(&ctx->d_path_hits, sizeof(uint32_t) * (size_t)need));
+            ctx->path_hits_cap = need;
+        }
+        p.path_hits = ctx->d_path_hits;
+        p.path_hits_stride = (uint32_t)lanes;
+    }
     PRT_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     PRT_TRY(ctx, launch_frame_begin(ctx, (uint32_t)frame_entries(ctx)));
     PRT_TRY(ctx, launch_adjoint(ctx, p, (ctx->profiling & PRT_PROFILE_COUNTERS) != 0));

@@ -35,6 +35,7 @@ constexpr int kTraceBlock = 256;      // threads per trace workgroup
 constexpr int64_t kLargeSceneBytes = int64_t(256) << 20;  // nodes + triangles beyond MI355X's 256 MiB Infinity Cache
 constexpr size_t kBuildKeepBytes = size_t(512) << 20;  // build scratch a context keeps (about 150 B per triangle)
 constexpr int kMaxQueueDepth = 16;    // per-depth ray statistics bins; the last bin holds depths >= 15
+constexpr int kPathHitsDepth = 64;    // deepest paths whose hits the adjoint records (64 MiB for 262144 lanes)
 constexpr int kMaxDepth = 1024;       // largest max_depth accepted (an R^k throughput below 1 is 0 in fp32 long before)
 
 // Triangle record: the three fp32 vertices (36 B), in BVH8 leaf order.
@@ -229,6 +230,8 @@ struct prt_hip_ctx {
     const float* d_albedo = nullptr;
     float4* d_rgb_planes = nullptr;  // per-sample RGB planes of the albedo forward
     int64_t rgb_planes_cap = 0;      // ... in float4
+    uint32_t* d_path_hits = nullptr; // hits of the adjoint's paths in flight
+    int64_t path_hits_cap = 0;       // ... in entries
     hipEvent_t kev[4 * 16] = {};    // per-launch timing events (trace/shade x begin/end)
 
     // cooperative tail of the persistent launches (prt_hip_set_tail)
@@ -331,6 +334,10 @@ struct PathLaunch {
     float inv_spp;
     const float* dldi;               // dLoss/dImage, 3 floats per pixel
     float* grad;                     // dLoss/dAlbedo, 3 floats per triangle (accumulated)
+    // adjoint: the triangles each lane's path has hit, entry (depth, lane) at
+    // depth * path_hits_stride + lane (nullptr: an escaped path is traced again)
+    uint32_t* path_hits;
+    uint32_t path_hits_stride;
     // RGB forward: when set, work items are (sample, path) for passes pass ..
     // pass + spp - 1, and each path writes its RGB to plane sample (W*H
     // float4 each) instead of adding to the accumulator

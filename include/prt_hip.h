@@ -304,10 +304,12 @@ int prt_hip_render_albedo_image_host(prt_hip_ctx* ctx, int pass0, int spp, int m
                                      prt_render_stats* out_stats);
 /* Path-replay adjoint of prt_hip_render_albedo_image: grad += dLoss/dalbedo
  * for dLoss/dImage = dldi (3 floats per pixel).  Each path is traced once to
- * get its per-channel albedo product, then re-traced from its sampler seed
- * (pass, pixelId) -- nothing about the path is stored -- and every hit
- * atomically adds dldi * (product of the path's other albedos) / spp.
- * rays in out_stats counts both traces. */
+ * get its per-channel albedo product; if it escapes, it is replayed and every
+ * hit atomically adds dldi * (product of the path's other albedos) / spp.  The
+ * replay reads the hits that the trace recorded (one triangle index per bounce
+ * of the paths in flight), or, for max_depth > 64, traces the path again from
+ * its sampler seed (pass, pixelId).  rays in out_stats counts the rays of the
+ * traces and of the replays. */
 int prt_hip_adjoint_albedo(prt_hip_ctx* ctx, int pass0, int spp, int max_depth, const float* d_dldi,
                            float* d_grad, prt_render_stats* out_stats);
 int prt_hip_adjoint_albedo_host(prt_hip_ctx* ctx, int pass0, int spp, int max_depth, const float* dldi,
