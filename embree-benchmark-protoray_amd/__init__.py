@@ -312,7 +312,7 @@ class HipDevice:
     # -- closest hit
     def intersect(self, rays: np.ndarray) -> np.ndarray:
         rays = np.ascontiguousarray(rays, dtype=np.float32).reshape(-1, 8)
-        hits = np.zeros((rays.shape[0], 4), dtype=np.float32)
+        hits = np.empty((rays.shape[0], 4), dtype=np.float32)
         self._check(self.lib.prt_hip_intersect_closest(self.ctx, _ptr(rays), _ptr(hits), rays.shape[0]),
                     "intersect_closest")
         return hits
@@ -321,7 +321,7 @@ class HipDevice:
         """Any-hit query (IntersectorStreamCuda::occluded): per ray, the distance
         of some blocking triangle in [tnear, tfar], or -1."""
         rays = np.ascontiguousarray(rays, dtype=np.float32).reshape(-1, 8)
-        out = np.zeros(rays.shape[0], dtype=np.float32)
+        out = np.empty(rays.shape[0], dtype=np.float32)
         self._check(self.lib.prt_hip_occluded(self.ctx, _ptr(rays), _ptr(out), rays.shape[0]), "occluded")
         return out
 
@@ -389,12 +389,12 @@ class HipDevice:
         self._check(self.lib.prt_hip_set_profiling(self.ctx, flags), "set_profiling")
 
     def accum(self) -> np.ndarray:
-        out = np.zeros((self.height, self.width, 4), dtype=np.float32)
+        out = np.empty((self.height, self.width, 4), dtype=np.float32)
         self._check(self.lib.prt_hip_accum_read(self.ctx, _ptr(out)), "accum_read")
         return out
 
     def frame_bgr8(self) -> np.ndarray:
-        out = np.zeros((self.height, self.width), dtype=np.int32)
+        out = np.empty((self.height, self.width), dtype=np.int32)
         self._check(self.lib.prt_hip_frame_read_bgr8(self.ctx, _ptr(out)), "frame_read_bgr8")
         return out
 
@@ -414,7 +414,7 @@ class HipDevice:
                 "tris": st.tris}
 
     def render_albedo_image(self, pass0: int, spp: int, max_depth: int) -> tuple[np.ndarray, dict]:
-        img = np.zeros((self.height, self.width, 3), dtype=np.float32)
+        img = np.empty((self.height, self.width, 3), dtype=np.float32)
         st = PrtRenderStats()
         self._check(self.lib.prt_hip_render_albedo_image_host(self.ctx, pass0, spp, max_depth, _ptr(img),
                                                               ctypes.byref(st)), "render_albedo_image")
@@ -484,7 +484,7 @@ class HipDevice:
 
     def batch_accum(self, job: int) -> np.ndarray:
         h, w = self._batch_sizes[job]
-        out = np.zeros((h, w, 4), dtype=np.float32)
+        out = np.empty((h, w, 4), dtype=np.float32)
         self._check(self.lib.prt_hip_batch_accum_read(self.ctx, job, _ptr(out)), "batch_accum_read")
         return out
 

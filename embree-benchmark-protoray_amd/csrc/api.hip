@@ -7,6 +7,7 @@
 // from device memory, so a frame issues no host round trip until the final
 // read of the per-depth counters for the ray statistics.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
@@ -42,6 +43,7 @@ void SceneBuffers::release()
     bvh_ready = false;
     node_count = 0;
     bvh_depth = 0;
+    idx_cap = pos_cap = bvh_cap = 0;
 }
 
 int set_error(prt_hip_ctx* ctx, const std::string& msg)
@@ -114,6 +116,48 @@ void free_ptr(void* p)
     if (p) (void)hipFree(p);
 }
 
+// Room for `count` elements (at least one) in a buffer that has room for cap of
+// them: kept if it is large enough and not over four times too large, else
+// replaced.
+template <class T>
+int ensure_room(prt_hip_ctx* ctx, T*& p, int64_t& cap, int64_t count)
+{
+    count = std::max<int64_t>(count, 16);
+    if (p && count <= cap && cap <= std::max<int64_t>(4 * count, 1 << 20)) return 0;
+    free_ptr(p);
+    p = nullptr;
+    cap = 0;
+    PRT_TRY(ctx, hipMalloc(&p, sizeof(T) * (size_t)count));
+    cap = count;
+    return 0;
+}
+
+// All of idx[0 .. n) in [0, vertex_count), checked in parts by several threads
+// when there are many.
+bool indices_valid(prt_hip_ctx* ctx, const int32_t* idx, int64_t n, int64_t vertex_count)
+{
+    struct Part {
+        const int32_t* idx;
+        int64_t n, step;
+        std::atomic<uint32_t> most{0};
+    } part;
+    part.idx = idx;
+    part.n = n;
+    part.step = (int64_t)1 << 18;
+    auto check = [](void* p, int k) {
+        Part& w = *static_cast<Part*>(p);
+        const int64_t end = std::min(w.n, (k + 1) * w.step);
+        uint32_t most = 0;  // a negative index is a large unsigned one
+        for (int64_t i = k * w.step; i < end; ++i) most = std::max(most, (uint32_t)w.idx[i]);
+        uint32_t seen = w.most.load();
+        while (most > seen && !w.most.compare_exchange_weak(seen, most)) {}
+    };
+    const int64_t parts = (n + part.step - 1) / part.step;
+    if (parts == 1) check(&part, 0);
+    else ctx->copy.workers().each((int)parts, check, &part);
+    return n == 0 || (int64_t)part.most.load() < vertex_count;
+}
+
 // Replaces the shading attributes of a scene: 3 floats per vertex of normals
 // and 2 of texture coordinates; a null pointer removes that attribute.
 int set_attributes(prt_hip_ctx* ctx, SceneBuffers& sb, const float* normals3, const float* texcoords2)
@@ -125,11 +169,11 @@ int set_attributes(prt_hip_ctx* ctx, SceneBuffers& sb, const float* normals3, co
     const int64_t nv = sb.vertex_count;
     if (normals3 && nv > 0) {
         PRT_TRY(ctx, hipMalloc(&sb.d_normals, 12 * nv));
-        PRT_TRY(ctx, hipMemcpyAsync(sb.d_normals, normals3, 12 * nv, hipMemcpyHostToDevice, ctx->stream));
+        PRT_TRY(ctx, ctx->copy.to_device(sb.d_normals, normals3, 12 * nv, ctx->stream));
     }
     if (texcoords2 && nv > 0) {
         PRT_TRY(ctx, hipMalloc(&sb.d_texcoords, 8 * nv));
-        PRT_TRY(ctx, hipMemcpyAsync(sb.d_texcoords, texcoords2, 8 * nv, hipMemcpyHostToDevice, ctx->stream));
+        PRT_TRY(ctx, ctx->copy.to_device(sb.d_texcoords, texcoords2, 8 * nv, ctx->stream));
     }
     PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return 0;
@@ -178,12 +222,17 @@ int add_wave_timing(prt_hip_ctx* ctx, int n, double& trace_ms, double& shade_ms)
     return 0;
 }
 
+// Enqueues the read of a query's error flag, before the copy of its results;
+// check_trace_error looks at it once the stream has been waited for.
+int fetch_trace_error(prt_hip_ctx* ctx)
+{
+    PRT_TRY(ctx, hipMemcpyAsync(ctx->h_readback, ctx->d_counters + 32, 4, hipMemcpyDeviceToHost, ctx->stream));
+    return 0;
+}
+
 int check_trace_error(prt_hip_ctx* ctx)
 {
-    uint32_t e = 0;
-    PRT_TRY(ctx, hipMemcpyAsync(&e, ctx->d_counters + 32, 4, hipMemcpyDeviceToHost, ctx->stream));
-    PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    if (e) return set_error(ctx, "trace: traversal stack overflow");
+    if (*static_cast<const uint32_t*>(ctx->h_readback)) return set_error(ctx, "trace: traversal stack overflow");
     return 0;
 }
 
@@ -241,6 +290,56 @@ int occluded_impl(prt_hip_ctx* ctx, const prt_ray* d_rays, float* d_t, int64_t n
     t.count = (uint32_t)n;
     t.fetch_ptr = ctx->d_counters + 16;
     PRT_TRY(ctx, launch_occluded(ctx, t, false));
+    return 0;
+}
+
+// A small query from host memory.  Its rays go to a pinned buffer that the
+// kernel reads and answers in place, and the query needs no work counter, so
+// one launch and one wait are the whole call: no staged copies, no counter
+// clear, no read of the error flag.
+// 1 ray 68 -> 38 us, 1024 102 -> 65, 4096 107 -> 70, 32768 175 -> 142 (start of
+// the copies to their end, with Python); larger queries are not spread.
+constexpr int64_t kDirectRays = 32768;
+
+struct DirectIo {
+    uint32_t err;
+    uint32_t reserved[15];
+    prt_ray rays[kDirectRays];
+    union {
+        prt_hit hits[kDirectRays];
+        float any_t[kDirectRays];
+    };
+};
+
+bool query_direct(const prt_hip_ctx* ctx, int64_t n)
+{
+    return ctx->scene.bvh_ready && n <= kDirectRays && query_spreads(ctx, n);
+}
+
+// hits or any_t: closest or any hit
+int run_direct(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* hits, float* any_t, int64_t n)
+{
+    if (ensure_trace_resources(ctx)) return 1;
+    if (!ctx->h_direct) PRT_TRY(ctx, hipHostMalloc(&ctx->h_direct, sizeof(DirectIo), hipHostMallocDefault));
+    DirectIo* io = static_cast<DirectIo*>(ctx->h_direct);
+    io->err = 0;
+    std::memcpy(io->rays, rays, sizeof(prt_ray) * (size_t)n);
+    TraceLaunch t{};
+    t.rays = reinterpret_cast<const float4*>(io->rays);
+    t.count = (uint32_t)n;
+    t.fetch_ptr = ctx->d_counters + 16;  // unused: every wave has its share
+    t.err = &io->err;
+    if (hits) {
+        t.hits = reinterpret_cast<float4*>(io->hits);
+        PRT_TRY(ctx, launch_trace(ctx, t, false));
+    } else {
+        t.any_t = io->any_t;
+        PRT_TRY(ctx, launch_occluded(ctx, t, false));
+    }
+    PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    if (hits) std::memcpy(hits, io->hits, sizeof(prt_hit) * (size_t)n);
+    else std::memcpy(any_t, io->any_t, sizeof(float) * (size_t)n);
+    if (io->err) return set_error(ctx, "trace: traversal stack overflow");
     return 0;
 }
 
@@ -313,6 +412,7 @@ int prt_hip_destroy(prt_hip_ctx* ctx)
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->h_readback) (void)hipHostFree(ctx->h_readback);
+    if (ctx->h_direct) (void)hipHostFree(ctx->h_direct);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return 0;
@@ -336,31 +436,26 @@ int prt_hip_scene_upload(prt_hip_ctx* ctx, const int32_t* idx3, int64_t tri_coun
         return set_error(ctx, "scene_upload: bad arguments");
     if (tri_count >= ((int64_t)1 << 31) || vertex_count >= ((int64_t)1 << 31))
         return set_error(ctx, "scene_upload: more than 2^31-1 triangles or vertices");
-    for (int64_t i = 0; i < 3 * tri_count; ++i)
-        if (idx3[i] < 0 || idx3[i] >= vertex_count)
-            return set_error(ctx, "scene_upload: vertex index out of range");
+    if (!indices_valid(ctx, idx3, 3 * tri_count, vertex_count))
+        return set_error(ctx, "scene_upload: vertex index out of range");
     ctx->scene_gen += 1;
-    free_ptr(ctx->scene.d_idx);
-    free_ptr(ctx->scene.d_pos);
-    free_ptr(ctx->scene.d_normals);
-    free_ptr(ctx->scene.d_texcoords);
-    ctx->scene.d_idx = nullptr;
-    ctx->scene.d_pos = nullptr;
-    ctx->scene.d_normals = nullptr;
-    ctx->scene.d_texcoords = nullptr;
-    ctx->scene.bvh_ready = false;
-    ctx->scene.tri_count = tri_count;
-    ctx->scene.vertex_count = vertex_count;
+    SceneBuffers& sc = ctx->scene;
+    free_ptr(sc.d_normals);
+    free_ptr(sc.d_texcoords);
+    sc.d_normals = nullptr;
+    sc.d_texcoords = nullptr;
+    sc.bvh_ready = false;
+    sc.tri_count = tri_count;
+    sc.vertex_count = vertex_count;
     free_ptr(ctx->d_albedo_own);
     ctx->d_albedo_own = nullptr;
     ctx->d_albedo = nullptr;
-    PRT_TRY(ctx, hipMalloc(&ctx->scene.d_idx, std::max<int64_t>(16, 12 * tri_count)));
-    PRT_TRY(ctx, hipMalloc(&ctx->scene.d_pos, std::max<int64_t>(16, 12 * vertex_count)));
+    if (ensure_room(ctx, sc.d_idx, sc.idx_cap, 3 * tri_count) || ensure_room(ctx, sc.d_pos, sc.pos_cap, 3 * vertex_count))
+        return 1;
     if (tri_count) {
-        PRT_TRY(ctx, hipMemcpyAsync(ctx->scene.d_idx, idx3, 12 * tri_count, hipMemcpyHostToDevice, ctx->stream));
-        PRT_TRY(ctx, hipMemcpyAsync(ctx->scene.d_pos, pos3, 12 * vertex_count, hipMemcpyHostToDevice, ctx->stream));
+        PRT_TRY(ctx, ctx->copy.to_device(sc.d_idx, idx3, 12 * tri_count, ctx->stream));
+        PRT_TRY(ctx, ctx->copy.to_device(sc.d_pos, pos3, 12 * vertex_count, ctx->stream));
     }
-    PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return 0;
 }
 
@@ -402,13 +497,14 @@ int prt_hip_intersect_closest(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* hi
     if (use_device(ctx)) return 1;
     if (n == 0) return 0;
     if (!rays || !hits) return set_error(ctx, "intersect: null array");
+    if (n > 0 && query_direct(ctx, n)) return run_direct(ctx, rays, hits, nullptr, n);
     if (ensure_io(ctx, n)) return 1;
-    PRT_TRY(ctx, hipMemcpyAsync(ctx->d_io_rays, rays, sizeof(prt_ray) * n, hipMemcpyHostToDevice, ctx->stream));
+    PRT_TRY(ctx, ctx->copy.to_device(ctx->d_io_rays, rays, sizeof(prt_ray) * n, ctx->stream));
     if (intersect_impl(ctx, reinterpret_cast<prt_ray*>(ctx->d_io_rays),
                        reinterpret_cast<prt_hit*>(ctx->d_io_hits), n, nullptr))
         return 1;
-    PRT_TRY(ctx, hipMemcpyAsync(hits, ctx->d_io_hits, sizeof(prt_hit) * n, hipMemcpyDeviceToHost, ctx->stream));
-    PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    if (fetch_trace_error(ctx)) return 1;
+    PRT_TRY(ctx, ctx->copy.to_host(hits, ctx->d_io_hits, sizeof(prt_hit) * n, ctx->stream));
     return check_trace_error(ctx);
 }
 
@@ -459,12 +555,13 @@ int prt_hip_occluded(prt_hip_ctx* ctx, const prt_ray* rays, float* out_t, int64_
     if (use_device(ctx)) return 1;
     if (n == 0) return 0;
     if (!rays || !out_t) return set_error(ctx, "occluded: null array");
+    if (n > 0 && query_direct(ctx, n)) return run_direct(ctx, rays, nullptr, out_t, n);
     if (ensure_io(ctx, n)) return 1;
     float* d_t = reinterpret_cast<float*>(ctx->d_io_hits);  // n floats fit in the n-hit buffer
-    PRT_TRY(ctx, hipMemcpyAsync(ctx->d_io_rays, rays, sizeof(prt_ray) * n, hipMemcpyHostToDevice, ctx->stream));
+    PRT_TRY(ctx, ctx->copy.to_device(ctx->d_io_rays, rays, sizeof(prt_ray) * n, ctx->stream));
     if (occluded_impl(ctx, reinterpret_cast<prt_ray*>(ctx->d_io_rays), d_t, n)) return 1;
-    PRT_TRY(ctx, hipMemcpyAsync(out_t, d_t, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
-    PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    if (fetch_trace_error(ctx)) return 1;
+    PRT_TRY(ctx, ctx->copy.to_host(out_t, d_t, sizeof(float) * n, ctx->stream));
     return check_trace_error(ctx);
 }
 
@@ -481,6 +578,7 @@ int prt_hip_intersect_counters(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* h
                        reinterpret_cast<prt_hit*>(ctx->d_io_hits), n, ctx->d_stats))
         return 1;
     unsigned long long st[8];
+    if (fetch_trace_error(ctx)) return 1;
     PRT_TRY(ctx, hipMemcpyAsync(hits, ctx->d_io_hits, sizeof(prt_hit) * n, hipMemcpyDeviceToHost, ctx->stream));
     PRT_TRY(ctx, hipMemcpyAsync(st, ctx->d_stats, sizeof(st), hipMemcpyDeviceToHost, ctx->stream));
     PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -911,17 +1009,25 @@ void batch_drop_graph(prt_hip_ctx* ctx)
 void batch_free_jobs(prt_hip_ctx* ctx)
 {
     batch_drop_graph(ctx);
-    void* ptrs[] = {ctx->d_batch_jobs, ctx->d_batch_work_begin, ctx->d_batch_pixel_begin, ctx->d_batch_samples,
-                    ctx->d_batch_accum};
-    for (void* p : ptrs) free_ptr(p);
+    free_ptr(ctx->d_batch_jobs);  // the three tables are one allocation
     ctx->d_batch_jobs = nullptr;
     ctx->d_batch_work_begin = nullptr;
     ctx->d_batch_pixel_begin = nullptr;
-    ctx->d_batch_samples = nullptr;
-    ctx->d_batch_accum = nullptr;
     ctx->batch_jobs.clear();
     ctx->batch_samples_len = ctx->batch_pixels = 0;
     ctx->batch_total_work = 0;
+}
+
+// Frees the sample planes and accumulators too, which a later job set of a
+// similar size reuses.
+void batch_free_all(prt_hip_ctx* ctx)
+{
+    batch_free_jobs(ctx);
+    free_ptr(ctx->d_batch_samples);
+    free_ptr(ctx->d_batch_accum);
+    ctx->d_batch_samples = nullptr;
+    ctx->d_batch_accum = nullptr;
+    ctx->batch_samples_cap = ctx->batch_accum_cap = 0;
 }
 
 BatchLaunch batch_launch_args(prt_hip_ctx* ctx)
@@ -975,16 +1081,15 @@ int prt_hip_batch_scene_add(prt_hip_ctx* ctx, const int32_t* idx3, int64_t tri_c
         return set_error(ctx, "batch_scene_add: bad arguments");
     if (tri_count >= ((int64_t)1 << 31) || vertex_count >= ((int64_t)1 << 31))
         return set_error(ctx, "batch_scene_add: more than 2^31-1 triangles or vertices");
-    for (int64_t i = 0; i < 3 * tri_count; ++i)
-        if (idx3[i] < 0 || idx3[i] >= vertex_count) return set_error(ctx, "batch_scene_add: vertex index out of range");
+    if (!indices_valid(ctx, idx3, 3 * tri_count, vertex_count))
+        return set_error(ctx, "batch_scene_add: vertex index out of range");
     SceneBuffers sb;
     sb.tri_count = tri_count;
     sb.vertex_count = vertex_count;
     hipError_t e = hipMalloc(&sb.d_idx, 12 * tri_count);
     if (e == hipSuccess) e = hipMalloc(&sb.d_pos, 12 * vertex_count);
-    if (e == hipSuccess) e = hipMemcpyAsync(sb.d_idx, idx3, 12 * tri_count, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(sb.d_pos, pos3, 12 * vertex_count, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = ctx->copy.to_device(sb.d_idx, idx3, 12 * tri_count, ctx->stream);
+    if (e == hipSuccess) e = ctx->copy.to_device(sb.d_pos, pos3, 12 * vertex_count, ctx->stream);
     if (e != hipSuccess) {
         sb.release();
         return check_hip(ctx, e, "batch_scene_add");
@@ -1023,7 +1128,7 @@ int prt_hip_batch_reset(prt_hip_ctx* ctx)
 {
     if (!ctx) return 1;
     (void)hipSetDevice(ctx->device);
-    batch_free_jobs(ctx);
+    batch_free_all(ctx);
     for (SceneBuffers& b : ctx->batch_scenes) b.release();
     ctx->batch_scenes.clear();
     free_ptr(ctx->d_batch_scenes);
@@ -1077,17 +1182,30 @@ int prt_hip_batch_set_jobs(prt_hip_ctx* ctx, const prt_batch_job* jobs, int n_jo
     work_begin[n_jobs] = (uint32_t)work;
     pixel_begin[n_jobs] = pixels;
     batch_free_jobs(ctx);
-    PRT_TRY(ctx, hipMalloc(&ctx->d_batch_jobs, sizeof(BatchJobDevice) * n_jobs));
-    PRT_TRY(ctx, hipMalloc(&ctx->d_batch_work_begin, sizeof(uint32_t) * (n_jobs + 1)));
-    PRT_TRY(ctx, hipMalloc(&ctx->d_batch_pixel_begin, sizeof(uint64_t) * (n_jobs + 1)));
-    PRT_TRY(ctx, hipMalloc(&ctx->d_batch_samples, sizeof(float) * samples));
-    PRT_TRY(ctx, hipMalloc(&ctx->d_batch_accum, sizeof(float4) * pixels));
-    PRT_TRY(ctx, hipMemcpy(ctx->d_batch_jobs, dj.data(), sizeof(BatchJobDevice) * n_jobs, hipMemcpyHostToDevice));
-    PRT_TRY(ctx, hipMemcpy(ctx->d_batch_work_begin, work_begin.data(), sizeof(uint32_t) * (n_jobs + 1),
-                           hipMemcpyHostToDevice));
-    PRT_TRY(ctx, hipMemcpy(ctx->d_batch_pixel_begin, pixel_begin.data(), sizeof(uint64_t) * (n_jobs + 1),
-                           hipMemcpyHostToDevice));
-    PRT_TRY(ctx, hipMemset(ctx->d_batch_accum, 0, sizeof(float4) * pixels));
+    // the tables in one allocation and one copy, 256-byte aligned
+    auto aligned = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const size_t at_work = aligned(sizeof(BatchJobDevice) * n_jobs);
+    const size_t at_pixel = at_work + aligned(sizeof(uint32_t) * (n_jobs + 1));
+    std::vector<char> tables(at_pixel + sizeof(uint64_t) * (n_jobs + 1));
+    std::memcpy(tables.data(), dj.data(), sizeof(BatchJobDevice) * n_jobs);
+    std::memcpy(tables.data() + at_work, work_begin.data(), sizeof(uint32_t) * (n_jobs + 1));
+    std::memcpy(tables.data() + at_pixel, pixel_begin.data(), sizeof(uint64_t) * (n_jobs + 1));
+    char* d_tables = nullptr;
+    PRT_TRY(ctx, hipMalloc(&d_tables, tables.size()));
+    ctx->d_batch_jobs = reinterpret_cast<BatchJobDevice*>(d_tables);
+    ctx->d_batch_work_begin = reinterpret_cast<uint32_t*>(d_tables + at_work);
+    ctx->d_batch_pixel_begin = reinterpret_cast<uint64_t*>(d_tables + at_pixel);
+    int64_t cap = (int64_t)ctx->batch_samples_cap;
+    int rc = ensure_room(ctx, ctx->d_batch_samples, cap, (int64_t)samples);
+    ctx->batch_samples_cap = (uint64_t)cap;
+    if (rc) return rc;
+    cap = (int64_t)ctx->batch_accum_cap;
+    rc = ensure_room(ctx, ctx->d_batch_accum, cap, (int64_t)pixels);
+    ctx->batch_accum_cap = (uint64_t)cap;
+    if (rc) return rc;
+    PRT_TRY(ctx, hipMemsetAsync(ctx->d_batch_accum, 0, sizeof(float4) * pixels, ctx->stream));
+    PRT_TRY(ctx, ctx->copy.to_device(d_tables, tables.data(), tables.size(), ctx->stream));
+    ctx->batch_rendered = false;
     ctx->batch_jobs = dj;
     ctx->batch_samples_len = samples;
     ctx->batch_pixels = pixels;
@@ -1105,7 +1223,10 @@ int prt_hip_batch_render(prt_hip_ctx* ctx, prt_batch_stats* out)
     // the graph holds the spill buffer and its per-lane stride as kernel
     // arguments: a later build of a deeper scene replaces both
     if (ctx->batch_graph_exec && ctx->batch_graph_spill_gen != ctx->spill_gen) batch_drop_graph(ctx);
-    if (graph && !ctx->batch_graph_exec) {
+    // a job set's first render is launched as it is: capturing pays from the
+    // second on
+    const bool replay = graph && ctx->batch_rendered;
+    if (replay && !ctx->batch_graph_exec) {
         PRT_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
         const int rc = batch_enqueue(ctx, ctx->batch_tuning, false, true);
         hipGraph_t g = nullptr;
@@ -1120,7 +1241,7 @@ int prt_hip_batch_render(prt_hip_ctx* ctx, prt_batch_stats* out)
         ctx->batch_graph_spill_gen = ctx->spill_gen;
     }
     PRT_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    if (graph) {
+    if (replay) {
         PRT_TRY(ctx, hipGraphLaunch(ctx->batch_graph_exec, ctx->stream));
     } else if (batch_enqueue(ctx, ctx->batch_tuning, counting, true)) {
         return 1;
@@ -1132,6 +1253,7 @@ int prt_hip_batch_render(prt_hip_ctx* ctx, prt_batch_stats* out)
     if (rb->counters[32]) return set_error(ctx, "batch_render: traversal stack overflow");
     float ms = 0.0f;
     PRT_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+    ctx->batch_rendered = true;
     int64_t paths = 0;
     for (BatchJobDevice& j : ctx->batch_jobs) {
         paths += (int64_t)j.spp * j.width * j.height;
@@ -1156,8 +1278,8 @@ int prt_hip_batch_accum_read(prt_hip_ctx* ctx, int job, float* dst)
     if (use_device(ctx)) return 1;
     if (job < 0 || job >= (int)ctx->batch_jobs.size() || !dst) return set_error(ctx, "batch_accum_read: bad job");
     const BatchJobDevice& j = ctx->batch_jobs[job];
-    PRT_TRY(ctx, hipMemcpy(dst, ctx->d_batch_accum + j.pixel_base, sizeof(float4) * (size_t)j.width * j.height,
-                           hipMemcpyDeviceToHost));
+    PRT_TRY(ctx, ctx->copy.to_host(dst, ctx->d_batch_accum + j.pixel_base, sizeof(float4) * (size_t)j.width * j.height,
+                                   ctx->stream));
     return 0;
 }
 
@@ -1322,7 +1444,7 @@ int prt_hip_set_albedo_host(prt_hip_ctx* ctx, const float* rgb)
     free_ptr(ctx->d_albedo_own);
     ctx->d_albedo_own = nullptr;
     PRT_TRY(ctx, hipMalloc(&ctx->d_albedo_own, sizeof(float) * 3 * ctx->scene.tri_count));
-    PRT_TRY(ctx, hipMemcpy(ctx->d_albedo_own, rgb, sizeof(float) * 3 * ctx->scene.tri_count, hipMemcpyHostToDevice));
+    PRT_TRY(ctx, ctx->copy.to_device(ctx->d_albedo_own, rgb, sizeof(float) * 3 * ctx->scene.tri_count, ctx->stream));
     ctx->d_albedo = ctx->d_albedo_own;
     return 0;
 }
@@ -1384,7 +1506,7 @@ int prt_hip_render_albedo_image_host(prt_hip_ctx* ctx, int pass0, int spp, int m
     PRT_TRY(ctx, hipMalloc(&d, sizeof(float) * n));
     int rc = prt_hip_render_albedo_image(ctx, pass0, spp, max_depth, d, out);
     if (rc == 0) {
-        hipError_t e = hipMemcpy(image, d, sizeof(float) * n, hipMemcpyDeviceToHost);
+        hipError_t e = ctx->copy.to_host(image, d, sizeof(float) * n, ctx->stream);
         if (e != hipSuccess) rc = check_hip(ctx, e, "render_albedo_image");
     }
     free_ptr(d);
@@ -1434,12 +1556,12 @@ int prt_hip_adjoint_albedo_host(prt_hip_ctx* ctx, int pass0, int spp, int max_de
     float *di = nullptr, *dg = nullptr;
     hipError_t e = hipMalloc(&di, sizeof(float) * ni);
     if (e == hipSuccess) e = hipMalloc(&dg, sizeof(float) * ng);
-    if (e == hipSuccess) e = hipMemcpy(di, dldi, sizeof(float) * ni, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(dg, grad, sizeof(float) * ng, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = ctx->copy.to_device(di, dldi, sizeof(float) * ni, ctx->stream);
+    if (e == hipSuccess) e = ctx->copy.to_device(dg, grad, sizeof(float) * ng, ctx->stream);
     int rc = e == hipSuccess ? prt_hip_adjoint_albedo(ctx, pass0, spp, max_depth, di, dg, out)
                              : check_hip(ctx, e, "adjoint_albedo");
     if (rc == 0) {
-        e = hipMemcpy(grad, dg, sizeof(float) * ng, hipMemcpyDeviceToHost);
+        e = ctx->copy.to_host(grad, dg, sizeof(float) * ng, ctx->stream);
         if (e != hipSuccess) rc = check_hip(ctx, e, "adjoint_albedo");
     }
     free_ptr(di);
@@ -1451,9 +1573,7 @@ int prt_hip_accum_read(prt_hip_ctx* ctx, float* dst)
 {
     if (use_device(ctx)) return 1;
     if (!ctx->d_accum || !dst) return set_error(ctx, "accum_read: no frame");
-    PRT_TRY(ctx, hipMemcpyAsync(dst, ctx->d_accum, sizeof(float4) * (int64_t)ctx->width * ctx->height,
-                                hipMemcpyDeviceToHost, ctx->stream));
-    PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    PRT_TRY(ctx, ctx->copy.to_host(dst, ctx->d_accum, sizeof(float4) * (size_t)ctx->width * ctx->height, ctx->stream));
     return 0;
 }
 
@@ -1462,9 +1582,7 @@ int prt_hip_frame_read_bgr8(prt_hip_ctx* ctx, int32_t* dst)
     if (use_device(ctx)) return 1;
     if (!ctx->d_accum || !dst) return set_error(ctx, "frame_read: no frame");
     PRT_TRY(ctx, launch_tonemap(ctx));
-    PRT_TRY(ctx, hipMemcpyAsync(dst, ctx->d_bgr8, sizeof(int32_t) * (int64_t)ctx->width * ctx->height,
-                                hipMemcpyDeviceToHost, ctx->stream));
-    PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    PRT_TRY(ctx, ctx->copy.to_host(dst, ctx->d_bgr8, sizeof(int32_t) * (size_t)ctx->width * ctx->height, ctx->stream));
     return 0;
 }
 

@@ -958,15 +958,23 @@ int build_bvh8(prt_hip_ctx* ctx, SceneBuffers& sb, prt_build_stats* stats)
     if (n <= 0) return set_error(ctx, "bvh_build: scene has no triangles");
     if (n >= (int64_t)1 << 31) return set_error(ctx, "bvh_build: more than 2^31-1 triangles");
 
-    if (sb.d_nodes) { (void)hipFree(sb.d_nodes); sb.d_nodes = nullptr; }
-    if (sb.d_tris) { (void)hipFree(sb.d_tris); sb.d_tris = nullptr; }
-    if (sb.d_prim_ids) { (void)hipFree(sb.d_prim_ids); sb.d_prim_ids = nullptr; }
     sb.bvh_ready = false;
-
     const int64_t max_nodes = std::max<int64_t>(1, n - 1);
-    PRT_TRY(ctx, hipMalloc(&sb.d_nodes, sizeof(Bvh8Node) * max_nodes));
-    PRT_TRY(ctx, hipMalloc(&sb.d_tris, sizeof(float) * 9 * n));
-    PRT_TRY(ctx, hipMalloc(&sb.d_prim_ids, sizeof(int32_t) * n));
+    // the last build's buffers serve again if they have room and are not over
+    // four times too large
+    if (!sb.d_nodes || n > sb.bvh_cap || sb.bvh_cap > std::max<int64_t>(4 * n, 1 << 18)) {
+        if (sb.d_nodes) (void)hipFree(sb.d_nodes);
+        if (sb.d_tris) (void)hipFree(sb.d_tris);
+        if (sb.d_prim_ids) (void)hipFree(sb.d_prim_ids);
+        sb.d_nodes = nullptr;
+        sb.d_tris = nullptr;
+        sb.d_prim_ids = nullptr;
+        sb.bvh_cap = 0;
+        PRT_TRY(ctx, hipMalloc(&sb.d_nodes, sizeof(Bvh8Node) * max_nodes));
+        PRT_TRY(ctx, hipMalloc(&sb.d_tris, sizeof(float) * 9 * n));
+        PRT_TRY(ctx, hipMalloc(&sb.d_prim_ids, sizeof(int32_t) * n));
+        sb.bvh_cap = n;
+    }
 
     const bool sah = ctx->bvh_collapse == PRT_COLLAPSE_SAH;
     Arena arena;

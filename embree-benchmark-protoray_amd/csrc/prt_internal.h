@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 
+#include "host_copy.h"
 #include "prt_math.h"
 #include "../../include/prt_hip.h"
 
@@ -104,6 +105,8 @@ __device__ __forceinline__ Frame attribute_frame(const int32_t* idx, const float
 // One scene on the device: the uploaded mesh and its BVH8.
 struct SceneBuffers {
     int64_t tri_count = 0, vertex_count = 0;
+    // what the buffers below have room for: indices, positions, BVH
+    int64_t idx_cap = 0, pos_cap = 0, bvh_cap = 0;
     int32_t* d_idx = nullptr;
     float* d_pos = nullptr;
     Bvh8Node* d_nodes = nullptr;
@@ -183,12 +186,14 @@ struct prt_hip_ctx {
     float* d_batch_samples = nullptr;
     float4* d_batch_accum = nullptr;
     uint64_t batch_samples_len = 0, batch_pixels = 0;
+    uint64_t batch_samples_cap = 0, batch_accum_cap = 0;  // room of the two buffers above
     uint32_t batch_total_work = 0;
     prt::BatchTuning batch_tuning;
     hipGraph_t batch_graph = nullptr;
     hipGraphExec_t batch_graph_exec = nullptr;
     uint64_t batch_graph_spill_gen = 0;  // spill_gen the graph was captured with (its kernel arguments)
     bool batch_use_graph = true;
+    bool batch_rendered = false;         // the jobs have been rendered once: the next render captures the graph
 
     // traversal spill stack (global part of the short stack)
     uint2* d_spill = nullptr;
@@ -220,6 +225,8 @@ struct prt_hip_ctx {
     float4* d_io_rays = nullptr;
     float4* d_io_hits = nullptr;
     int64_t io_cap = 0;
+    void* h_direct = nullptr;                 // pinned rays and hits of small host queries
+    prt::HostCopy copy;                       // copies from and to pageable memory
 
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int profiling = 0;
@@ -283,6 +290,7 @@ struct TraceLaunch {
     uint32_t count;
     uint32_t* fetch_ptr;        // device fetch counter, zero before launch
     unsigned long long* stats;  // nullptr unless instrumented
+    uint32_t* err;              // error flag (nullptr: the context's)
 };
 // PathLaunch::coop: a wave's last rays or paths on 8 lanes each (0: never), or
 // a small launch spread over the waves that way from its start
@@ -360,6 +368,9 @@ int ensure_trace_resources(prt_hip_ctx* ctx);
 // persistent workgroups of a diffuse frame of `entries` path slots under the
 // lookahead
 int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries);
+// a query of `rays` rays is spread over the waves from its start, without the
+// work counter
+bool query_spreads(const prt_hip_ctx* ctx, int64_t rays);
 // frames of so many path slots are faster with the lookahead
 bool lookahead_pays(const prt_hip_ctx* ctx, uint32_t entries);
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented);

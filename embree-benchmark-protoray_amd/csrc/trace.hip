@@ -1449,7 +1449,7 @@ template <int kMode>
 hipError_t launch_mode(prt_hip_ctx* ctx, const TraceLaunch& t, const PathLaunch& paths, bool instrumented)
 {
     const SceneDevice sc = ctx->scene.device();
-    uint32_t* err = ctx->d_counters + 32;
+    uint32_t* err = t.err ? t.err : ctx->d_counters + 32;
     const BatchLaunch bl{};
     PathLaunch p = paths;
     const int grid = p.look ? diffuse_grid(ctx, p.entries)
@@ -1549,6 +1549,11 @@ int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries) { return grid_for(ctx
 // 13-frame chains, in groups / lookahead: 3072 path slots 161 / 191, 32256 211 /
 // 220, 282 / 311, 227 / 235 (three scenes), 64000 266 / 240, 348 / 328, 298 / 243.
 bool lookahead_pays(const prt_hip_ctx* ctx, uint32_t entries) { return !ctx->tail_coop || entries > 32768; }
+
+bool query_spreads(const prt_hip_ctx* ctx, int64_t rays)
+{
+    return ctx->tail_coop && rays >= 0 && (uint64_t)rays <= kSpreadRays;
+}
 
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented)
 {
