@@ -1374,8 +1374,10 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
 //             262 k 0.457 0.320 0.337 0.377; 518 k 0.806 0.717 0.769 0.810;
 //             0.92 M 1.392 0.979 0.995 1.120; 1.05 M 1.476 0.919 0.792 0.768;
 //             2.07 M 2.260 1.389 1.182 1.167
-//   ray query 60 k 0.098 0.112 0.124 0.132; 200 k 0.314 0.268 0.264 0.274;
-//             1 M 1.071 0.628 0.500 0.481
+//   closest   50 k rays 0.132 0.141 0.153 0.164; 100 k 0.177 0.154 0.167 0.176;
+//             200 k 0.285 0.204 0.185 0.205; 300 k 0.389 0.261 0.232 0.224;
+//             600 k 0.676 0.412 0.344 0.333: no bounces, so the drain is short
+//   any hit   200 k 0.184 0.145 0.143 0.158; 1 M 0.622 0.412 0.405 0.409
 //   diffuse2  290 k 0.690 0.770 0.846 0.796; 1.35 M 1.585 1.124 1.115 1.224:
 //             two rays a hit make its drain twice as long, so it counts half
 //   primary   262 k 0.088 0.093 0.106 0.118; 8.3 M 1.737 1.729 1.743 1.766:
@@ -1386,8 +1388,13 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
 int grid_for(const prt_hip_ctx* ctx, int mode, uint64_t items)
 {
     if (mode == kModeDiffuse2) items /= 2;
-    int per_cu = items <= (128u << 10) ? 1 : (items <= (640u << 10) ? 2 : (items <= (1000u << 10) ? 3 : 4));
+    const bool query = mode == kModeTrace || mode == kModeOccluded;
+    const uint64_t upto1 = query ? 64u << 10 : 128u << 10;
+    const uint64_t upto2 = query ? 160u << 10 : 640u << 10;
+    const uint64_t upto3 = query ? 256u << 10 : 1000u << 10;
+    int per_cu = items <= upto1 ? 1 : (items <= upto2 ? 2 : (items <= upto3 ? 3 : 4));
     if (mode == kModePrimary) per_cu = std::min(per_cu, 2);
+    if (mode == kModeOccluded) per_cu = std::min(per_cu, 3);
     int limit = ctx->trace_per_cu;
     if (mode == kModeDiffuse && limit > 1) {
         const SceneBuffers& s = ctx->scene;
