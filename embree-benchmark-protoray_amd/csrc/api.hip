@@ -81,7 +81,7 @@ int read_back(prt_hip_ctx* ctx, const ReadBack** out)
     return 0;
 }
 
-constexpr size_t kScratchHeader = 256;
+constexpr size_t kScratchHeader = kWorkWords * sizeof(uint32_t);
 constexpr int kScratchMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kScratchMaxDevices] = {};
@@ -265,13 +265,13 @@ int intersect_impl(prt_hip_ctx* ctx, const prt_ray* d_rays, prt_hit* d_hits, int
     if (!ctx->scene.bvh_ready) return set_error(ctx, "intersect: no BVH (call prt_hip_bvh_build)");
     if (n < 0 || n > (int64_t)UINT32_MAX / 2) return set_error(ctx, "intersect: bad ray count");
     if (ensure_trace_resources(ctx)) return 1;
-    PRT_TRY(ctx, launch_zero_u32(ctx->d_counters, 33, ctx->stream));
+    PRT_TRY(ctx, launch_zero_u32(ctx->d_work, kWorkWords + 33, ctx->stream));
     TraceLaunch t{};
     t.rays = reinterpret_cast<const float4*>(d_rays);
     t.hits = reinterpret_cast<float4*>(d_hits);
     t.count_ptr = nullptr;
     t.count = (uint32_t)n;
-    t.fetch_ptr = ctx->d_counters + 16;
+    t.work = ctx->d_work;
     t.stats = d_stats;
     PRT_TRY(ctx, launch_trace(ctx, t, d_stats != nullptr));
     return 0;
@@ -282,13 +282,13 @@ int occluded_impl(prt_hip_ctx* ctx, const prt_ray* d_rays, float* d_t, int64_t n
     if (!ctx->scene.bvh_ready) return set_error(ctx, "occluded: no BVH (call prt_hip_bvh_build)");
     if (n < 0 || n > (int64_t)UINT32_MAX / 2) return set_error(ctx, "occluded: bad ray count");
     if (ensure_trace_resources(ctx)) return 1;
-    PRT_TRY(ctx, launch_zero_u32(ctx->d_counters, 33, ctx->stream));
+    PRT_TRY(ctx, launch_zero_u32(ctx->d_work, kWorkWords + 33, ctx->stream));
     TraceLaunch t{};
     t.rays = reinterpret_cast<const float4*>(d_rays);
     t.any_t = d_t;
     t.count_ptr = nullptr;
     t.count = (uint32_t)n;
-    t.fetch_ptr = ctx->d_counters + 16;
+    t.work = ctx->d_work;
     PRT_TRY(ctx, launch_occluded(ctx, t, false));
     return 0;
 }
@@ -327,7 +327,7 @@ int run_direct(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* hits, float* any_
     TraceLaunch t{};
     t.rays = reinterpret_cast<const float4*>(io->rays);
     t.count = (uint32_t)n;
-    t.fetch_ptr = ctx->d_counters + 16;  // unused: every wave has its share
+    t.work = ctx->d_work;  // unused: every wave has its share
     t.err = &io->err;
     if (hits) {
         t.hits = reinterpret_cast<float4*>(io->hits);
@@ -364,9 +364,10 @@ int prt_hip_create(int device_index, prt_hip_ctx** out_ctx)
         hipGetDeviceProperties(&prop, device_index) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
-        // counters ([48] batch work counter) and statistics share one
-        // allocation, so a frame reads both back with one copy
-        hipMalloc(&ctx->d_counters, 64 * sizeof(uint32_t) + 32 * sizeof(unsigned long long)) != hipSuccess ||
+        // work counters, counters and statistics share one allocation, so a
+        // query clears the first two with one launch and a frame reads the
+        // last two back with one copy
+        hipMalloc(&ctx->d_work, (kWorkWords + 64) * sizeof(uint32_t) + 32 * sizeof(unsigned long long)) != hipSuccess ||
         // pinned, so the per-call read-back is one direct copy
         hipHostMalloc(&ctx->h_readback, 64 * sizeof(uint32_t) + 32 * sizeof(unsigned long long),
                       hipHostMallocDefault) != hipSuccess) {
@@ -378,10 +379,11 @@ int prt_hip_create(int device_index, prt_hip_ctx** out_ctx)
         prt_hip_destroy(ctx);
         return 5;
     }
+    ctx->d_counters = ctx->d_work + kWorkWords;
     ctx->d_stats = reinterpret_cast<unsigned long long*>(ctx->d_counters + 64);
     ctx->num_cus = prop.multiProcessorCount;
     ctx->device_name = prop.name[0] ? std::string(prop.name) : std::string("AMD ") + prop.gcnArchName;
-    if (hipMemsetAsync(ctx->d_counters, 0, 64 * sizeof(uint32_t), ctx->stream) != hipSuccess ||
+    if (hipMemsetAsync(ctx->d_work, 0, (kWorkWords + 64) * sizeof(uint32_t), ctx->stream) != hipSuccess ||
         hipStreamSynchronize(ctx->stream) != hipSuccess) {
         prt_hip_destroy(ctx);
         return 5;
@@ -402,7 +404,7 @@ int prt_hip_destroy(prt_hip_ctx* ctx)
     free_ptr(ctx->d_path_hits);
     void* ptrs[] = {ctx->d_spill,
                     ctx->d_accum, ctx->d_bgr8, ctx->d_rays[0], ctx->d_rays[1], ctx->d_hits,
-                    ctx->d_pix[0], ctx->d_pix[1], ctx->d_rng[0], ctx->d_rng[1], ctx->d_counters,
+                    ctx->d_pix[0], ctx->d_pix[1], ctx->d_rng[0], ctx->d_rng[1], ctx->d_work,
                     ctx->d_io_rays, ctx->d_io_hits, ctx->d_look, ctx->d_look_side, ctx->d_look_flags, ctx->d_build};
     for (void* p : ptrs) free_ptr(p);
     for (auto& level : ctx->d_look_q)
@@ -530,13 +532,13 @@ int prt_hip_intersect_closest_device_noalloc(prt_hip_ctx* ctx, const prt_ray* d_
     int grid = ctx->trace_grid;
     if ((size_t)grid > blocks_fit) grid = (int)blocks_fit;
     uint32_t* hdr = static_cast<uint32_t*>(ctx->d_scratch);
-    PRT_TRY(ctx, launch_zero_u32(hdr, 2, ctx->stream));  // a kernel, not a memset: safe under graph capture
+    PRT_TRY(ctx, launch_zero_u32(hdr, kWorkWords, ctx->stream));  // a kernel, not a memset: safe under graph capture
     TraceLaunch t{};
     t.rays = reinterpret_cast<const float4*>(d_rays);
     t.hits = reinterpret_cast<float4*>(d_hits);
     t.count_ptr = nullptr;
     t.count = (uint32_t)n;
-    t.fetch_ptr = hdr;
+    t.work = hdr;
     t.stats = nullptr;
     PRT_TRY(ctx, launch_trace_scratch(ctx, t, reinterpret_cast<uint2*>(static_cast<char*>(ctx->d_scratch) + kScratchHeader),
                                       need, hdr + 1, grid));
@@ -853,7 +855,7 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
         p.accum = ctx->d_accum;
         p.max_depth = last;
         p.albedo = albedo;
-        p.path_counter = ctx->d_counters + 16;
+        p.work = ctx->d_work;
         p.depth_rays = ctx->d_stats + 16;
         p.stats = ctx->d_stats;
         p.fast = fast;
@@ -872,8 +874,6 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
             p.q_cap = ctx->look_q_cap;
             p.look_gen = ctx->look_gen;
             p.look_flags = ctx->d_look_flags;
-            p.path_counter = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ctx->d_look) +
-                                                         offsetof(LookState, counter));
         }
         if (timing) PRT_TRY(ctx, hipEventRecord(ctx->kev[0], ctx->stream));
         PRT_TRY(ctx, launch_paths(ctx, p, renderer, counting));
@@ -892,7 +892,7 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
             t.hits = ctx->d_hits;
             t.count_ptr = ctx->d_counters + slot;
             t.count = 0;
-            t.fetch_ptr = ctx->d_counters + 16 + slot;
+            t.work = ctx->d_counters + 16 + slot;
             t.stats = counting ? ctx->d_stats : nullptr;
             const int ev = slot;  // timing events of depth k: set k mod 16, read every 16 depths
             if (timing) PRT_TRY(ctx, hipEventRecord(ctx->kev[4 * ev + 0], ctx->stream));
@@ -1039,7 +1039,7 @@ BatchLaunch batch_launch_args(prt_hip_ctx* ctx)
     bl.scenes = ctx->d_batch_scenes;
     bl.samples = ctx->d_batch_samples;
     bl.total_work = ctx->batch_total_work;
-    bl.work_counter = ctx->d_counters + 48;
+    bl.work = ctx->d_work;
     bl.stats = ctx->d_stats;
     return bl;
 }
@@ -1383,7 +1383,7 @@ PathLaunch frame_path_launch(prt_hip_ctx* ctx, int pass, int max_depth)
     p.accum = ctx->d_accum;
     p.max_depth = max_depth;
     p.albedo = 0.0f;
-    p.path_counter = ctx->d_counters + 16;
+    p.work = ctx->d_work;
     p.depth_rays = ctx->d_stats + 16;
     p.stats = ctx->d_stats;
     p.albedo_rgb = ctx->d_albedo;
@@ -1487,7 +1487,7 @@ int prt_hip_render_albedo_image(prt_hip_ctx* ctx, int pass0, int spp, int max_de
         PathLaunch p = frame_path_launch(ctx, pass0 + s0, max_depth);
         p.spp = n;
         p.rgb_planes = ctx->d_rgb_planes;
-        PRT_TRY(ctx, launch_zero_u32(ctx->d_counters + 16, 1, ctx->stream));
+        PRT_TRY(ctx, launch_zero_u32(ctx->d_work, kWorkWords, ctx->stream));
         PRT_TRY(ctx, launch_paths_rgb(ctx, p, (ctx->profiling & PRT_PROFILE_COUNTERS) != 0));
         PRT_TRY(ctx, launch_rgb_planes_add(ctx, ctx->d_rgb_planes, n));
     }

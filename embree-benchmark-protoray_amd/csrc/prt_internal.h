@@ -143,7 +143,7 @@ struct BatchLaunch {
     const SceneDevice* scenes;
     float* samples;              // path radiance per (job, sample, pixel)
     uint32_t total_work;
-    uint32_t* work_counter;      // zero before launch
+    uint32_t* work;              // work counters (kWorkWords), zero before launch
     unsigned long long* stats;   // [0..2] instrumented counters, [3] rays
 };
 
@@ -217,6 +217,8 @@ struct prt_hip_ctx {
     float4* d_hits = nullptr;                 // 1 float4 per hit
     int32_t* d_pix[2] = {nullptr, nullptr};
     uint32_t* d_rng[2] = {nullptr, nullptr};
+    // one allocation: work counters (kWorkWords), counters, statistics
+    uint32_t* d_work = nullptr;
     uint32_t* d_counters = nullptr;           // [0..15] queue sizes, [16..31] fetch, [32] error
     void* h_readback = nullptr;               // pinned host copy of d_counters + d_stats
     unsigned long long* d_stats = nullptr;    // instrumented counters
@@ -282,13 +284,17 @@ namespace prt {
 int build_bvh8(prt_hip_ctx* ctx, SceneBuffers& sb, prt_build_stats* stats);
 
 // trace.hip
+// Work counters of a persistent launch: 16 of them, a 128 B line each.
+constexpr uint32_t kWorkCountersLg = 4;
+constexpr uint32_t kWorkCounterStride = 32;
+constexpr int kWorkWords = (int)kWorkCounterStride << kWorkCountersLg;
 struct TraceLaunch {
     const float4* rays;
     float4* hits;               // closest-hit records
     float* any_t;               // any-hit query: distance of a blocking triangle, or -1
     const uint32_t* count_ptr;  // device count of rays (nullptr: use count)
     uint32_t count;
-    uint32_t* fetch_ptr;        // device fetch counter, zero before launch
+    uint32_t* work;             // work counters, zero before launch: kWorkWords, or one when count_ptr is set
     unsigned long long* stats;  // nullptr unless instrumented
     uint32_t* err;              // error flag (nullptr: the context's)
 };
@@ -311,7 +317,6 @@ constexpr int kCoopTail = 1, kCoopSpread = 2;
 // finished wait in a per-pixel side buffer, tagged with the call that adds
 // them to the accumulator.
 struct LookState {
-    uint32_t counter;       // work counter over this frame's space
     uint32_t spec_counter;  // work counter over the later frames' space
     uint32_t target;        // items of this frame's space (0: the frame is finished)
     uint32_t live;          // waves that hold, or can still take, paths of this frame
@@ -332,7 +337,7 @@ struct PathLaunch {
     float4* accum;
     int max_depth;
     float albedo;
-    uint32_t* path_counter;          // zero before launch
+    uint32_t* work;                  // work counters (kWorkWords), zero before launch
     unsigned long long* depth_rays;  // [16] rays traced per depth, zero before launch
     unsigned long long* stats;       // instrumented counters; [3] rays
     // per-triangle RGB albedo (RGB forward and adjoint modes), original triangle order

@@ -60,11 +60,19 @@ __global__ __launch_bounds__(kBlock) void k_raygen(Camera cam, int width, int he
     rng[gid] = s;
 }
 
-__global__ __launch_bounds__(kBlock) void k_frame_begin(uint32_t* counters, uint32_t n0,
-                                                        unsigned long long* stats)
+// Clears the counters and statistics of a frame, in one block.
+__device__ __forceinline__ void clear_counters(uint32_t* work, uint32_t* counters, uint32_t n0,
+                                               unsigned long long* stats)
 {
+    if (threadIdx.x < 1u << kWorkCountersLg) work[threadIdx.x * kWorkCounterStride] = 0u;
     if (threadIdx.x < 33) counters[threadIdx.x] = threadIdx.x == 0 ? n0 : 0u;
     if (threadIdx.x < 32) stats[threadIdx.x] = threadIdx.x == 9 ? ~0ull : 0ull;  // [9]: a minimum
+}
+
+__global__ __launch_bounds__(64) void k_frame_begin(uint32_t* work, uint32_t* counters, uint32_t n0,
+                                                    unsigned long long* stats)
+{
+    clear_counters(work, counters, n0, stats);
 }
 
 __device__ __forceinline__ void tri_vertices(const int32_t* idx, const float* pos, int prim, f3& p0,
@@ -99,15 +107,14 @@ __device__ __forceinline__ void accum_add(float4* accum, int pixel, float c, boo
 //    earlier calls finished (side slot tag % kLookLevels, tagged `tag`) to
 //    their pixels' accumulators; those pixels get no other sample in this
 //    call.
-__global__ __launch_bounds__(kBlock) void k_look_call_begin(uint32_t* counters, uint32_t n0,
+__global__ __launch_bounds__(kBlock) void k_look_call_begin(uint32_t* work, uint32_t* counters, uint32_t n0,
                                                             unsigned long long* stats, LookState* ls,
                                                             uint32_t entries, int valid, uint32_t q_cap,
                                                             uint32_t waves, const uint2* side, float4* accum, int n,
                                                             uint32_t tag)
 {
     if (blockIdx.x == 0) {
-        if (threadIdx.x < 33) counters[threadIdx.x] = threadIdx.x == 0 ? n0 : 0u;
-        if (threadIdx.x < 32) stats[threadIdx.x] = threadIdx.x == 9 ? ~0ull : 0ull;  // [9]: a minimum
+        clear_counters(work, counters, n0, stats);
         __syncthreads();
         if (threadIdx.x == 0) {
             LookState nx{};
@@ -300,12 +307,10 @@ __global__ void k_queue_recycle(uint32_t* counters, unsigned long long* stats, i
 }
 
 // ---- batched form
-__global__ __launch_bounds__(64) void k_batch_begin(uint32_t* counters, unsigned long long* stats)
+__global__ __launch_bounds__(64) void k_batch_begin(uint32_t* work, uint32_t* counters, unsigned long long* stats)
 {
-    if (threadIdx.x == 0) {
-        counters[32] = 0u;
-        counters[48] = 0u;
-    }
+    if (threadIdx.x < 1u << kWorkCountersLg) work[threadIdx.x * kWorkCounterStride] = 0u;
+    if (threadIdx.x == 0) counters[32] = 0u;
     if (threadIdx.x < 16) stats[threadIdx.x] = 0ull;
 }
 
@@ -369,7 +374,7 @@ hipError_t launch_raygen(prt_hip_ctx* ctx, int pass, float4* rays, int32_t* pix,
     const int tiles_x = (ctx->width + 7) / 8, tiles_y = (ctx->height + 7) / 8;
     const int tiles = tiles_x * tiles_y;
     const uint32_t entries = (uint32_t)tiles * 64u;
-    k_frame_begin<<<1, 64, 0, ctx->stream>>>(ctx->d_counters, entries, ctx->d_stats);
+    k_frame_begin<<<1, 64, 0, ctx->stream>>>(ctx->d_work, ctx->d_counters, entries, ctx->d_stats);
     const float inv_w = 1.0f / (float)ctx->width, inv_h = 1.0f / (float)ctx->height;
     k_raygen<<<(tiles * 64 + kBlock - 1) / kBlock, kBlock, 0, ctx->stream>>>(
         to_camera(ctx->cam), ctx->width, ctx->height, tiles_x, tiles, pass, inv_w, inv_h, rays, pix, rng);
@@ -378,7 +383,7 @@ hipError_t launch_raygen(prt_hip_ctx* ctx, int pass, float4* rays, int32_t* pix,
 
 hipError_t launch_frame_begin(prt_hip_ctx* ctx, uint32_t entries)
 {
-    k_frame_begin<<<1, 64, 0, ctx->stream>>>(ctx->d_counters, entries, ctx->d_stats);
+    k_frame_begin<<<1, 64, 0, ctx->stream>>>(ctx->d_work, ctx->d_counters, entries, ctx->d_stats);
     return hipGetLastError();
 }
 
@@ -387,7 +392,7 @@ hipError_t launch_look_call_begin(prt_hip_ctx* ctx, bool valid, uint32_t entries
     const int n = ctx->width * ctx->height;
     const int grid = valid ? (n + kBlock - 1) / kBlock : 1;
     k_look_call_begin<<<grid, kBlock, 0, ctx->stream>>>(
-        ctx->d_counters, entries, ctx->d_stats, ctx->d_look, entries, valid ? 1 : 0, ctx->look_q_cap,
+        ctx->d_work, ctx->d_counters, entries, ctx->d_stats, ctx->d_look, entries, valid ? 1 : 0, ctx->look_q_cap,
         (uint32_t)diffuse_grid(ctx, entries) * (uint32_t)(kTraceBlock / 64), ctx->d_look_side, ctx->d_accum, n,
         ctx->look_gen);
     return hipGetLastError();
@@ -433,7 +438,7 @@ hipError_t launch_accum_mean_rgb(prt_hip_ctx* ctx, float* image)
 
 hipError_t launch_batch_begin(prt_hip_ctx* ctx)
 {
-    k_batch_begin<<<1, 64, 0, ctx->stream>>>(ctx->d_counters, ctx->d_stats);
+    k_batch_begin<<<1, 64, 0, ctx->stream>>>(ctx->d_work, ctx->d_counters, ctx->d_stats);
     return hipGetLastError();
 }
 
