@@ -1429,36 +1429,48 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     }
 }
 
-// Persistent workgroups of a launch over `items` rays or paths.  Each wave pays
-// for the drain of its own last items (about 50 steps at a few active lanes),
-// so a launch that has few items per lane gains more from fewer waves than it
-// loses in latency hiding.  Measured per frame or launch with 1 / 2 / 3 / 4
-// workgroups per CU (256 CUs of 256 lanes each), ms:
-//   diffuse   24 k paths 0.248 0.246 0.263 0.283; 140 k 0.618 0.631 0.606 0.623;
-//             262 k 0.457 0.320 0.337 0.377; 518 k 0.806 0.717 0.769 0.810;
-//             0.92 M 1.392 0.979 0.995 1.120; 1.05 M 1.476 0.919 0.792 0.768;
-//             2.07 M 2.260 1.389 1.182 1.167
-//   closest   50 k rays 0.132 0.141 0.153 0.164; 100 k 0.177 0.154 0.167 0.176;
-//             200 k 0.285 0.204 0.185 0.205; 300 k 0.389 0.261 0.232 0.224;
-//             600 k 0.676 0.412 0.344 0.333: no bounces, so the drain is short
-//   any hit   200 k 0.184 0.145 0.143 0.158; 1 M 0.622 0.412 0.405 0.409
-//   diffuse2  290 k 0.690 0.770 0.846 0.796; 1.35 M 1.585 1.124 1.115 1.224:
-//             two rays a hit make its drain twice as long, so it counts half
-//   primary   262 k 0.088 0.093 0.106 0.118; 8.3 M 1.737 1.729 1.743 1.766:
-//             coherent rays fill the issue slots with 2
+// Persistent workgroups of a launch over `items` rays or paths.  Each wave of a
+// path launch pays for the drain of its own last paths (about 50 steps at a few
+// active lanes), so one that has few items per lane gains more from fewer waves
+// than it loses in latency hiding.  Rays drain fast, and up to a run for every
+// wave they need no counter, so their launches take all waves, except where a
+// few runs would be left over for a second round.  Measured per frame or launch
+// with 1 / 2 / 3 / 4 workgroups per CU (256 CUs of 256 lanes each), ms, on the
+// spheres and on a mixed scene of 400 k triangles:
+//   closest    70 k 0.153 0.128 0.128 0.127, 0.244 0.241 0.243 0.242;
+//             260 k 0.335 0.224 0.203 0.167, 0.427 0.314 0.291 0.279;
+//             300 k 0.376 0.240 0.214 0.217, 0.498 0.343 0.301 0.321;
+//             2 M   2.045 1.144 0.874 0.774, 2.183 1.277 1.022 0.911
+//   any hit   260 k 0.241 0.171 0.159 0.124, 0.260 0.207 0.199 0.192;
+//             280 k 0.261 0.182 0.168 0.186, 0.268 0.200 0.194 0.212;
+//             2 M   1.456 0.827 0.659 0.586, 1.250 0.755 0.621 0.569
+//   primary   144 k 0.129 0.134 0.125 0.126, 0.179 0.186 0.177 0.177;
+//             262 k 0.182 0.166 0.167 0.138, 0.252 0.205 0.193 0.177;
+//             2 M   0.502 0.374 0.341 0.330, 0.738 0.503 0.457 0.433
+//   diffuse   495 k 0.992 0.707 0.710 0.767, 1.415 0.984 0.998 1.098;
+//             640 k 1.214 0.799 0.728 0.780, 1.739 1.194 1.055 1.130;
+//             0.97 M 1.724 1.092 0.919 0.900, 2.452 1.571 1.389 1.298
+//   diffuse2  495 k 1.673 1.150 1.177 1.296, 2.222 1.515 1.581 1.789;
+//             640 k 2.048 1.343 1.227 1.305, 2.761 1.855 1.656 1.798;
+//             1.05 M 3.068 1.907 1.601 1.545, 4.160 2.655 2.310 2.160
+// With the lookahead the drain is filled with later frames' work:
+//   diffuse   262 k 0.620 0.413 0.435 0.447, 0.820 0.611 0.620 0.639;
+//             495 k 0.972 0.638 0.487 0.513, 1.394 0.839 0.742 0.755;
+//             810 k 1.456 0.906 0.747 0.630, 2.075 1.306 1.047 0.924
 // On scenes whose nodes and triangles outgrow the memory-side cache (256 MiB)
 // diffuse launches run at most one below the occupancy limit: their paths take
 // long, so does the drain; the albedo and query launches are faster with all.
-int grid_for(const prt_hip_ctx* ctx, int mode, uint64_t items)
+int grid_for(const prt_hip_ctx* ctx, int mode, uint64_t items, bool look = false)
 {
-    if (mode == kModeDiffuse2) items /= 2;
-    const bool query = mode == kModeTrace || mode == kModeOccluded;
-    const uint64_t upto1 = query ? 64u << 10 : 128u << 10;
-    const uint64_t upto2 = query ? 160u << 10 : 640u << 10;
-    const uint64_t upto3 = query ? 256u << 10 : 1000u << 10;
-    int per_cu = items <= upto1 ? 1 : (items <= upto2 ? 2 : (items <= upto3 ? 3 : 4));
-    if (mode == kModePrimary) per_cu = std::min(per_cu, 2);
-    if (mode == kModeOccluded) per_cu = std::min(per_cu, 3);
+    int per_cu;
+    if (mode == kModeTrace || mode == kModeOccluded || mode == kModePrimary)
+        per_cu = items > 256u << 10 && items <= 400u << 10 ? 3 : 4;
+    else if (items <= 128u << 10)
+        per_cu = 1;
+    else if (items <= (look ? 384u : 576u) << 10)
+        per_cu = 2;
+    else
+        per_cu = items <= (look ? 640u : 928u) << 10 ? 3 : 4;
     int limit = ctx->trace_per_cu;
     if (mode == kModeDiffuse && limit > 1) {
         const SceneBuffers& s = ctx->scene;
@@ -1614,7 +1626,7 @@ int ensure_trace_resources(prt_hip_ctx* ctx)
     return 0;
 }
 
-int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries) { return grid_for(ctx, kModeDiffuse, entries); }
+int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries) { return grid_for(ctx, kModeDiffuse, entries, true); }
 
 // Frames that gain more from groups than from the lookahead: us per frame of
 // 13-frame chains, in groups / lookahead: 3072 path slots 161 / 191, 32256 211 /
