@@ -405,10 +405,8 @@ int prt_hip_destroy(prt_hip_ctx* ctx)
     void* ptrs[] = {ctx->d_spill,
                     ctx->d_accum, ctx->d_bgr8, ctx->d_rays[0], ctx->d_rays[1], ctx->d_hits,
                     ctx->d_pix[0], ctx->d_pix[1], ctx->d_rng[0], ctx->d_rng[1], ctx->d_work,
-                    ctx->d_io_rays, ctx->d_io_hits, ctx->d_look, ctx->d_look_side, ctx->d_look_flags, ctx->d_build};
+                    ctx->d_io_rays, ctx->d_io_hits, ctx->d_look, ctx->d_look_side, ctx->d_build};
     for (void* p : ptrs) free_ptr(p);
-    for (auto& level : ctx->d_look_q)
-        for (uint4* q : level) free_ptr(q);
     for (hipEvent_t e : ctx->kev)
         if (e) (void)hipEventDestroy(e);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
@@ -724,20 +722,16 @@ int prt_hip_set_lookahead(prt_hip_ctx* ctx, int enable)
 
 namespace {
 
-// Buffers of the frame lookahead: the state, kLookLevels side entries per
-// pixel and, per level, two queues (read by this call, written for the next)
-// of one path per lane.
-int ensure_look_resources(prt_hip_ctx* ctx)
+// Buffers of the frame lookahead: kLookLevels side entries per pixel and, in
+// one allocation, the state, the stop flags and, per level, two queues (read by
+// this call, written for the next) of one path per lane of the launch, item
+// uint4 each.
+int ensure_look_resources(prt_hip_ctx* ctx, uint32_t entries, int item)
 {
     const int64_t pixels = (int64_t)ctx->width * ctx->height;
     const int64_t side_len = pixels * kLookLevels;
-    const uint32_t cap = (uint32_t)ctx->trace_grid * (uint32_t)kTraceBlock;
+    const uint32_t lanes = (uint32_t)diffuse_grid(ctx, entries) * (uint32_t)kTraceBlock;
     bool fresh = false;
-    if (!ctx->d_look) {
-        PRT_TRY(ctx, hipMalloc(&ctx->d_look, sizeof(LookState)));
-        PRT_TRY(ctx, hipMemsetAsync(ctx->d_look, 0, sizeof(LookState), ctx->stream));
-        fresh = true;
-    }
     if (side_len != ctx->look_side_len) {
         free_ptr(ctx->d_look_side);
         ctx->d_look_side = nullptr;
@@ -747,32 +741,51 @@ int ensure_look_resources(prt_hip_ctx* ctx)
         ctx->look_side_len = side_len;
         fresh = true;
     }
-    if (cap > ctx->look_q_cap) {
+    const uint64_t words = (uint64_t)lanes * (uint64_t)item;
+    if (words > ctx->look_q_words) {
+        free_ptr(ctx->d_look);
+        ctx->d_look = nullptr;
+        ctx->look_q_words = 0;
+        constexpr size_t kStateBytes = (sizeof(LookState) + 255) & ~(size_t)255;
+        const size_t flag_bytes = sizeof(uint32_t) * kLookFlagStride * (size_t)ctx->trace_grid;
+        const size_t q_bytes = sizeof(uint4) * (size_t)words;
+        PRT_TRY(ctx, hipMalloc(&ctx->d_look, kStateBytes + flag_bytes + 2 * kLookLevels * q_bytes));
+        PRT_TRY(ctx, hipMemsetAsync(ctx->d_look, 0, kStateBytes + flag_bytes, ctx->stream));
+        char* at = reinterpret_cast<char*>(ctx->d_look) + kStateBytes;
+        ctx->d_look_flags = reinterpret_cast<uint32_t*>(at);
+        at += flag_bytes;
         for (auto& level : ctx->d_look_q)
             for (uint4*& q : level) {
-                free_ptr(q);
-                q = nullptr;
+                q = reinterpret_cast<uint4*>(at);
+                at += q_bytes;
             }
-        free_ptr(ctx->d_look_flags);
-        ctx->d_look_flags = nullptr;
-        ctx->look_q_cap = 0;
-        for (auto& level : ctx->d_look_q)
-            for (uint4*& q : level) PRT_TRY(ctx, hipMalloc(&q, 3 * sizeof(uint4) * (size_t)cap));
-        const size_t flag_bytes = sizeof(uint32_t) * kLookFlagStride * (size_t)ctx->trace_grid;
-        PRT_TRY(ctx, hipMalloc(&ctx->d_look_flags, flag_bytes));
-        PRT_TRY(ctx, hipMemsetAsync(ctx->d_look_flags, 0, flag_bytes, ctx->stream));
-        ctx->look_q_cap = cap;
+        ctx->look_q_words = words;
         fresh = true;
     }
+    ctx->look_q_cap = (uint32_t)(ctx->look_q_words / (uint64_t)item);
     if (fresh) ctx->look_prev_spec = false;  // nothing the previous call left is kept
     return 0;
+}
+
+// The first frame of a chain, from 0, that runs the lookahead.  That frame pays
+// for the work that it starts: a chain that ends with it is slower for it, one
+// that goes on is faster from the second frame after it.  ms per frame of
+// chains of 2, 4 and 13 frames without / with the lookahead from frame 1 on
+// (1280x720, spheres, depth 6): diffuse 0.722 / 0.984, 0.722 / 0.736, 0.731 /
+// 0.561; diffuse2 1.188 / 1.581, 1.202 / 1.077, 1.203 / 0.792.  The first frame
+// of diffuse2 costs more, half a frame above 640 k path slots, so there it waits
+// until that is small against the frames before.
+int look_from(int renderer, uint32_t entries)
+{
+    if (renderer != PRT_RENDERER_DIFFUSE2) return 1;
+    return entries > 640u << 10 ? 7 : 2;
 }
 
 // The previous call's lookahead work belongs to this call: the same inputs and
 // the next pass.
 bool look_follows(const prt_hip_ctx::LookKey& prev, const prt_hip_ctx::LookKey& cur)
 {
-    return prev.scene_gen == cur.scene_gen && std::memcmp(&prev.cam, &cur.cam, sizeof(prt_camera)) == 0 &&
+    return prev.renderer == cur.renderer && prev.scene_gen == cur.scene_gen && std::memcmp(&prev.cam, &cur.cam, sizeof(prt_camera)) == 0 &&
            prev.width == cur.width && prev.height == cur.height && prev.max_depth == cur.max_depth &&
            prev.grid == cur.grid && prev.albedo_bits == cur.albedo_bits && prev.pass + 1 == cur.pass;
 }
@@ -816,15 +829,15 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
     const int tiles_x = (ctx->width + 7) / 8;
     const uint32_t entries = (uint32_t)frame_entries(ctx);
 
-    // Lookahead: only in a call that continues the previous call's inputs
-    // (the next pass, same scene, camera, size, depth and albedo), so a
+    // Lookahead: only in a call that continues a chain of calls with the same
+    // inputs (the next pass, same scene, camera, size, depth and albedo), so a
     // camera that moves every frame renders each frame exactly as without
     // it; the work is kept only if that previous call ran the lookahead too.
-    const bool look_on = fused && renderer == PRT_RENDERER_DIFFUSE && !fast && !counting && ctx->lookahead != 0 &&
-                         lookahead_pays(ctx, entries) &&
+    const bool look_on = fused && renderer != PRT_RENDERER_PRIMARY && !fast && !counting && ctx->lookahead != 0 &&
                          ctx->pass < INT32_MAX - kLookLevels;  // the passes started ahead must not overflow
     prt_hip_ctx::LookKey key{};
     if (look_on) {
+        key.renderer = renderer;
         key.scene_gen = ctx->scene_gen;
         key.cam = ctx->cam;
         key.width = ctx->width;
@@ -834,9 +847,10 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
         key.grid = diffuse_grid(ctx, entries);
         std::memcpy(&key.albedo_bits, &albedo, sizeof(float));
     }
-    const bool look_run = look_on && ctx->look_prev_on && look_follows(ctx->look_prev, key);
+    const int chain = look_on && ctx->look_prev_on && look_follows(ctx->look_prev, key) ? ctx->look_chain + 1 : 0;
+    const bool look_run = look_on && chain >= look_from(renderer, entries);
     ctx->look_prev_on = false;  // set again once this call has succeeded
-    if (look_run && ensure_look_resources(ctx)) return 1;
+    if (look_run && ensure_look_resources(ctx, entries, look_item(renderer))) return 1;
     const bool look_valid = look_run && ctx->look_prev_spec;
 
     PRT_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
@@ -941,6 +955,7 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
     if (look_on) {
         ctx->look_prev = key;
         ctx->look_prev_on = true;
+        ctx->look_chain = chain;
         ctx->look_prev_spec = look_run;
     }
     ctx->pass += 1;

@@ -162,7 +162,14 @@ struct BatchTuning {
 };
 
 struct LookState;
-constexpr int kLookLevels = 2;  // frames past its own that a diffuse call may start
+// Frames past its own that a diffuse or diffuse2 call may start.  1 / 2 / 3 / 4,
+// Mrays/s of diffuse chains: spheres 1920x1080 3798 3819 3772 3745, city 2418
+// 2714 2808 2823, 400 k mixed triangles 1280x720 1682 1860 2007 2014, height
+// field 512x512 2697 2912 2856 2838; ms per diffuse2 frame of 290 k paths 0.58
+// 0.49 0.45 0.45.
+constexpr int kLookLevels = 3;
+// uint4 of a suspended path
+constexpr int look_item(int renderer) { return renderer == PRT_RENDERER_DIFFUSE2 ? 5 : 3; }
 
 }  // namespace prt
 
@@ -253,16 +260,18 @@ struct prt_hip_ctx {
     uint2* d_look_side = nullptr;       // kLookLevels slots of one entry per pixel
     int64_t look_side_len = 0;
     uint4* d_look_q[prt::kLookLevels][2] = {};  // per level, read by this call / written for the next
-    uint32_t look_q_cap = 0;
+    uint64_t look_q_words = 0;          // uint4 per queue
+    uint32_t look_q_cap = 0;            // paths per queue in the current call
     uint32_t* d_look_flags = nullptr;   // one stop flag per block of the launch
     uint32_t look_gen = 0;
     struct LookKey {
         uint64_t scene_gen;
         prt_camera cam;
-        int width, height, max_depth, pass, grid;
+        int renderer, width, height, max_depth, pass, grid;
         uint32_t albedo_bits;
     } look_prev{};
-    bool look_prev_on = false;    // look_prev holds the inputs of the last successful diffuse call
+    bool look_prev_on = false;    // look_prev holds the inputs of the last successful diffuse or diffuse2 call
+    int look_chain = 0;           // ... which was this frame of a chain of calls that continue each other
     bool look_prev_spec = false;  // ... and that call ran the lookahead (its state is meaningful)
 
     // device address of the library's fixed scratch array on this context's
@@ -302,7 +311,7 @@ struct TraceLaunch {
 // a small launch spread over the waves that way from its start
 constexpr int kCoopTail = 1, kCoopSpread = 2;
 // Fused path launch (one frame, one sample per pixel)
-// Frame lookahead of the fused diffuse renderer: device state that one render
+// Frame lookahead of the fused diffuse and diffuse2 renderers: device state that one render
 // call hands to the next.  A call renders frame p; a path of frame p + l is
 // "at level l".  Work items, in the order they are handed out:
 //  - this frame's space: the items of frame p that earlier calls did not
@@ -360,10 +369,10 @@ struct PathLaunch {
     bool fast;
     // cooperative tracing (kCoopTail, kCoopSpread or 0); set by the launch
     int coop;
-    // diffuse frames: frame lookahead (nullptr: off)
+    // diffuse and diffuse2 frames: frame lookahead (nullptr: off)
     LookState* look;
     uint2* side;          // kLookLevels slots of W*H: (sample bits, tag of the call that adds it)
-    const uint4* q_in[kLookLevels];   // suspended paths of frame p + l, 3 uint4 each
+    const uint4* q_in[kLookLevels];   // suspended paths of frame p + l, 3 uint4 each (diffuse2: 5)
     uint4* q_out[kLookLevels];        // suspended paths of frame p + l + 1 (the next call's level l)
     uint32_t q_cap;       // capacity of each queue in paths (>= lanes of the launch)
     uint32_t look_gen;    // this call's tag
@@ -376,8 +385,6 @@ int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries);
 // a query of `rays` rays is spread over the waves from its start, without the
 // work counter
 bool query_spreads(const prt_hip_ctx* ctx, int64_t rays);
-// frames of so many path slots are faster with the lookahead
-bool lookahead_pays(const prt_hip_ctx* ctx, uint32_t entries);
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented);
 // closest-hit launch over at most max_grid persistent workgroups whose stack
 // spill (stack_entries per lane) and error flag the caller provides

@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     uint2* const g_spill = spill + ((size_t)blockIdx.x * kBlock + (tid & ~7)) * (size_t)stack_entries;
     auto group_slot = [&](int q) -> int { return ((q >> 3) & (kStack - 1)) * kBlock + (tid & ~7) + (q & 7); };
 
-    // Frame lookahead (kModeDiffuse, LookState); a path of frame pass + l is
+    // Frame lookahead (diffuse and diffuse2, LookState); a path of frame pass + l is
     // at level l.  This frame's space, from LookState::counter: [0, F) are
     // its items S_0..entries-1 (F = entries - S_0), then the paths the
     // previous call suspended, level by level: queue l holds lk_res[l + 1] -
@@ -214,7 +214,8 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     //  - After the stop no more items are taken, and paths of later frames
     //    leave for the queue of their level: at a bounce, or in the middle
     //    of a ray, which the next call then traces again from its origin.
-    constexpr bool kLookMode = kMode == kModeDiffuse && kLook;
+    constexpr bool kLookMode = (kMode == kModeDiffuse || kMode == kModeDiffuse2) && kLook;
+    constexpr int kLookItem = look_item(kMode == kModeDiffuse2 ? PRT_RENDERER_DIFFUSE2 : PRT_RENDERER_DIFFUSE);
     LookState* const look = kLookMode ? pl.look : nullptr;
     uint32_t lk_F = 0, lk_fresh_end = 0, lk_target = 0;
     uint32_t lk_S[kLookLevels + 1] = {};         // S_l
@@ -357,19 +358,26 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         } else if (kLookMode && look && !spec_claim && my >= lk_F) {
             // a path that the previous call stopped at a bounce
             // (or in the middle of a ray): its next ray
-            const uint4* q = pl.q_in[0] + 3 * (size_t)(my - lk_res[0]);
+            const uint4* q = pl.q_in[0] + kLookItem * (size_t)(my - lk_res[0]);
             level = 0;
 #pragma unroll
             for (int l = 1; l < kLookLevels; ++l)
                 if (my >= lk_res[l]) {
-                    q = pl.q_in[l] + 3 * (size_t)(my - lk_res[l]);
+                    q = pl.q_in[l] + kLookItem * (size_t)(my - lk_res[l]);
                     level = l;
                 }
             const uint4 e0 = q[0], e1 = q[1], e2 = q[2];
             pixel = (int32_t)e0.w;
             rng = e1.w;
             depth = (int)e2.x;
-            lw = __uint_as_float(e2.y);
+            lw = as_f(e2.y);
+            if (kMode == kModeDiffuse2) {
+                const uint4 e3 = q[3], e4 = q[4];
+                lsum = as_f(e2.z);
+                shadow = e2.w != 0;
+                eo = mk3(as_f(e3.x), as_f(e3.y), as_f(e3.z));
+                ed = mk3(as_f(e3.w), as_f(e4.x), as_f(e4.y));
+            }
             start_ray(mk3(as_f(e0.x), as_f(e0.y), as_f(e0.z)), mk3(as_f(e1.x), as_f(e1.y), as_f(e1.z)),
                       0.0f, 3.402823466e38f);
             active = true;
@@ -446,6 +454,25 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         if (add && gw_b * db != 0.0f) atomicAdd(g + 2, gw_b * db);
     };
 
+    // Counts a ray for the frame that its path belongs to.
+    auto count_ray = [&](bool lead) __attribute__((always_inline)) {
+        if (kLookMode && level > 0) {
+#pragma unroll
+            for (int l = 1; l <= kLookLevels; ++l)
+                if (level == l && lead) ++n_ahead[l - 1];
+        } else {
+            n_rays += lead ? 1u : 0u;
+        }
+    };
+
+    // A later frame's sample, for the call whose tag it carries.
+    auto side_sample = [&](float c, bool lead) __attribute__((always_inline)) {
+        const uint32_t tag = pl.look_gen + (uint32_t)level;
+        if (lead)
+            pl.side[(size_t)(tag % (uint32_t)kLookLevels) * (size_t)(pl.width * pl.height) + pixel] =
+                make_uint2(__float_as_uint(c), tag);
+    };
+
     // Shades the lanes whose ray has finished (active, not tracing).  lead: the
     // lane counts and writes for its path; grouped: its path is held by a group
     // of 8 lanes.
@@ -460,7 +487,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
             if (kMode == kModeDiffuse2 && shadow) {
                 // shadow ray done: light from the sky unless blocked (MIS weight 1/2)
                 if constexpr (kCount) { if (lead) atomicAdd(&depth_hist[min(depth, kMaxQueueDepth - 1)], 1u); }
-                n_rays += lead ? 1u : 0u;
+                count_ray(lead);
                 if (best_prim < 0) lsum += lw * 0.5f;
                 shadow = false;
                 start_ray(eo, ed, 0.0f, 3.402823466e38f);
@@ -486,13 +513,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
                 break;
             }
             if constexpr (kCount && kMode != kModeBatch) { if (lead) atomicAdd(&depth_hist[min(depth, kMaxQueueDepth - 1)], 1u); }
-            if (kLookMode && level > 0) {
-#pragma unroll
-                for (int l = 1; l <= kLookLevels; ++l)
-                    if (level == l && lead) ++n_ahead[l - 1];
-            } else {
-                n_rays += lead ? 1u : 0u;
-            }
+            count_ray(lead);
             float4* acc = kMode == kModeBatch ? nullptr : pl.accum + pixel;
             if (kMode == kModeDiffuse2) {
                 // extension ray done (render/diffuse2_integrator_single.h:52-85)
@@ -504,9 +525,13 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
                     done = true;
                 }
                 if (done) {
+                    active = false;
+                    if (kLookMode && level > 0) {
+                        side_sample(lsum, lead);
+                        break;
+                    }
                     const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
                     if (lead) *acc = make_float4(a.x + lsum, a.y + lsum, a.z + lsum, a.w + 1.0f);
-                    active = false;
                     break;
                 }
                 lw *= albedo;
@@ -582,11 +607,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
                         if (lead) *acc = make_float4(a.x + c, a.y + cg, a.z + cb, a.w + 1.0f);
                     }
                 } else if (kLookMode && level > 0) {
-                    // a later frame's sample, for the call whose tag it carries
-                    const uint32_t tag = pl.look_gen + (uint32_t)level;
-                    if (lead)
-                        pl.side[(size_t)(tag % (uint32_t)kLookLevels) * (size_t)(pl.width * pl.height) + pixel] =
-                            make_uint2(__float_as_uint(c), tag);
+                    side_sample(c, lead);
                 } else {
                     const float4 a = pl.fast ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
                     if (lead) *acc = make_float4(a.x + c, a.y + c, a.z + c, a.w + 1.0f);
@@ -1000,6 +1021,11 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         // them over in groups, so this code runs for many lanes at once
         // instead of stalling every traversal step of the wave for one lane
         shade(true, false);
+        if (kMode == kModeDiffuse2 && kLookMode && stop && tracing) {
+            suspend = true;  // at a bounce, or between its shadow ray and its next
+            tracing = false;
+            active = false;
+        }
 
         // ---- refill idle lanes (wave-uniform branch)
         const uint64_t idle = __ballot(!active);
@@ -1410,11 +1436,16 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
                         if (level == l + 1) sm = left[l];
                     slot += (uint32_t)__popcll(sm & lane_lt);
                     if (slot < pl.q_cap) {
-                        uint4* q = pl.q_out[level - 1] + 3 * (size_t)slot;
+                        uint4* q = pl.q_out[level - 1] + kLookItem * (size_t)slot;
                         q[0] = make_uint4(__float_as_uint(o.x), __float_as_uint(o.y), __float_as_uint(o.z),
                                           (uint32_t)pixel);
                         q[1] = make_uint4(__float_as_uint(d.x), __float_as_uint(d.y), __float_as_uint(d.z), rng);
-                        q[2] = make_uint4((uint32_t)depth, __float_as_uint(lw), 0u, 0u);
+                        q[2] = make_uint4((uint32_t)depth, __float_as_uint(lw), __float_as_uint(lsum), shadow ? 1u : 0u);
+                        if (kMode == kModeDiffuse2) {
+                            q[3] = make_uint4(__float_as_uint(eo.x), __float_as_uint(eo.y), __float_as_uint(eo.z),
+                                              __float_as_uint(ed.x));
+                            q[4] = make_uint4(__float_as_uint(ed.y), __float_as_uint(ed.z), 0u, 0u);
+                        }
                     } else {
                         atomicOr(err, 2u);
                     }
@@ -1542,7 +1573,7 @@ hipError_t launch_mode(prt_hip_ctx* ctx, const TraceLaunch& t, const PathLaunch&
             sc, t, p, bl, ctx->d_spill, ctx->stack_entries, kRefill, err);
         return hipGetLastError();
     }
-    if constexpr (kMode == kModeDiffuse) {
+    if constexpr (kMode == kModeDiffuse || kMode == kModeDiffuse2) {
         if (p.look != nullptr) {
             k_trace<false, kMode, kTraceBlock, kStackLds, true><<<grid, kTraceBlock, 0, ctx->stream>>>(
                 sc, t, p, bl, ctx->d_spill, ctx->stack_entries, kRefill, err);
@@ -1586,15 +1617,17 @@ hipError_t launch_batch_variant(prt_hip_ctx* ctx, const BatchLaunch& bl, int blo
 int ensure_trace_resources(prt_hip_ctx* ctx)
 {
     if (ctx->trace_per_cu == 0) {
-        // the lookahead variant's workgroups must all be resident at once: a
+        // the lookahead variants' workgroups must all be resident at once: a
         // workgroup that starts only when another ends would hold the frame's
         // stop (every wave leaves the live count) until then
-        int per_cu = 0, per_cu_look = 0;
+        int per_cu = 0, per_cu_look = 0, per_cu_look2 = 0;
         PRT_TRY(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<false, kModeDiffuse>,
                                                                   kTraceBlock, 0));
         PRT_TRY(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(
                          &per_cu_look, k_trace<false, kModeDiffuse, kTraceBlock, kStackLds, true>, kTraceBlock, 0));
-        if (per_cu_look < per_cu) per_cu = per_cu_look;
+        PRT_TRY(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                         &per_cu_look2, k_trace<false, kModeDiffuse2, kTraceBlock, kStackLds, true>, kTraceBlock, 0));
+        per_cu = std::min(per_cu, std::min(per_cu_look, per_cu_look2));
         if (per_cu * kTraceBlock > 2048) per_cu = 2048 / kTraceBlock;
         if (per_cu < 1) per_cu = 1;
         ctx->trace_per_cu = per_cu;
@@ -1627,11 +1660,6 @@ int ensure_trace_resources(prt_hip_ctx* ctx)
 }
 
 int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries) { return grid_for(ctx, kModeDiffuse, entries, true); }
-
-// Frames that gain more from groups than from the lookahead: us per frame of
-// 13-frame chains, in groups / lookahead: 3072 path slots 161 / 191, 32256 211 /
-// 220, 282 / 311, 227 / 235 (three scenes), 64000 266 / 240, 348 / 328, 298 / 243.
-bool lookahead_pays(const prt_hip_ctx* ctx, uint32_t entries) { return !ctx->tail_coop || entries > 32768; }
 
 bool query_spreads(const prt_hip_ctx* ctx, int64_t rays)
 {

@@ -264,18 +264,17 @@ int prt_hip_set_pipeline(prt_hip_ctx* ctx, int pipeline);
 #define PRT_TAIL_LANES       0
 #define PRT_TAIL_COOPERATIVE 1
 int prt_hip_set_tail(prt_hip_ctx* ctx, int mode);
-/* Frame lookahead of the fused diffuse renderer (no counterpart in the
- * reference; default on).  In a call that continues the previous call (pass
- * p + 1 after pass p, with the same scene, camera, frame size, max depth and
- * albedo), idle lanes start paths of the next two passes while the last
- * paths of this one run; the call returns when its own frame is complete, and the
- * next call keeps that work if it continues this one (else drops it).  The
- * first call after any change renders as without the lookahead.  The
- * accumulator after each call and its ray count are those of rendering the
- * frames one by one.  Off for the primary, diffuse2 and Fast renderers, the
- * wavefront pipeline, under PRT_PROFILE_COUNTERS, and for frames of at most
- * 32768 path slots with the cooperative tail, which trace each path on 8 lanes
- * from the start. */
+/* Frame lookahead of the fused diffuse and diffuse2 renderers (no counterpart
+ * in the reference; default on).  In a call that continues a chain of calls
+ * (pass p + 1 after pass p, with the same renderer, scene, camera, frame size,
+ * max depth and albedo), idle lanes start paths of the next three passes while
+ * the last paths of this one run; the call returns when its own frame is
+ * complete, and the next call keeps that work if it continues this one (else
+ * drops it).  The first call after any change (diffuse2: the first two; frames
+ * of more than 640 k path slots: the first seven) renders as without the
+ * lookahead.  The accumulator after each call and its ray count are those of rendering the
+ * frames one by one.  Off for the primary and Fast renderers, the wavefront
+ * pipeline and under PRT_PROFILE_COUNTERS. */
 int prt_hip_set_lookahead(prt_hip_ctx* ctx, int enable);
 
 /* --- frame buffer read-back -------------------------------------------- */
