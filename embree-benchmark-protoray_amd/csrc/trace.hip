@@ -115,6 +115,11 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         depth_hist = hist;
     }
     uint32_t n_rays = 0;
+    uint4* grad_sums = nullptr;  // add_gradient
+    if constexpr (kMode == kModeAdjoint) {
+        __shared__ uint4 sums[kBlock];
+        grad_sums = sums;
+    }
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -442,16 +447,33 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     };
 
     // Adjoint: adds a hit's gradient, dL_c/da_c(t) = product of the path's other
-    // albedos.
+    // albedos.  The lanes here hand their triangles and three sums to each other
+    // through LDS, so that three lanes next to each other add the channels of
+    // one triangle: one request of 12 bytes to the memory instead of three.
+    // Requests bound these adds.  Adjoint of 512x512 x 8 spp, depth 6, ms with
+    // every lane adding its own three / this / no adds at all: 33.5 k triangles
+    // 2.46 / 2.15 / 2.06, 2.4 k triangles 1.98 / 1.43 / 1.20.
     auto add_gradient = [&](uint32_t tri, float ar, float ag, float ab, bool add) __attribute__((always_inline)) {
-        float* g = pl.grad + 3 * (size_t)tri;
         const uint32_t zr = zeros & 0xffu, zg = (zeros >> 8) & 0xffu, zb = zeros >> 16;
         const float dr = zr == 0 ? pr / ar : (zr == 1 && ar == 0.0f ? pr : 0.0f);
         const float dg = zg == 0 ? pg / ag : (zg == 1 && ag == 0.0f ? pg : 0.0f);
         const float db = zb == 0 ? pb / ab : (zb == 1 && ab == 0.0f ? pb : 0.0f);
-        if (add && gw_r * dr != 0.0f) atomicAdd(g + 0, gw_r * dr);
-        if (add && gw_g * dg != 0.0f) atomicAdd(g + 1, gw_g * dg);
-        if (add && gw_b * db != 0.0f) atomicAdd(g + 2, gw_b * db);
+        if (!add) return;
+        uint4* const sums = grad_sums + (tid & ~63);
+        const uint64_t here = __ballot(1);
+        const uint32_t n = (uint32_t)__popcll(here), rank = (uint32_t)__popcll(here & lane_lt);
+        sums[rank] = make_uint4(tri, __float_as_uint(gw_r * dr), __float_as_uint(gw_g * dg), __float_as_uint(gw_b * db));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (uint32_t j = 0; j < 3; ++j) {
+            const uint32_t slot = j * n + rank;  // of 3 n <= 192
+            const uint32_t from = (slot * 171u) >> 9, c = slot - 3u * from;  // slot / 3, exact below 256
+            const uint32_t* e = reinterpret_cast<const uint32_t*>(sums + from);
+            const float v = __uint_as_float(e[1 + c]);
+            if (v != 0.0f) atomicAdd(pl.grad + 3 * (size_t)e[0] + c, v);
+        }
+        __builtin_amdgcn_wave_barrier();
     };
 
     // Counts a ray for the frame that its path belongs to.
