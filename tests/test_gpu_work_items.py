@@ -68,3 +68,27 @@ def test_frames(dev, prt, scene, size):
     for accum, rays in got[1:]:
         assert rays == got[0][1]
         assert np.array_equal(accum.view(np.uint32), got[0][0].view(np.uint32))
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+@pytest.mark.parametrize("sizes", [[(1, 1)], [(8, 8), (9, 7)], [(64, 33), (3, 2), (31, 65)], [(256, 64), (128, 128)],
+                                   [(256, 64), (129, 128)], [(256, 192), (257, 192)]])
+def test_small_job_sets(dev, prt, scene, sizes, variant):
+    mesh, _ = scene
+    dev.upload_scene(mesh.idx, mesh.pos)
+    dev.build()
+    with prt.HipDevice(0) as batch:
+        sid, _ = batch.batch_add_scene(mesh.idx, mesh.pos)
+        cams = [prt.camera_from_view([0.0, 1.9, 2.1], 0.75, 0.0, 0.9, w / h) for w, h in sizes]
+        batch.batch_set_tuning(variant)
+        batch.batch_set_jobs([dict(scene=sid, width=w, height=h, spp=1, max_depth=5, albedo=0.8, camera=c)
+                              for (w, h), c in zip(sizes, cams)])
+        got = [batch.batch_render()["ray"] for _ in range(3)]     # as launched, captured, replayed
+        ref = np.zeros(3, np.int64)
+        for j, ((w, h), c) in enumerate(zip(sizes, cams)):
+            dev.set_camera(c)
+            dev.init_frame(w, h)
+            dev.clear_frame()
+            ref += [dev.render("diffuseHip", 5, 0.8)["ray"] for _ in range(3)]
+            assert np.array_equal(batch.batch_accum(j).view(np.uint32), dev.accum().view(np.uint32))
+        assert got == list(ref)
