@@ -1549,8 +1549,12 @@ int prt_hip_adjoint_albedo(prt_hip_ctx* ctx, int pass0, int spp, int max_depth, 
             free_ptr(ctx->d_path_hits);
             ctx->d_path_hits = nullptr;
             ctx->path_hits_cap = 0;
-            PRT_TRY(ctx, hipMalloc(&ctx->d_path_hits, sizeof(uint32_t) * (size_t)need));
-            ctx->path_hits_cap = need;
+            if (hipMalloc(&ctx->d_path_hits, sizeof(uint32_t) * (size_t)need) == hipSuccess) {
+                ctx->path_hits_cap = need;
+            } else {
+                (void)hipGetLastError();
+                ctx->d_path_hits = nullptr;  // no room: escaped paths are traced again
+            }
         }
         p.path_hits = ctx->d_path_hits;
         p.path_hits_stride = (uint32_t)lanes;
