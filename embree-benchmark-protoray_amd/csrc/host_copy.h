@@ -33,11 +33,13 @@ private:
     int left_ = 0;
 };
 
-// A few threads for memcpy-like jobs, made at first use; they never call HIP.
+// A few threads for memcpy-like jobs, made by open or at first use; they never
+// call HIP.
 // Nothing here allocates per job or throws.
 class Workers {
 public:
     ~Workers();
+    void open();
     // Runs fn(arg) on a worker (here, if there is none).
     void start(void (*fn)(void*), void* arg);
     // fn(arg, 0) .. fn(arg, n - 1), this thread helping; returns when all are done.
@@ -63,6 +65,9 @@ private:
 class HostCopy {
 public:
     ~HostCopy();
+    // Lays out the ring and starts the threads now instead of in the first large
+    // copy.  A failure is left for that copy to report.
+    void reserve();
     // Both wait until the copy is done.  Work already on the stream comes first.
     hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
     hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t s);

@@ -44,16 +44,20 @@ void Workers::run()
     }
 }
 
+void Workers::open()
+{
+    if (started_) return;
+    started_ = true;
+    try {
+        for (; nthreads_ < kThreads; ++nthreads_) threads_[nthreads_] = std::thread([this] { run(); });
+    } catch (...) {
+        // as many threads as the system gives
+    }
+}
+
 void Workers::start(void (*fn)(void*), void* arg)
 {
-    if (!started_) {
-        started_ = true;
-        try {
-            for (; nthreads_ < kThreads; ++nthreads_) threads_[nthreads_] = std::thread([this] { run(); });
-        } catch (...) {
-            // as many threads as the system gives
-        }
-    }
+    open();
     {
         std::unique_lock<std::mutex> lock(mu_);
         if (nthreads_ > 0 && count_ < kJobs) {
@@ -119,6 +123,12 @@ hipError_t HostCopy::prepare()
             if (e != hipSuccess) return e;
         }
     return hipSuccess;
+}
+
+void HostCopy::reserve()
+{
+    if (prepare() != hipSuccess) (void)hipGetLastError();
+    workers_.open();
 }
 
 // Starts the memcpy of a slot; its latch tells when it is done.

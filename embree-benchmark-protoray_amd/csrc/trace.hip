@@ -7,16 +7,16 @@
 // modes, the raygen / shade kernels and the per-bounce host loop of
 // DiffuseRendererCuda::render (render/diffuse_renderer_cuda.cu:27-120,159-212).
 //
-// One ray per lane.  The kernel is persistent: each wave takes work from a
-// global counter; when at least kRefill of its 64 lanes are idle, the wave
+// One ray per lane.  The kernel is persistent: each wave takes work from the
+// launch's counters; when at least kRefill of its 64 lanes are idle, the wave
 // ballots them, takes that many work items with one atomic and hands them out
 // by lane prefix, so lanes stay busy on incoherent bounces.  The traversal
 // stack is a per-lane ring of kStackLds entries in LDS; deeper entries spill
 // to a per-lane slice of global memory.  Each entry keeps the entry distance
 // of its box, so nodes behind the closest hit are dropped when popped.
 //
-// The loop is bound by VALU issue (about 90 % busy with 30 % of the lanes
-// active), so a step costs what it issues.  A push wraps its positions only in
+// The loop is bound by VALU issue (every slot taken, with 27 to 34 % of the
+// lanes active), so a step costs what it issues.  A push wraps its positions only in
 // waves where some stack has passed the ring's end, the node's exponents scale
 // by ldexp, the near and far offsets share one fma, a leaf slot's byte comes
 // out by one permute, and hit coordinates are computed once per ray: 1.3 M
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     unsigned long long n_wsteps = 0, n_lsteps = 0, n_wshade = 0;  // instrumented SIMT occupancy
     unsigned long long n_dwsteps = 0, n_dlsteps = 0;              // ... after the work ran out
     unsigned long long t_exhausted = 0;                           // wall clock when it ran out
-    bool exhausted = false;  // wave-uniform: the work counter has run past count
+    bool exhausted = false;  // wave-uniform: the work is handed out
     // Cooperative traversal of a wave's last paths (see coop_traverse below)
     constexpr bool kCoop = !kLook;
     const bool coop_on = kCoop && pl.coop != 0;
