@@ -902,14 +902,15 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
         bool stopped = false;  // left the loop early: no path left
         for (int depth = 0; depth <= last; ++depth) {
             traced = depth;
-            // queue size and fetch counter of depth k live in slot k mod 16
+            // the queue size of depth k lives in slot k mod 16; its shading clears
+            // the work counters for the next depth
             const int slot = depth & (kMaxQueueDepth - 1);
             TraceLaunch t{};
             t.rays = ctx->d_rays[depth & 1];
             t.hits = ctx->d_hits;
             t.count_ptr = ctx->d_counters + slot;
             t.count = 0;
-            t.work = ctx->d_counters + 16 + slot;
+            t.work = ctx->d_work;
             t.stats = counting ? ctx->d_stats : nullptr;
             const int ev = slot;  // timing events of depth k: set k mod 16, read every 16 depths
             if (timing) PRT_TRY(ctx, hipEventRecord(ctx->kev[4 * ev + 0], ctx->stream));

@@ -226,7 +226,7 @@ struct prt_hip_ctx {
     uint32_t* d_rng[2] = {nullptr, nullptr};
     // one allocation: work counters (kWorkWords), counters, statistics
     uint32_t* d_work = nullptr;
-    uint32_t* d_counters = nullptr;           // [0..15] queue sizes, [16..31] fetch, [32] error
+    uint32_t* d_counters = nullptr;           // [0..15] queue sizes, [32] error
     void* h_readback = nullptr;               // pinned host copy of d_counters + d_stats
     unsigned long long* d_stats = nullptr;    // instrumented counters
 
@@ -303,7 +303,7 @@ struct TraceLaunch {
     float* any_t;               // any-hit query: distance of a blocking triangle, or -1
     const uint32_t* count_ptr;  // device count of rays (nullptr: use count)
     uint32_t count;
-    uint32_t* work;             // work counters, zero before launch: kWorkWords, or one when count_ptr is set
+    uint32_t* work;             // work counters (kWorkWords), zero before launch
     unsigned long long* stats;  // nullptr unless instrumented
     uint32_t* err;              // error flag (nullptr: the context's)
 };

@@ -157,18 +157,20 @@ __global__ __launch_bounds__(kBlock) void k_shade_diffuse(const float4* rays_in,
                                                           const int32_t* pix_in, const uint32_t* rng_in,
                                                           const uint32_t* count_ptr, float4* rays_out,
                                                           int32_t* pix_out, uint32_t* rng_out,
-                                                          uint32_t* out_count, float4* accum,
+                                                          uint32_t* out_count, uint32_t* work, float4* accum,
                                                           const int32_t* idx, const float* pos,
                                                           const float* normals, const float* texcoords,
                                                           float throughput, int final_depth, bool overwrite)
 {
+    constexpr int kWaves = kBlock / 64;
+    __shared__ uint32_t first[kWaves + 1];
+    // the work counters of the next depth's trace
+    if (blockIdx.x == 0 && threadIdx.x < 1u << kWorkCountersLg) work[threadIdx.x * kWorkCounterStride] = 0u;
     const uint32_t count = *count_ptr;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t lt = lanes_below(lane);
-    const uint32_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-    const uint32_t nwaves = (gridDim.x * kBlock) >> 6;
-    for (uint32_t base = wave * 64; base < count; base += nwaves * 64) {
-        const uint32_t i = base + lane;
+    for (uint32_t base = blockIdx.x * kBlock; base < count; base += gridDim.x * kBlock) {
+        const uint32_t i = base + threadIdx.x;
         bool cont = false;
         float4 r0, r1;
         f3 no, nd;
@@ -202,20 +204,31 @@ __global__ __launch_bounds__(kBlock) void k_shade_diffuse(const float4* rays_in,
                 }
             }
         }
+        // one atomic per block: those on one line take 11.5 ns each.  With one
+        // per wave here, and one work counter for each depth's trace, frames of
+        // 2.07 M paths took 2.95 ms instead of 1.84, of 0.92 M (400 k mixed
+        // triangles) 2.59 instead of 2.30
         const uint64_t m = __ballot(cont);
-        if (m) {
-            const int leader = __ffsll((unsigned long long)m) - 1;
-            uint32_t ob = 0;
-            if (lane == leader) ob = atomicAdd(out_count, (uint32_t)__popcll(m));
-            ob = __shfl(ob, leader, 64);
-            if (cont) {
-                const uint32_t o = ob + (uint32_t)__popcll(m & lt);
-                rays_out[2 * (size_t)o] = make_float4(no.x, no.y, no.z, 0.0f);
-                rays_out[2 * (size_t)o + 1] = make_float4(nd.x, nd.y, nd.z, 3.402823466e38f);
-                pix_out[o] = p;
-                rng_out[o] = s;
+        if (lane == 0) first[wave] = (uint32_t)__popcll(m);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t sum = 0;
+            for (int w = 0; w < kWaves; ++w) {
+                const uint32_t c = first[w];
+                first[w] = sum;
+                sum += c;
             }
+            first[kWaves] = sum ? atomicAdd(out_count, sum) : 0u;
         }
+        __syncthreads();
+        if (cont) {
+            const uint32_t o = first[kWaves] + first[wave] + (uint32_t)__popcll(m & lt);
+            rays_out[2 * (size_t)o] = make_float4(no.x, no.y, no.z, 0.0f);
+            rays_out[2 * (size_t)o + 1] = make_float4(nd.x, nd.y, nd.z, 3.402823466e38f);
+            pix_out[o] = p;
+            rng_out[o] = s;
+        }
+        __syncthreads();
     }
 }
 
@@ -292,18 +305,17 @@ __global__ __launch_bounds__(kBlock) void k_zero_u32(uint32_t* p, int n)
     if (i < n) p[i] = 0u;
 }
 
-// Wavefront frames deeper than 16: the queue-size and fetch-counter slot of
+// Wavefront frames deeper than 16: the queue-size slot of
 // depth k is k mod 16.  Before depth d (d >= 16) reuses its slot, the count
 // of depth d - 16 moves to its statistics bin (the last bin holds depths >=
-// 15; depth 0's count is the pixel count, known on the host) and both
-// counters are cleared.
+// 15; depth 0's count is the pixel count, known on the host) and the
+// slot is cleared.
 __global__ void k_queue_recycle(uint32_t* counters, unsigned long long* stats, int old_depth)
 {
     if (threadIdx.x != 0) return;
     const int slot = old_depth & (kMaxQueueDepth - 1);
     if (old_depth > 0) stats[16 + min(old_depth, kMaxQueueDepth - 1)] += counters[slot];
     counters[slot] = 0u;
-    counters[16 + slot] = 0u;
 }
 
 // ---- batched form
@@ -469,7 +481,7 @@ hipError_t launch_shade_diffuse(prt_hip_ctx* ctx, int depth, int max_depth, floa
     const int slot = depth & (kMaxQueueDepth - 1), next = (depth + 1) & (kMaxQueueDepth - 1);
     k_shade_diffuse<<<persistent_blocks(ctx), kBlock, 0, ctx->stream>>>(
         ctx->d_rays[cur], ctx->d_hits, ctx->d_pix[cur], ctx->d_rng[cur], ctx->d_counters + slot,
-        ctx->d_rays[1 - cur], ctx->d_pix[1 - cur], ctx->d_rng[1 - cur], ctx->d_counters + next,
+        ctx->d_rays[1 - cur], ctx->d_pix[1 - cur], ctx->d_rng[1 - cur], ctx->d_counters + next, ctx->d_work,
         ctx->d_accum, ctx->scene.d_idx, ctx->scene.d_pos, fast ? nullptr : ctx->scene.d_normals,
         fast ? nullptr : ctx->scene.d_texcoords, throughput, depth == max_depth ? 1 : 0, fast);
     return hipGetLastError();

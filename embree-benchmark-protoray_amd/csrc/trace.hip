@@ -976,8 +976,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     // a small launch is traced in groups from its start (wave-uniform)
     const bool spread = kCoop && pl.coop == kCoopSpread;
     const uint32_t run_lg = spread ? 3u : 6u;
-    const uint32_t ctr_lg = kRayQuery && tl.count_ptr ? 0u : kWorkCountersLg;
-    const uint32_t ctr_last = (1u << ctr_lg) - 1u;
+    constexpr uint32_t ctr_lg = kWorkCountersLg, ctr_last = (1u << ctr_lg) - 1u;
     const uint32_t items = kLookMode && look ? lk_fresh_end : count;
     const uint32_t n_waves = gridDim.x * (uint32_t)(kBlock / 64);
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);

@@ -2,7 +2,7 @@
 counters, the first run of each wave without one.  Item counts around the
 borders (as many runs as waves, one more or less, runs that do not divide by
 16, a last run of one item) against the oracle, and frames against the
-wavefront pipeline, which counts on the device with one counter."""
+wavefront pipeline, whose launches take their counts from the device."""
 import numpy as np
 import pytest
 
