@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "launch_shape.h"
 #include "prt_internal.h"
 
 // Fixed scratch of prt_hip_intersect_closest_device_noalloc: a header
@@ -294,9 +295,9 @@ int occluded_impl(prt_hip_ctx* ctx, const prt_ray* d_rays, float* d_t, int64_t n
 }
 
 // A small query from host memory.  Its rays go to a pinned buffer that the
-// kernel reads and answers in place, and the query needs no work counter, so
-// one launch and one wait are the whole call: no staged copies, no counter
-// clear, no read of the error flag.
+// kernel reads and answers in place, and where every ray belongs to some wave's
+// first run (spread_covers) no work counter is read, so one launch and one wait are the
+// whole call: no staged copies, no counter clear, no read of the error flag.
 // 1 ray 68 -> 38 us, 1024 102 -> 65, 4096 107 -> 70, 32768 175 -> 142 (start of
 // the copies to their end, with Python); larger queries are not spread.
 constexpr int64_t kDirectRays = 32768;
@@ -313,7 +314,10 @@ struct DirectIo {
 
 bool query_direct(const prt_hip_ctx* ctx, int64_t n)
 {
-    return ctx->scene.bvh_ready && n <= kDirectRays && query_spreads(ctx, n);
+    static_assert(kDirectRays <= (int64_t)kSpreadRays, "small queries are spread");
+    constexpr int kBlockWaves = kTraceBlock / 64;
+    return ctx->scene.bvh_ready && ctx->tail_coop && n <= kDirectRays &&
+           spread_covers(spread_grid(ctx->num_cus, (uint64_t)n, kBlockWaves, ctx->trace_grid), kBlockWaves, (uint64_t)n);
 }
 
 // hits or any_t: closest or any hit

@@ -382,9 +382,6 @@ int ensure_trace_resources(prt_hip_ctx* ctx);
 // persistent workgroups of a diffuse frame of `entries` path slots under the
 // lookahead
 int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries);
-// a query of `rays` rays is spread over the waves from its start, without the
-// work counter
-bool query_spreads(const prt_hip_ctx* ctx, int64_t rays);
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented);
 // closest-hit launch over at most max_grid persistent workgroups whose stack
 // spill (stack_entries per lane) and error flag the caller provides

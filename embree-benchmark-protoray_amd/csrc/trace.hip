@@ -46,6 +46,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "launch_shape.h"
 #include "prt_internal.h"
 
 namespace prt {
@@ -1551,31 +1552,9 @@ uint64_t launch_items(int mode, const TraceLaunch& t, const PathLaunch& p)
     return p.entries;
 }
 
-// Launches of at most this many items are traced in groups of 8 lanes from
-// their start: with so few, a launch takes as long as its longest path's chain
-// of steps, and a step of a group is shorter.  Above, throughput decides: a
-// group's 8 lanes do the work of one.  Measured lane by lane / in groups, us:
-//   closest hits  512 rays 112 / 73, 8192 144 / 92, 32768 172 / 104,
-//                 49152 174 / 177, 65536 173 / 217
-//   primary       9216 74 / 46, 32256 83 / 82, 64000 107 / 126
-//   diffuse       32256 265 / 172, 64000 324 / 279, 96000 584 / 473, 286 /
-//                 283, 324 / 319 (three scenes), 140000 314 / 356
-//   diffuse2      32256 425 / 317, 64000 467 / 381, 96000 939 / 762, 454 /
-//                 409, 140000 484 / 494
-// The albedo modes trace the same paths as diffuse.
-constexpr uint64_t kSpreadRays = 32768, kSpreadPaths = 96 << 10;
-
 uint64_t spread_limit(int mode)
 {
     return mode == kModeTrace || mode == kModeOccluded || mode == kModePrimary ? kSpreadRays : kSpreadPaths;
-}
-
-// Workgroups of such a launch: a wave per 8 items, on as many CUs as there are
-// waves, then up to all waves of each.
-int spread_grid(const prt_hip_ctx* ctx, uint64_t items, int block_waves, int most)
-{
-    const int waves = (int)std::min<uint64_t>((items + 7) / 8, 1u << 30);
-    return std::min(most, std::max(1, std::max(std::min(waves, ctx->num_cus), (waves + block_waves - 1) / block_waves)));
 }
 
 // Tail mode and grid of a launch.
@@ -1584,7 +1563,7 @@ int launch_shape(const prt_hip_ctx* ctx, int mode, uint64_t items, int& coop)
     coop = ctx->tail_coop ? kCoopTail : 0;
     if (coop && items <= spread_limit(mode)) {
         coop = kCoopSpread;
-        return spread_grid(ctx, items, kTraceBlock / 64, ctx->trace_grid);
+        return spread_grid(ctx->num_cus, items, kTraceBlock / 64, ctx->trace_grid);
     }
     return grid_for(ctx, mode, items);
 }
@@ -1639,7 +1618,7 @@ hipError_t launch_batch_variant(prt_hip_ctx* ctx, const BatchLaunch& bl, int blo
     // 16 k 43 / 39, 20 k 44 / 43, 40 k 44 / 71, so these stop at the rays' limit.
     if (p.coop && bl.total_work <= kSpreadRays) {
         p.coop = kCoopSpread;
-        grid = spread_grid(ctx, bl.total_work, kBlock / 64, grid);
+        grid = spread_grid(ctx->num_cus, bl.total_work, kBlock / 64, grid);
     }
     if (instrumented)
         k_trace<true, kModeBatch, kBlock, kStack><<<grid, kBlock, 0, ctx->stream>>>(
@@ -1698,11 +1677,6 @@ int ensure_trace_resources(prt_hip_ctx* ctx)
 }
 
 int diffuse_grid(const prt_hip_ctx* ctx, uint32_t entries) { return grid_for(ctx, kModeDiffuse, entries, true); }
-
-bool query_spreads(const prt_hip_ctx* ctx, int64_t rays)
-{
-    return ctx->tail_coop && rays >= 0 && (uint64_t)rays <= kSpreadRays;
-}
 
 hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool instrumented)
 {

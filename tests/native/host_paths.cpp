@@ -1,0 +1,165 @@
+// Host control flow of the library against a stand-in for the HIP runtime
+// (hip/hip_runtime.h beside this file): the entry points as they are, with the
+// launches replaced by what their kernels leave in memory.
+//   host_paths NAME   runs one check; prints what failed and returns 1
+#include <cstdio>
+
+#include "../../embree-benchmark-protoray_amd/csrc/api.hip"
+#include "../../embree-benchmark-protoray_amd/csrc/host_copy.hip"
+#include "../../embree-benchmark-protoray_amd/csrc/launch_shape.h"
+
+namespace {
+
+int g_failed = 0;
+#define EXPECT(cond)                                                        \
+    do {                                                                    \
+        if (!(cond)) {                                                      \
+            std::printf("%s:%d: %s\n", __FILE__, __LINE__, #cond);          \
+            g_failed = 1;                                                   \
+        }                                                                   \
+    } while (0)
+
+int g_per_cu = 4;                 // workgroups per CU that fit
+
+// A ray's record: its own first origin coordinate, so that a test knows it.
+prt_hit answer(const float4& r0) { return prt_hit{r0.x, 7, 0.25f, 0.5f}; }
+
+// What a query launch writes: the waves' first runs always, the others only if
+// the work counters start from zero.
+hipError_t query(prt_hip_ctx* ctx, const prt::TraceLaunch& t, bool any)
+{
+    const uint64_t n = t.count;
+    const bool spread = ctx->tail_coop && n <= prt::kSpreadRays;
+    uint64_t reached = n;
+    if (spread) reached = 4 * prt::kSpreadRun * (uint64_t)prt::spread_grid(ctx->num_cus, n, 4, ctx->trace_grid);
+    for (int w = 0; w < prt::kWorkWords; w += prt::kWorkCounterStride)
+        if (t.work[w] == 0) reached = n;
+    for (uint64_t k = 0; k < std::min(n, reached); ++k) {
+        if (any) t.any_t[k] = t.rays[2 * k].x;
+        else reinterpret_cast<prt_hit*>(t.hits)[k] = answer(t.rays[2 * k]);
+    }
+    for (int w = 0; w < prt::kWorkWords; w += prt::kWorkCounterStride) t.work[w] += 12345;  // what a launch leaves
+    return hipSuccess;
+}
+
+}  // namespace
+
+namespace prt {
+
+int ensure_trace_resources(prt_hip_ctx* ctx)
+{
+    ctx->trace_per_cu = g_per_cu;
+    ctx->trace_grid = g_per_cu * ctx->num_cus;
+    return 0;
+}
+int diffuse_grid(const prt_hip_ctx* ctx, uint32_t) { return ctx->trace_grid; }
+hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool) { return query(ctx, t, false); }
+hipError_t launch_occluded(prt_hip_ctx* ctx, const TraceLaunch& t, bool) { return query(ctx, t, true); }
+hipError_t launch_trace_scratch(prt_hip_ctx*, const TraceLaunch&, uint2*, int, uint32_t*, int) { return hipSuccess; }
+hipError_t launch_zero_u32(uint32_t* p, int n, hipStream_t) { std::memset(p, 0, 4 * (size_t)n); return hipSuccess; }
+hipError_t launch_paths(prt_hip_ctx*, const PathLaunch&, int, bool) { return hipSuccess; }
+hipError_t launch_look_call_begin(prt_hip_ctx*, bool, uint32_t) { return hipSuccess; }
+hipError_t launch_paths_rgb(prt_hip_ctx*, const PathLaunch&, bool) { return hipSuccess; }
+hipError_t launch_adjoint(prt_hip_ctx*, const PathLaunch&, bool) { return hipSuccess; }
+const BatchKernelConfig kBatchVariants[kBatchVariantCount] = {{256, 16}, {256, 8}, {128, 16}, {128, 8}};
+hipError_t launch_batch(prt_hip_ctx*, const BatchLaunch&, const BatchTuning&, bool, int* max_blocks_per_cu)
+{
+    if (max_blocks_per_cu) *max_blocks_per_cu = g_per_cu;
+    return hipSuccess;
+}
+hipError_t launch_raygen(prt_hip_ctx*, int, float4*, int32_t*, uint32_t*) { return hipSuccess; }
+hipError_t launch_frame_begin(prt_hip_ctx*, uint32_t) { return hipSuccess; }
+hipError_t launch_shade_diffuse(prt_hip_ctx*, int, int, float, bool) { return hipSuccess; }
+hipError_t launch_queue_recycle(prt_hip_ctx*, int) { return hipSuccess; }
+hipError_t launch_shade_primary(prt_hip_ctx*, bool) { return hipSuccess; }
+hipError_t launch_tonemap(prt_hip_ctx*) { return hipSuccess; }
+hipError_t launch_batch_begin(prt_hip_ctx*) { return hipSuccess; }
+hipError_t launch_accum_mean_rgb(prt_hip_ctx*, float*) { return hipSuccess; }
+hipError_t launch_rgb_planes_add(prt_hip_ctx*, const float4*, int) { return hipSuccess; }
+hipError_t launch_batch_finalize(prt_hip_ctx*) { return hipSuccess; }
+hipError_t launch_batch_advance(prt_hip_ctx*) { return hipSuccess; }
+hipError_t launch_unpack_rays(const float4*, const int32_t*, const uint32_t*, int64_t, int, int, prt_ray*, uint32_t*,
+                              hipStream_t)
+{
+    return hipSuccess;
+}
+Camera to_camera(const prt_camera&) { return Camera{}; }
+int build_bvh8(prt_hip_ctx*, SceneBuffers& sb, prt_build_stats*)
+{
+    sb.bvh_ready = true;
+    sb.bvh_depth = 4;
+    sb.node_count = 1;
+    return 0;
+}
+
+}  // namespace prt
+
+namespace {
+
+struct Context {
+    prt_hip_ctx* ctx = nullptr;
+    explicit Context(int num_cus = 256, int per_cu = 4)
+    {
+        fake::state().num_cus = num_cus;
+        g_per_cu = per_cu;
+        EXPECT(prt_hip_create(0, &ctx) == 0);
+    }
+    ~Context() { EXPECT(prt_hip_destroy(ctx) == 0); }
+    operator prt_hip_ctx*() const { return ctx; }
+};
+
+const int32_t kIdx[3] = {0, 1, 2};
+const float kPos[9] = {0, 0, 0, 1, 0, 0, 0, 1, 0};
+
+void with_scene(prt_hip_ctx* ctx)
+{
+    EXPECT(prt_hip_scene_upload(ctx, kIdx, 1, kPos, 3) == 0);
+    EXPECT(prt_hip_bvh_build(ctx, nullptr) == 0);
+}
+
+// Every ray of a small host query is answered on devices of any size: the
+// launch goes without work counters only where each ray has a wave.
+void small_query_on_small_devices()
+{
+    for (int num_cus : {1, 4, 32, 64, 128, 255, 256, 304})
+        for (int per_cu : {1, 2, 3, 4, 8}) {
+            Context c(num_cus, per_cu);
+            with_scene(c);
+            float base = 1.0f;
+            for (int64_t n : {1, 7, 8, 9, 31, 1000, 8191, 8192, 8193, 24577, 32767, 32768, 32769, 1}) {
+                std::vector<prt_ray> rays(n);
+                for (int64_t k = 0; k < n; ++k) reinterpret_cast<float*>(&rays[k])[0] = base + (float)k;
+                std::vector<prt_hit> hits(n);
+                std::vector<float> any(n);
+                EXPECT(prt_hip_intersect_closest(c, rays.data(), hits.data(), n) == 0);
+                EXPECT(prt_hip_occluded(c, rays.data(), any.data(), n) == 0);
+                int64_t bad = 0;
+                for (int64_t k = 0; k < n; ++k)
+                    bad += reinterpret_cast<const float*>(&hits[k])[0] != base + (float)k || any[k] != base + (float)k;
+                if (bad) std::printf("%d CUs, %d workgroups each, %lld rays: %lld not answered\n", num_cus, per_cu,
+                                     (long long)n, (long long)bad);
+                EXPECT(bad == 0);
+                base += 100000.0f;
+            }
+        }
+}
+
+const struct {
+    const char* name;
+    void (*run)();
+} kChecks[] = {
+    {"small_query_on_small_devices", small_query_on_small_devices},
+};
+
+}  // namespace
+
+int main(int argc, char** argv)
+{
+    for (const auto& c : kChecks)
+        if (argc > 1 && std::strcmp(argv[1], c.name) == 0) {
+            c.run();
+            return g_failed;
+        }
+    std::printf("no such check\n");
+    return 2;
+}
