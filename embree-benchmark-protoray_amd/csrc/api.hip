@@ -260,11 +260,14 @@ double wall_clock_hz(prt_hip_ctx* ctx)
     return (double)khz * 1e3;
 }
 
+// What the queries accept; asked before any copy of n rays.
+bool ray_count_ok(int64_t n) { return n >= 0 && n <= (int64_t)UINT32_MAX / 2; }
+
 int intersect_impl(prt_hip_ctx* ctx, const prt_ray* d_rays, prt_hit* d_hits, int64_t n,
                    unsigned long long* d_stats)
 {
     if (!ctx->scene.bvh_ready) return set_error(ctx, "intersect: no BVH (call prt_hip_bvh_build)");
-    if (n < 0 || n > (int64_t)UINT32_MAX / 2) return set_error(ctx, "intersect: bad ray count");
+    if (!ray_count_ok(n)) return set_error(ctx, "intersect: bad ray count");
     if (ensure_trace_resources(ctx)) return 1;
     PRT_TRY(ctx, launch_zero_u32(ctx->d_work, kWorkWords + 33, ctx->stream));
     TraceLaunch t{};
@@ -281,7 +284,7 @@ int intersect_impl(prt_hip_ctx* ctx, const prt_ray* d_rays, prt_hit* d_hits, int
 int occluded_impl(prt_hip_ctx* ctx, const prt_ray* d_rays, float* d_t, int64_t n)
 {
     if (!ctx->scene.bvh_ready) return set_error(ctx, "occluded: no BVH (call prt_hip_bvh_build)");
-    if (n < 0 || n > (int64_t)UINT32_MAX / 2) return set_error(ctx, "occluded: bad ray count");
+    if (!ray_count_ok(n)) return set_error(ctx, "occluded: bad ray count");
     if (ensure_trace_resources(ctx)) return 1;
     PRT_TRY(ctx, launch_zero_u32(ctx->d_work, kWorkWords + 33, ctx->stream));
     TraceLaunch t{};
@@ -504,7 +507,8 @@ int prt_hip_intersect_closest(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* hi
     if (use_device(ctx)) return 1;
     if (n == 0) return 0;
     if (!rays || !hits) return set_error(ctx, "intersect: null array");
-    if (n > 0 && query_direct(ctx, n)) return run_direct(ctx, rays, hits, nullptr, n);
+    if (!ray_count_ok(n)) return set_error(ctx, "intersect: bad ray count");
+    if (query_direct(ctx, n)) return run_direct(ctx, rays, hits, nullptr, n);
     if (ensure_io(ctx, n)) return 1;
     PRT_TRY(ctx, ctx->copy.to_device(ctx->d_io_rays, rays, sizeof(prt_ray) * n, ctx->stream));
     if (intersect_impl(ctx, reinterpret_cast<prt_ray*>(ctx->d_io_rays),
@@ -520,7 +524,7 @@ int prt_hip_intersect_closest_device_noalloc(prt_hip_ctx* ctx, const prt_ray* d_
     if (use_device(ctx)) return 1;
     if (!ctx->scene.bvh_ready || ctx->trace_per_cu <= 0)
         return set_error(ctx, "intersect_noalloc: no BVH (call prt_hip_bvh_build)");
-    if (n < 0 || n > (int64_t)UINT32_MAX / 2) return set_error(ctx, "intersect_noalloc: bad ray count");
+    if (!ray_count_ok(n)) return set_error(ctx, "intersect_noalloc: bad ray count");
     if (n == 0) return 0;
     if (!d_rays || !d_hits) return set_error(ctx, "intersect_noalloc: null array");
     if (!ctx->d_scratch) return set_error(ctx, "intersect_noalloc: no scratch on this device");
@@ -562,7 +566,8 @@ int prt_hip_occluded(prt_hip_ctx* ctx, const prt_ray* rays, float* out_t, int64_
     if (use_device(ctx)) return 1;
     if (n == 0) return 0;
     if (!rays || !out_t) return set_error(ctx, "occluded: null array");
-    if (n > 0 && query_direct(ctx, n)) return run_direct(ctx, rays, nullptr, out_t, n);
+    if (!ray_count_ok(n)) return set_error(ctx, "occluded: bad ray count");
+    if (query_direct(ctx, n)) return run_direct(ctx, rays, nullptr, out_t, n);
     if (ensure_io(ctx, n)) return 1;
     float* d_t = reinterpret_cast<float*>(ctx->d_io_hits);  // n floats fit in the n-hit buffer
     PRT_TRY(ctx, ctx->copy.to_device(ctx->d_io_rays, rays, sizeof(prt_ray) * n, ctx->stream));
@@ -578,6 +583,7 @@ int prt_hip_intersect_counters(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* h
     if (use_device(ctx)) return 1;
     if (!rays || !hits || !out) return set_error(ctx, "intersect_counters: null argument");
     if (n == 0) { std::memset(out, 0, sizeof(*out)); return 0; }
+    if (!ray_count_ok(n)) return set_error(ctx, "intersect_counters: bad ray count");
     if (ensure_io(ctx, n)) return 1;
     PRT_TRY(ctx, hipMemsetAsync(ctx->d_stats, 0, 16 * sizeof(unsigned long long), ctx->stream));
     PRT_TRY(ctx, hipMemcpyAsync(ctx->d_io_rays, rays, sizeof(prt_ray) * n, hipMemcpyHostToDevice, ctx->stream));

@@ -144,11 +144,35 @@ void small_query_on_small_devices()
         }
 }
 
+// A count that no query accepts is refused before anything is copied.
+void bad_ray_counts()
+{
+    Context c;
+    with_scene(c);
+    std::vector<prt_ray> rays(4);
+    std::vector<prt_hit> hits(4);
+    std::vector<float> any(4);
+    prt_trace_counters counters;
+    const size_t copies = fake::state().copies.size();
+    for (int64_t n : {(int64_t)-1, (int64_t)-2, -((int64_t)1 << 21), -((int64_t)3 << 46), -((int64_t)1 << 62), INT64_MIN,
+                      (int64_t)1 << 31, (int64_t)1 << 58, INT64_MAX}) {
+        EXPECT(prt_hip_intersect_closest(c, rays.data(), hits.data(), n) != 0);
+        EXPECT(prt_hip_occluded(c, rays.data(), any.data(), n) != 0);
+        EXPECT(prt_hip_intersect_counters(c, rays.data(), hits.data(), n, &counters) != 0);
+        EXPECT(std::string(prt_hip_last_error(c)).find("bad ray count") != std::string::npos);
+        EXPECT(prt_hip_intersect_closest_device(c, rays.data(), hits.data(), n) != 0);
+        EXPECT(prt_hip_occluded_device(c, rays.data(), any.data(), n) != 0);
+    }
+    EXPECT(fake::state().copies.size() == copies);
+    EXPECT(prt_hip_intersect_closest(c, rays.data(), hits.data(), 4) == 0);
+}
+
 const struct {
     const char* name;
     void (*run)();
 } kChecks[] = {
     {"small_query_on_small_devices", small_query_on_small_devices},
+    {"bad_ray_counts", bad_ray_counts},
 };
 
 }  // namespace
