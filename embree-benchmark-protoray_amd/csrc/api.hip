@@ -315,19 +315,26 @@ struct DirectIo {
     };
 };
 
-bool query_direct(const prt_hip_ctx* ctx, int64_t n)
+// The query can go this way; lays out the pinned buffer.  Where the system gives
+// none, small queries are copied as large ones are.
+bool query_direct(prt_hip_ctx* ctx, int64_t n)
 {
     static_assert(kDirectRays <= (int64_t)kSpreadRays, "small queries are spread");
     constexpr int kBlockWaves = kTraceBlock / 64;
-    return ctx->scene.bvh_ready && ctx->tail_coop && n <= kDirectRays &&
-           spread_covers(spread_grid(ctx->num_cus, (uint64_t)n, kBlockWaves, ctx->trace_grid), kBlockWaves, (uint64_t)n);
+    if (!ctx->scene.bvh_ready || !ctx->tail_coop || n > kDirectRays ||
+        !spread_covers(spread_grid(ctx->num_cus, (uint64_t)n, kBlockWaves, ctx->trace_grid), kBlockWaves, (uint64_t)n))
+        return false;
+    if (!ctx->h_direct && hipHostMalloc(&ctx->h_direct, sizeof(DirectIo), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->h_direct = nullptr;
+    }
+    return ctx->h_direct != nullptr;
 }
 
 // hits or any_t: closest or any hit
 int run_direct(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* hits, float* any_t, int64_t n)
 {
     if (ensure_trace_resources(ctx)) return 1;
-    if (!ctx->h_direct) PRT_TRY(ctx, hipHostMalloc(&ctx->h_direct, sizeof(DirectIo), hipHostMallocDefault));
     DirectIo* io = static_cast<DirectIo*>(ctx->h_direct);
     io->err = 0;
     std::memcpy(io->rays, rays, sizeof(prt_ray) * (size_t)n);

@@ -66,7 +66,8 @@ class HostCopy {
 public:
     ~HostCopy();
     // Lays out the ring and starts the threads now instead of in the first large
-    // copy.  A failure is left for that copy to report.
+    // copy.  Where the system gives no pinned memory, copies go through the
+    // runtime's own staging.
     void reserve();
     // Both wait until the copy is done.  Work already on the stream comes first.
     hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
@@ -82,12 +83,14 @@ private:
         size_t bytes;
         Latch copied;
     };
-    hipError_t prepare();
+    bool prepare();
+    static hipError_t plain(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s);
     void hand(int slot, void* to, const void* from, size_t bytes);
     Workers workers_;
     Slot slots_[kSlots];
     char* ring_ = nullptr;          // kSlots * kChunk, pinned
     hipEvent_t ev_[kSlots] = {};    // last DMA of each slot
+    bool refused_ = false;          // no ring: the system gave no pinned memory
 };
 
 }  // namespace prt

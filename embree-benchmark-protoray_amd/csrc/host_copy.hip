@@ -108,27 +108,34 @@ HostCopy::~HostCopy()
     if (ring_) (void)hipHostFree(ring_);
 }
 
-hipError_t HostCopy::prepare()
+bool HostCopy::prepare()
 {
-    if (!ring_) {
-        const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&ring_), kSlots * kChunk, hipHostMallocDefault);
-        if (e != hipSuccess) {
-            ring_ = nullptr;
-            return e;
-        }
+    if (refused_) return false;
+    if (!ring_ &&
+        hipHostMalloc(reinterpret_cast<void**>(&ring_), kSlots * kChunk, hipHostMallocDefault) != hipSuccess) {
+        ring_ = nullptr;
+        refused_ = true;
     }
     for (hipEvent_t& v : ev_)
-        if (!v) {
-            const hipError_t e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
-            if (e != hipSuccess) return e;
+        if (!refused_ && !v && hipEventCreateWithFlags(&v, hipEventDisableTiming) != hipSuccess) {
+            v = nullptr;
+            refused_ = true;
         }
-    return hipSuccess;
+    if (refused_) (void)hipGetLastError();
+    return !refused_;
 }
 
 void HostCopy::reserve()
 {
-    if (prepare() != hipSuccess) (void)hipGetLastError();
-    workers_.open();
+    if (prepare()) workers_.open();
+}
+
+// One copy by the runtime, which stages pageable memory itself.
+hipError_t HostCopy::plain(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s)
+{
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
+    const hipError_t w = hipStreamSynchronize(s);
+    return e == hipSuccess ? w : e;
 }
 
 // Starts the memcpy of a slot; its latch tells when it is done.
@@ -151,8 +158,8 @@ void HostCopy::hand(int slot, void* to, const void* from, size_t bytes)
 hipError_t HostCopy::to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
 {
     if (bytes == 0) return hipStreamSynchronize(s);
-    hipError_t e = prepare();
-    if (e != hipSuccess) return e;
+    if (!prepare()) return plain(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    hipError_t e = hipSuccess;
     char* out = static_cast<char*>(dst);
     const char* in = static_cast<const char*>(src);
     if (bytes <= kChunk) {
@@ -203,14 +210,9 @@ hipError_t HostCopy::to_host(void* dst, const void* src, size_t bytes, hipStream
 hipError_t HostCopy::to_device(void* dst, const void* src, size_t bytes, hipStream_t s)
 {
     if (bytes == 0) return hipSuccess;
-    if (bytes <= 2 * kChunk) {
-        // too little to gain from a second thread: the runtime's own staging
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
-        const hipError_t w = hipStreamSynchronize(s);
-        return e == hipSuccess ? w : e;
-    }
-    hipError_t e = prepare();
-    if (e != hipSuccess) return e;
+    // too little to gain from a second thread: the runtime's own staging
+    if (bytes <= 2 * kChunk || !prepare()) return plain(dst, src, bytes, hipMemcpyHostToDevice, s);
+    hipError_t e = hipSuccess;
     char* out = static_cast<char*>(dst);
     const char* in = static_cast<const char*>(src);
     // chunk c: a worker fills slot c mod kSlots, then the DMA; the slot is

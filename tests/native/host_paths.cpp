@@ -167,12 +167,78 @@ void bad_ray_counts()
     EXPECT(prt_hip_intersect_closest(c, rays.data(), hits.data(), 4) == 0);
 }
 
+// Without pinned memory beyond the context's own small block, every host copy and
+// query still does its work.
+void no_pinned_memory()
+{
+    fake::state().pinned_fail_from = 2;
+    Context c;
+    with_scene(c);
+    for (int64_t n : {1, 1000, 40000, 300000}) {
+        std::vector<prt_ray> rays(n);
+        for (int64_t k = 0; k < n; ++k) reinterpret_cast<float*>(&rays[k])[0] = 3.0f + (float)k;
+        std::vector<prt_hit> hits(n);
+        std::vector<float> any(n);
+        EXPECT(prt_hip_intersect_closest(c, rays.data(), hits.data(), n) == 0);
+        EXPECT(prt_hip_occluded(c, rays.data(), any.data(), n) == 0);
+        for (int64_t k = 0; k < n; k += n > 1 ? n - 1 : 1)
+            EXPECT(reinterpret_cast<const float*>(&hits[k])[0] == 3.0f + (float)k && any[k] == 3.0f + (float)k);
+    }
+    for (int w : {1, 64, 700, 1500}) {
+        EXPECT(prt_hip_frame_init(c, w, w) == 0);
+        std::vector<float> image((size_t)4 * w * w, -1.0f);
+        EXPECT(prt_hip_accum_read(c, image.data()) == 0);
+        EXPECT(image.front() == 0.0f && image.back() == 0.0f);
+    }
+    EXPECT(hipGetLastError() == hipSuccess);   // a launch check would take it for its own
+}
+
+// Copies of every length class, one chunk, two halves, a ring that wraps, both
+// ways and with two contexts on two threads at once; then copies that fail part
+// way, after which the next one works.
+void host_copies()
+{
+    constexpr size_t kChunk = size_t(2) << 20;
+    auto copies = [](uint32_t seed) {
+        HostCopy copy;
+        for (size_t bytes : {(size_t)1, kChunk / 4, kChunk / 4 + 1, kChunk - 1, kChunk, kChunk + 1, 2 * kChunk, 2 * kChunk + 1,
+                             5 * kChunk, 6 * kChunk - 3, 6 * kChunk, 6 * kChunk + 1, 13 * kChunk + 12345}) {
+            std::vector<unsigned char> src(bytes), dst(bytes + 2, 0xee);
+            uint32_t s = seed + (uint32_t)bytes;
+            for (unsigned char& b : src) b = (unsigned char)((s = s * 1664525u + 1013904223u) >> 24);
+            EXPECT(copy.to_host(dst.data() + 1, src.data(), bytes, nullptr) == hipSuccess);
+            EXPECT(std::memcmp(dst.data() + 1, src.data(), bytes) == 0 && dst.front() == 0xee && dst.back() == 0xee);
+            std::fill(dst.begin(), dst.end(), (unsigned char)0xee);
+            EXPECT(copy.to_device(dst.data() + 1, src.data(), bytes, nullptr) == hipSuccess);
+            EXPECT(std::memcmp(dst.data() + 1, src.data(), bytes) == 0 && dst.front() == 0xee && dst.back() == 0xee);
+        }
+    };
+    std::thread other([&] { copies(99); });
+    copies(1);
+    other.join();
+    HostCopy copy;
+    std::vector<unsigned char> src(9 * kChunk + 5, 7), dst(src.size(), 0);
+    for (int fail = 1; fail <= 11; ++fail)
+        for (int up = 0; up < 2; ++up) {
+            fake::state().copy_fail_at = fake::state().copy_calls + fail;
+            const hipError_t e = up ? copy.to_device(dst.data(), src.data(), src.size(), nullptr)
+                                    : copy.to_host(dst.data(), src.data(), src.size(), nullptr);
+            EXPECT((e != hipSuccess) == (fail <= 10));
+            fake::state().copy_fail_at = 1 << 30;
+            std::fill(dst.begin(), dst.end(), (unsigned char)0);
+            EXPECT(copy.to_host(dst.data(), src.data(), src.size(), nullptr) == hipSuccess && dst == src);
+            (void)hipGetLastError();
+        }
+}
+
 const struct {
     const char* name;
     void (*run)();
 } kChecks[] = {
     {"small_query_on_small_devices", small_query_on_small_devices},
     {"bad_ray_counts", bad_ray_counts},
+    {"no_pinned_memory", no_pinned_memory},
+    {"host_copies", host_copies},
 };
 
 }  // namespace

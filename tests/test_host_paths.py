@@ -24,6 +24,8 @@ def exe(tmp_path_factory):
 @pytest.mark.parametrize("name", [
     "small_query_on_small_devices",
     "bad_ray_counts",
+    "no_pinned_memory",
+    "host_copies",
 ])
 def test_host_path(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
