@@ -8,7 +8,8 @@
 // MB 1030 -> 454, 1.2 MB 111 -> 76; 24 MB of a scene up 1599 -> 998.  Copies up
 // of at most 4 MB stay with the runtime's own staging: waking a worker costs
 // more than it saves (1.6 MB of rays and 0.8 MB of hits 146 us with it, 232
-// with quarter chunks on the workers).
+// with quarter chunks on the workers).  Memory that the caller has pinned is
+// copied by one DMA without the ring.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -77,6 +78,7 @@ public:
 private:
     static constexpr int kSlots = 6;
     static constexpr size_t kChunk = size_t(2) << 20;
+    static constexpr size_t kAskBytes = size_t(64) << 10;  // a smaller copy gains less than the question costs
     struct Slot {
         void* to;
         const void* from;

@@ -155,10 +155,22 @@ void HostCopy::hand(int slot, void* to, const void* from, size_t bytes)
         &s);
 }
 
+// The caller's memory is pinned (or the device's): the DMA engine takes it
+// where it is.  Asked for copies of at least kAskBytes only.
+static bool takes_dma(const void* p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();  // memory that HIP does not know is an error to it
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
 hipError_t HostCopy::to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
 {
     if (bytes == 0) return hipStreamSynchronize(s);
-    if (!prepare()) return plain(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    if ((bytes >= kAskBytes && takes_dma(dst)) || !prepare()) return plain(dst, src, bytes, hipMemcpyDeviceToHost, s);
     hipError_t e = hipSuccess;
     char* out = static_cast<char*>(dst);
     const char* in = static_cast<const char*>(src);
@@ -211,7 +223,7 @@ hipError_t HostCopy::to_device(void* dst, const void* src, size_t bytes, hipStre
 {
     if (bytes == 0) return hipSuccess;
     // too little to gain from a second thread: the runtime's own staging
-    if (bytes <= 2 * kChunk || !prepare()) return plain(dst, src, bytes, hipMemcpyHostToDevice, s);
+    if (bytes <= 2 * kChunk || takes_dma(src) || !prepare()) return plain(dst, src, bytes, hipMemcpyHostToDevice, s);
     hipError_t e = hipSuccess;
     char* out = static_cast<char*>(dst);
     const char* in = static_cast<const char*>(src);

@@ -231,6 +231,34 @@ void host_copies()
         }
 }
 
+// Pinned memory of the caller is copied in one piece, straight to or from it;
+// pageable memory in chunks through the ring.
+void pinned_caller()
+{
+    HostCopy copy;
+    for (size_t bytes : {(size_t)64 << 10, (size_t)1 << 20, (size_t)5 << 20, ((size_t)40 << 20) + 4}) {
+        char *pinned = nullptr, *device = nullptr;
+        EXPECT(hipHostMalloc(&pinned, bytes + 8, hipHostMallocDefault) == hipSuccess);
+        EXPECT(hipMalloc(&device, bytes) == hipSuccess);
+        std::memset(device, 5, bytes);
+        auto& copies = fake::state().copies;
+        copies.clear();
+        EXPECT(copy.to_host(pinned + 4, device, bytes, nullptr) == hipSuccess);   // inside the allocation
+        EXPECT(copies.size() == 1 && copies[0].dst == pinned + 4 && copies[0].bytes == bytes);
+        EXPECT(pinned[3] == 0 && pinned[4] == 5 && pinned[3 + bytes] == 5 && pinned[4 + bytes] == 0);
+        copies.clear();
+        EXPECT(copy.to_device(device, pinned, bytes, nullptr) == hipSuccess);
+        EXPECT(copies.size() == 1 && copies[0].src == pinned && copies[0].bytes == bytes);
+        std::vector<char> pageable(bytes, 9);
+        copies.clear();
+        EXPECT(copy.to_device(device, pageable.data(), bytes, nullptr) == hipSuccess);
+        EXPECT(bytes <= (size_t)4 << 20 || copies.size() > 2);
+        EXPECT(device[0] == 9 && device[bytes - 1] == 9);
+        EXPECT(hipGetLastError() == hipSuccess);
+        EXPECT(hipFree(device) == hipSuccess && hipHostFree(pinned) == hipSuccess);
+    }
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -239,6 +267,7 @@ const struct {
     {"bad_ray_counts", bad_ray_counts},
     {"no_pinned_memory", no_pinned_memory},
     {"host_copies", host_copies},
+    {"pinned_caller", pinned_caller},
 };
 
 }  // namespace

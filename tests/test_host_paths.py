@@ -26,6 +26,7 @@ def exe(tmp_path_factory):
     "bad_ray_counts",
     "no_pinned_memory",
     "host_copies",
+    "pinned_caller",
 ])
 def test_host_path(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
