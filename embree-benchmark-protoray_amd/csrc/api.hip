@@ -395,9 +395,11 @@ int prt_hip_create(int device_index, prt_hip_ctx** out_ctx)
     }
     ctx->d_counters = ctx->d_work + kWorkWords;
     ctx->d_stats = reinterpret_cast<unsigned long long*>(ctx->d_counters + 64);
-    // 90 us here (50 -> 137 us a create); a context's first image of 5 MB took
-    // 1.85 ms where the first large copy did it, 1.1 ms so
-    ctx->copy.reserve();
+    // the ring here, its threads with the first large copy: a create takes 115 us
+    // (without the ring 95, with the threads 150), a first image of 5 MB 215 us
+    // (ring laid out by it 235; in a process's first two contexts 1.1 ms either
+    // way, most of it the runtime's first use of a copy engine)
+    (void)ctx->copy.prepare();
     ctx->num_cus = prop.multiProcessorCount;
     ctx->device_name = prop.name[0] ? std::string(prop.name) : std::string("AMD ") + prop.gcnArchName;
     if (hipMemsetAsync(ctx->d_work, 0, (kWorkWords + 64) * sizeof(uint32_t), ctx->stream) != hipSuccess ||

@@ -34,13 +34,12 @@ private:
     int left_ = 0;
 };
 
-// A few threads for memcpy-like jobs, made by open or at first use; they never
+// A few threads for memcpy-like jobs, started by the first of them; they never
 // call HIP.
 // Nothing here allocates per job or throws.
 class Workers {
 public:
     ~Workers();
-    void open();
     // Runs fn(arg) on a worker (here, if there is none).
     void start(void (*fn)(void*), void* arg);
     // fn(arg, 0) .. fn(arg, n - 1), this thread helping; returns when all are done.
@@ -53,6 +52,7 @@ private:
         void (*fn)(void*);
         void* arg;
     };
+    void open();
     void run();
     std::mutex mu_;
     std::condition_variable wake_;
@@ -66,10 +66,9 @@ private:
 class HostCopy {
 public:
     ~HostCopy();
-    // Lays out the ring and starts the threads now instead of in the first large
-    // copy.  Where the system gives no pinned memory, copies go through the
-    // runtime's own staging.
-    void reserve();
+    // Lays out the ring; false: the system gives no pinned memory, and copies go
+    // through the runtime's own staging.  The first copy does it if nobody has.
+    bool prepare();
     // Both wait until the copy is done.  Work already on the stream comes first.
     hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
     hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t s);
@@ -85,7 +84,6 @@ private:
         size_t bytes;
         Latch copied;
     };
-    bool prepare();
     static hipError_t plain(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s);
     void hand(int slot, void* to, const void* from, size_t bytes);
     Workers workers_;

@@ -125,11 +125,6 @@ bool HostCopy::prepare()
     return !refused_;
 }
 
-void HostCopy::reserve()
-{
-    if (prepare()) workers_.open();
-}
-
 // One copy by the runtime, which stages pageable memory itself.
 hipError_t HostCopy::plain(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s)
 {

@@ -47,10 +47,10 @@ struct State {
     std::vector<Copy> copies;
     int num_cus = 256;
     int captures = 0, replays = 0, threads = 0;
-    hipError_t last = hipSuccess;
 };
 inline State& state() { static State s; return s; }
-inline hipError_t note(hipError_t e) { if (e != hipSuccess) state().last = e; return e; }
+inline thread_local hipError_t last_error = hipSuccess;
+inline hipError_t note(hipError_t e) { if (e != hipSuccess) last_error = e; return e; }
 inline hipError_t take(std::map<const char*, size_t>& where, void** p, size_t bytes)
 {
     char* m = static_cast<char*>(std::calloc(std::max<size_t>(bytes, 1), 1));
@@ -128,7 +128,7 @@ inline hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMe
 }
 inline hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) { return hipMemcpyAsync(d, s, n, k, nullptr); }
 inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { std::memset(d, v, n); return hipSuccess; }
-inline hipError_t hipGetLastError() { auto& s = fake::state(); const hipError_t e = s.last; s.last = hipSuccess; return e; }
+inline hipError_t hipGetLastError() { const hipError_t e = fake::last_error; fake::last_error = hipSuccess; return e; }
 inline const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "invalid argument"; }
 inline hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }

@@ -3,6 +3,7 @@
 // launches replaced by what their kernels leave in memory.
 //   host_paths NAME   runs one check; prints what failed and returns 1
 #include <cstdio>
+#include <filesystem>
 
 #include "../../embree-benchmark-protoray_amd/csrc/api.hip"
 #include "../../embree-benchmark-protoray_amd/csrc/host_copy.hip"
@@ -259,6 +260,33 @@ void pinned_caller()
     }
 }
 
+int threads()
+{
+    int n = 0;
+    for (const auto& e : std::filesystem::directory_iterator("/proc/self/task")) n += e.exists();
+    return n;
+}
+
+// A context starts its copy threads with the first copy that needs them, and
+// ends them with itself.
+void copy_threads()
+{
+    const int before = threads();
+    {
+        Context c;
+        with_scene(c);
+        std::vector<prt_ray> rays(40000);
+        std::vector<prt_hit> hits(40000);
+        EXPECT(prt_hip_intersect_closest(c, rays.data(), hits.data(), 40000) == 0);
+        EXPECT(threads() == before);
+        EXPECT(prt_hip_frame_init(c, 1000, 1000) == 0);
+        std::vector<float> image(4000000);
+        EXPECT(prt_hip_accum_read(c, image.data()) == 0);
+        EXPECT(threads() > before);
+    }
+    EXPECT(threads() == before);
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -268,6 +296,7 @@ const struct {
     {"no_pinned_memory", no_pinned_memory},
     {"host_copies", host_copies},
     {"pinned_caller", pinned_caller},
+    {"copy_threads", copy_threads},
 };
 
 }  // namespace

@@ -27,6 +27,7 @@ def exe(tmp_path_factory):
     "no_pinned_memory",
     "host_copies",
     "pinned_caller",
+    "copy_threads",
 ])
 def test_host_path(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
