@@ -8,6 +8,7 @@
 
 #include "host_copy.h"
 #include "prt_math.h"
+#include "work_deal.h"
 #include "../../include/prt_hip.h"
 
 namespace prt {
@@ -293,10 +294,6 @@ namespace prt {
 int build_bvh8(prt_hip_ctx* ctx, SceneBuffers& sb, prt_build_stats* stats);
 
 // trace.hip
-// Work counters of a persistent launch: 16 of them, a 128 B line each.
-constexpr uint32_t kWorkCountersLg = 4;
-constexpr uint32_t kWorkCounterStride = 32;
-constexpr int kWorkWords = (int)kWorkCounterStride << kWorkCountersLg;
 struct TraceLaunch {
     const float4* rays;
     float4* hits;               // closest-hit records

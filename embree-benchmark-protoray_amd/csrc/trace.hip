@@ -55,8 +55,8 @@ namespace {
 constexpr int kStackLds = 16;      // default LDS entries per lane (power of two)
 constexpr int kRefill = 32;        // default: refill when this many lanes are idle
 // In launches of at least so many waves a wave stops when its own work counter
-// has run out: 64 waves serve each of the 16, the runs deal the work evenly, and
-// a look at all counters for items left queues up at their lines when all waves
+// has run out: 64 waves serve each of the 16, which hold about the same work
+// (work_deal.h), and a look at all counters for items left queues up at their lines when all waves
 // take it at the end.  With / without that look, us: closest hits 300 k 206 /
 // 186, 600 k 262 / 223, 1 M 432 / 398, any hit 500 k 214 / 177; Mrays/s of plain
 // frames 3270 / 3630, 2100 / 2270, 1390 / 1500, 2320 / 2500 (four scenes); 300 k
@@ -217,14 +217,17 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     // previous call suspended, level by level: queue l holds lk_res[l + 1] -
     // lk_res[l] of them from lk_res[l] on (they are part way through, so
     // they go last).
-    //  - A wave that has seen all of them handed out takes items of the
+    //  - A wave whose work counter has none of them left (in small launches:
+    //    no counter has) takes items of the
     //    later frames from LookState::spec_counter (level l: path S_l + j
     //    for the j-th item of its share), but only while it holds no path of
     //    this frame: waves that do take nothing more, stay sparse and issue
     //    first (s_setprio).
     //  - Every wave starts registered in LookState::live and leaves it once,
-    //    at that same point (all handed out, no level-0 path held); the last
-    //    to leave writes this call's tag into each block's stop flag.
+    //    at that same point (none left for it, no level-0 path held); every
+    //    counter has waves that stay until it has run out, so all are handed
+    //    out when the last leaves, which writes this call's tag into each
+    //    block's stop flag.
     //  - After the stop no more items are taken, and paths of later frames
     //    leave for the queue of their level: at a bounce, or in the middle
     //    of a ray, which the next call then traces again from its origin.
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         for (int l = 1; l <= kLookLevels + 1; ++l) lk_spec[l] = look->spec_begin[l];
     }
     bool stop = kLookMode && look && lk_target == 0;  // wave-uniform: this frame is finished
-    bool fresh_out = false;  // wave-uniform: every item of this frame's space is handed out
+    bool fresh_out = false;  // wave-uniform: this wave takes no more of this frame's space
     bool live = kLookMode && look;  // wave-uniform: registered in LookState::live
     int level = 0;           // the lane's path belongs to frame pass + level
     bool suspend = false;    // the lane's later-frame path waits in (o, d) for the queue
@@ -971,10 +974,10 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     };
 
     // ---- work items.  They are dealt in runs of 64 (spread: 8) to the
-    // counters, run r to counter r mod 16, and each wave starts with the run of
-    // its own number without asking.  It goes on with the counter of that run
-    // and, in launches of few waves, when that has run out with the next that has
-    // not (kOwnCounterWaves).
+    // counters (work_deal.h), and each wave starts with the run of its own number
+    // without asking.  It goes on with the counter of that run and, in launches
+    // of few waves, when that has run out with the next that has not
+    // (kOwnCounterWaves).
     // Measured: atomics on one line take 11.5 ns each, whoever asks, so one
     // counter spends 47 us on the first items of 4096 waves and 0.7 ms on a
     // frame of 2.07 M paths, taken 34 at a time; 16 lines take 0.9 ns each.
@@ -986,28 +989,28 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
     // a small launch is traced in groups from its start (wave-uniform)
     const bool spread = kCoop && pl.coop == kCoopSpread;
     const uint32_t run_lg = spread ? 3u : 6u;
-    constexpr uint32_t ctr_lg = kWorkCountersLg, ctr_last = (1u << ctr_lg) - 1u;
+    constexpr uint32_t ctr_last = kWorkCounterLast;
     const uint32_t items = kLookMode && look ? lk_fresh_end : count;
     const uint32_t n_waves = gridDim.x * (uint32_t)(kBlock / 64);
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t my_run = spread ? blockIdx.x + gridDim.x * wave : blockIdx.x * (uint32_t)(kBlock / 64) + wave;
-    uint32_t ctr = my_run & ctr_last;
+    uint32_t ctr = deal_counter(my_run);
     bool first_run = true, work_out = false;  // wave-uniform; work_out: all items are handed out
     // positions of counter c: the waves' first runs end at dealt(c, n_waves),
     // its items at dealt(c, runs of all items)
-    auto dealt = [&](uint32_t c, uint32_t runs) -> uint32_t { return ((runs + ctr_last - c) >> ctr_lg) << run_lg; };
+    auto dealt = [&](uint32_t c, uint32_t runs) -> uint32_t { return dealt_runs(c, runs) << run_lg; };
     const uint32_t n_runs = (items + (1u << run_lg) - 1u) >> run_lg;
     // Hands n items out to the lanes or groups that take part, numbered by
     // rank; false: none for this one.
     auto claim = [&](uint32_t n, uint32_t rank, uint32_t& my) -> bool {
-        uint32_t base = (my_run >> ctr_lg) << run_lg;
+        uint32_t base = (my_run >> kWorkCountersLg) << run_lg;
         const uint32_t end = dealt(ctr, n_runs);
         if (!first_run) {
             if (lane == 0) base = atomicAdd(work + ctr * kWorkCounterStride, n);
             base = dealt(ctr, n_waves) + (uint32_t)__builtin_amdgcn_readfirstlane((int)base);  // wave-uniform
         }
         const uint32_t at = base + rank;
-        my = ((((at >> run_lg) << ctr_lg) | ctr) << run_lg) | (at & ((1u << run_lg) - 1u));
+        my = (deal_run(ctr, at >> run_lg) << run_lg) | (at & ((1u << run_lg) - 1u));
         const bool ok = at < end && my < items;
         const bool ended = first_run ? dealt(ctr, n_waves) >= end : base + n >= end;
         if (n_waves >= n_runs || (ended && n_waves >= kOwnCounterWaves)) {

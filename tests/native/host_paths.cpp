@@ -287,6 +287,36 @@ void copy_threads()
     EXPECT(threads() == before);
 }
 
+// The deal of work items: each run belongs to one counter, in its order, and no
+// column of a frame's tiles leaves more than half of its runs to one counter.
+void work_deal()
+{
+    for (uint32_t runs : {0u, 1u, 15u, 16u, 17u, 31u, 33u, 255u, 4096u, 4097u, 70001u}) {
+        std::vector<uint32_t> next(16, 0);
+        for (uint32_t r = 0; r < runs; ++r) {
+            const uint32_t c = deal_counter(r);
+            EXPECT(c < 16 && deal_run(c, r >> 4) == r && next[c] == r >> 4);
+            EXPECT(dealt_runs(c, r) == next[c]);
+            ++next[c];
+        }
+        uint32_t all = 0;
+        for (uint32_t c = 0; c < 16; ++c) {
+            EXPECT(dealt_runs(c, runs) == next[c]);
+            all += dealt_runs(c, runs);
+        }
+        EXPECT(all == runs);
+    }
+    // the most runs of a launch: 2^32 - 2^20 items in runs of 64
+    for (uint32_t r : {67092479u, 67092478u, 67092464u, 67092463u}) EXPECT(deal_run(deal_counter(r), r >> 4) == r);
+    for (uint32_t tiles = 16; tiles <= 512; tiles += 16)
+        for (uint32_t rows : {16u, 64u, 135u})
+            for (uint32_t x = 0; x < tiles; ++x) {
+                std::vector<uint32_t> count(16, 0);
+                for (uint32_t y = 0; y < rows; ++y) ++count[deal_counter(y * tiles + x)];
+                EXPECT(*std::max_element(count.begin(), count.end()) <= (rows + 1) / 2);
+            }
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -297,6 +327,7 @@ const struct {
     {"host_copies", host_copies},
     {"pinned_caller", pinned_caller},
     {"copy_threads", copy_threads},
+    {"work_deal", work_deal},
 };
 
 }  // namespace

@@ -28,6 +28,7 @@ def exe(tmp_path_factory):
     "host_copies",
     "pinned_caller",
     "copy_threads",
+    "work_deal",
 ])
 def test_host_path(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
