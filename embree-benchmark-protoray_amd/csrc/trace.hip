@@ -153,6 +153,13 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
         __syncthreads();
     }
 
+    // A stack overflow.  A small query's flag is in pinned host memory, where the
+    // link may not carry an atomic OR; a query raises nothing else, so it stores.
+    auto raise_overflow = [&]() {
+        if constexpr (kRayQuery) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        else atomicOr(err, 1u);
+    };
+
     bool active = false;   // the lane holds a ray or path
     bool tracing = false;  // ... and is traversing (else its ray waits for shading)
     uint32_t ray_idx = 0;
@@ -952,7 +959,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
                         const int npush = __popc(pm) + 1;
                         bool room = true;
                         while (sp + npush - bottom > kGStack) {
-                            if (bottom >= spill_cap) { if (gj == 0) atomicOr(err, 1u); room = false; break; }
+                            if (bottom >= spill_cap) { if (gj == 0) raise_overflow(); room = false; break; }
                             const int bs = group_slot(bottom);
                             g_spill[bottom] = make_uint2(st_node[bs], __float_as_uint(st_t[bs]));
                             ++bottom;
@@ -1347,7 +1354,7 @@ __global__ __launch_bounds__(kBlock, kMode == kModeBatch || kMode == kModeAdjoin
                             // entries to the lane's global slice
                             bool ok = true;
                             while (sp + npush - bottom > kStack) {
-                                if (bottom >= spill_cap) { atomicOr(err, 1u); ok = false; break; }
+                                if (bottom >= spill_cap) { raise_overflow(); ok = false; break; }
                                 const uint32_t boff = ring_off(bottom);
                                 my_spill[bottom] = make_uint2(ring_node(boff), __float_as_uint(ring_t(boff)));
                                 ++bottom;
