@@ -688,6 +688,7 @@ int prt_hip_frame_init(prt_hip_ctx* ctx, int width, int height)
     free_ptr(ctx->d_bgr8);
     ctx->d_accum = nullptr;
     ctx->d_bgr8 = nullptr;
+    ctx->look_refused = false;
     ctx->width = width;
     ctx->height = height;
     PRT_TRY(ctx, hipMalloc(&ctx->d_accum, sizeof(float4) * (int64_t)width * height));
@@ -737,6 +738,7 @@ int prt_hip_set_lookahead(prt_hip_ctx* ctx, int enable)
     if (!ctx) return 1;
     ctx->lookahead = enable ? 1 : 0;
     ctx->look_prev_on = false;
+    ctx->look_refused = false;
     return 0;
 }
 
@@ -748,45 +750,62 @@ namespace {
 // one allocation, the state, the stop flags and, per level, two queues (read by
 // this call, written for the next) of one path per lane of the launch, item
 // uint4 each.
-int ensure_look_resources(prt_hip_ctx* ctx, uint32_t entries, int item)
+// False: no room for them, now and until the next frame_init or set_lookahead;
+// the frames render without the lookahead.
+bool ensure_look_resources(prt_hip_ctx* ctx, uint32_t entries, int item)
 {
+    if (ctx->look_refused) return false;
     const int64_t pixels = (int64_t)ctx->width * ctx->height;
     const int64_t side_len = pixels * kLookLevels;
     const uint32_t lanes = (uint32_t)diffuse_grid(ctx, entries) * (uint32_t)kTraceBlock;
     bool fresh = false;
+    hipError_t e = hipSuccess;
     if (side_len != ctx->look_side_len) {
         free_ptr(ctx->d_look_side);
         ctx->d_look_side = nullptr;
         ctx->look_side_len = 0;
-        PRT_TRY(ctx, hipMalloc(&ctx->d_look_side, sizeof(uint2) * side_len));
-        PRT_TRY(ctx, hipMemsetAsync(ctx->d_look_side, 0, sizeof(uint2) * side_len, ctx->stream));
+        e = hipMalloc(&ctx->d_look_side, sizeof(uint2) * side_len);
+        if (e == hipSuccess) e = hipMemsetAsync(ctx->d_look_side, 0, sizeof(uint2) * side_len, ctx->stream);
         ctx->look_side_len = side_len;
         fresh = true;
     }
     const uint64_t words = (uint64_t)lanes * (uint64_t)item;
-    if (words > ctx->look_q_words) {
+    if (e == hipSuccess && words > ctx->look_q_words) {
         free_ptr(ctx->d_look);
         ctx->d_look = nullptr;
         ctx->look_q_words = 0;
         constexpr size_t kStateBytes = (sizeof(LookState) + 255) & ~(size_t)255;
         const size_t flag_bytes = sizeof(uint32_t) * kLookFlagStride * (size_t)ctx->trace_grid;
         const size_t q_bytes = sizeof(uint4) * (size_t)words;
-        PRT_TRY(ctx, hipMalloc(&ctx->d_look, kStateBytes + flag_bytes + 2 * kLookLevels * q_bytes));
-        PRT_TRY(ctx, hipMemsetAsync(ctx->d_look, 0, kStateBytes + flag_bytes, ctx->stream));
-        char* at = reinterpret_cast<char*>(ctx->d_look) + kStateBytes;
-        ctx->d_look_flags = reinterpret_cast<uint32_t*>(at);
-        at += flag_bytes;
-        for (auto& level : ctx->d_look_q)
-            for (uint4*& q : level) {
-                q = reinterpret_cast<uint4*>(at);
-                at += q_bytes;
-            }
-        ctx->look_q_words = words;
+        e = hipMalloc(&ctx->d_look, kStateBytes + flag_bytes + 2 * kLookLevels * q_bytes);
+        if (e == hipSuccess) {
+            e = hipMemsetAsync(ctx->d_look, 0, kStateBytes + flag_bytes, ctx->stream);
+            char* at = reinterpret_cast<char*>(ctx->d_look) + kStateBytes;
+            ctx->d_look_flags = reinterpret_cast<uint32_t*>(at);
+            at += flag_bytes;
+            for (auto& level : ctx->d_look_q)
+                for (uint4*& q : level) {
+                    q = reinterpret_cast<uint4*>(at);
+                    at += q_bytes;
+                }
+            ctx->look_q_words = words;
+        }
         fresh = true;
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // the next launch would take it for its own
+        free_ptr(ctx->d_look_side);
+        free_ptr(ctx->d_look);
+        ctx->d_look_side = nullptr;
+        ctx->d_look = nullptr;
+        ctx->look_side_len = 0;
+        ctx->look_q_words = 0;
+        ctx->look_refused = true;
+        return false;
     }
     ctx->look_q_cap = (uint32_t)(ctx->look_q_words / (uint64_t)item);
     if (fresh) ctx->look_prev_spec = false;  // nothing the previous call left is kept
-    return 0;
+    return true;
 }
 
 // The first frame of a chain, from 0, that runs the lookahead.  That frame pays
@@ -870,9 +889,9 @@ int prt_hip_render(prt_hip_ctx* ctx, int renderer, int max_depth, float albedo, 
         std::memcpy(&key.albedo_bits, &albedo, sizeof(float));
     }
     const int chain = look_on && ctx->look_prev_on && look_follows(ctx->look_prev, key) ? ctx->look_chain + 1 : 0;
-    const bool look_run = look_on && chain >= look_from(renderer, entries);
     ctx->look_prev_on = false;  // set again once this call has succeeded
-    if (look_run && ensure_look_resources(ctx, entries, look_item(renderer))) return 1;
+    const bool look_run =
+        look_on && chain >= look_from(renderer, entries) && ensure_look_resources(ctx, entries, look_item(renderer));
     const bool look_valid = look_run && ctx->look_prev_spec;
 
     PRT_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));

@@ -265,6 +265,7 @@ struct prt_hip_ctx {
     uint32_t look_q_cap = 0;            // paths per queue in the current call
     uint32_t* d_look_flags = nullptr;   // one stop flag per block of the launch
     uint32_t look_gen = 0;
+    bool look_refused = false;          // no memory for the lookahead's buffers
     struct LookKey {
         uint64_t scene_gen;
         prt_camera cam;

@@ -21,6 +21,8 @@ int g_failed = 0;
     } while (0)
 
 int g_per_cu = 4;                 // workgroups per CU that fit
+prt::PathLaunch g_paths;          // the last path launch
+bool g_look_valid = false;        // ... and whether the lookahead kept earlier work for it
 
 // A ray's record: its own first origin coordinate, so that a test knows it.
 prt_hit answer(const float4& r0) { return prt_hit{r0.x, 7, 0.25f, 0.5f}; }
@@ -58,8 +60,16 @@ hipError_t launch_trace(prt_hip_ctx* ctx, const TraceLaunch& t, bool) { return q
 hipError_t launch_occluded(prt_hip_ctx* ctx, const TraceLaunch& t, bool) { return query(ctx, t, true); }
 hipError_t launch_trace_scratch(prt_hip_ctx*, const TraceLaunch&, uint2*, int, uint32_t*, int) { return hipSuccess; }
 hipError_t launch_zero_u32(uint32_t* p, int n, hipStream_t) { std::memset(p, 0, 4 * (size_t)n); return hipSuccess; }
-hipError_t launch_paths(prt_hip_ctx*, const PathLaunch&, int, bool) { return hipSuccess; }
-hipError_t launch_look_call_begin(prt_hip_ctx*, bool, uint32_t) { return hipSuccess; }
+hipError_t launch_paths(prt_hip_ctx*, const PathLaunch& p, int, bool)
+{
+    g_paths = p;
+    return hipGetLastError();
+}
+hipError_t launch_look_call_begin(prt_hip_ctx*, bool valid, uint32_t)
+{
+    g_look_valid = valid;
+    return hipGetLastError();
+}
 hipError_t launch_paths_rgb(prt_hip_ctx*, const PathLaunch&, bool) { return hipSuccess; }
 hipError_t launch_adjoint(prt_hip_ctx*, const PathLaunch&, bool) { return hipSuccess; }
 const BatchKernelConfig kBatchVariants[kBatchVariantCount] = {{256, 16}, {256, 8}, {128, 16}, {128, 8}};
@@ -317,6 +327,34 @@ void work_deal()
             }
 }
 
+// Frames render where the lookahead's buffers find no room, and with it again
+// once there is.
+void no_room_for_the_lookahead()
+{
+    for (int renderer : {PRT_RENDERER_DIFFUSE, PRT_RENDERER_DIFFUSE2})
+        for (size_t room : {(size_t)0, (size_t)1 << 20, (size_t)10 << 20}) {  // none, ..., the side samples alone
+            Context c;
+            with_scene(c);
+            prt_camera cam{};
+            cam.focal_distance = 1.0f;
+            EXPECT(prt_hip_camera_set(c, &cam) == 0);
+            EXPECT(prt_hip_frame_init(c, 717, 405) == 0);
+            fake::state().device_limit = fake::state().device_bytes + room;
+            for (int k = 0; k < 6; ++k) {
+                EXPECT(prt_hip_render(c, renderer, 6, 0.8f, nullptr) == 0);
+                EXPECT(g_paths.look == nullptr);
+            }
+            fake::state().device_limit = ~size_t(0);
+            EXPECT(prt_hip_set_lookahead(c, 1) == 0);
+            int runs = 0;
+            for (int k = 0; k < 6; ++k) {
+                EXPECT(prt_hip_render(c, renderer, 6, 0.8f, nullptr) == 0);
+                if (g_paths.look) EXPECT(g_look_valid == (runs++ > 0));
+            }
+            EXPECT(runs >= 3);
+        }
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -328,6 +366,7 @@ const struct {
     {"pinned_caller", pinned_caller},
     {"copy_threads", copy_threads},
     {"work_deal", work_deal},
+    {"no_room_for_the_lookahead", no_room_for_the_lookahead},
 };
 
 }  // namespace
