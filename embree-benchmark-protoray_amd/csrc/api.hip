@@ -117,19 +117,48 @@ void free_ptr(void* p)
     if (p) (void)hipFree(p);
 }
 
-// Room for `count` elements (at least one) in a buffer that has room for cap of
-// them: kept if it is large enough and not over four times too large, else
-// replaced.
+// A buffer that outlives its contents, with room for cap elements.
 template <class T>
-int ensure_room(prt_hip_ctx* ctx, T*& p, int64_t& cap, int64_t count)
+struct Kept {
+    T*& p;
+    int64_t& cap;
+    int64_t count;  // elements needed; room for at least 16 is laid out
+    void drop()
+    {
+        free_ptr(p);
+        p = nullptr;
+        cap = 0;
+    }
+    // kept if it is large enough and not over four times too large
+    void drop_unless_fit()
+    {
+        if (!p || room() > cap || cap > std::max<int64_t>(4 * room(), 1 << 20)) drop();
+    }
+    int64_t room() const { return std::max<int64_t>(count, 16); }
+    hipError_t ensure()
+    {
+        if (p) return hipSuccess;
+        const hipError_t e = hipMalloc(&p, sizeof(T) * (size_t)room());
+        if (e == hipSuccess) cap = room();
+        else p = nullptr;
+        return e;
+    }
+};
+
+// Room in two buffers that are filled together.  What does not fit is freed
+// before the first is allocated, and what is larger than needed where there is
+// no room otherwise, so that neither stands in the other's room.
+template <class A, class B>
+int ensure_room(prt_hip_ctx* ctx, Kept<A> a, Kept<B> b)
 {
-    count = std::max<int64_t>(count, 16);
-    if (p && count <= cap && cap <= std::max<int64_t>(4 * count, 1 << 20)) return 0;
-    free_ptr(p);
-    p = nullptr;
-    cap = 0;
-    PRT_TRY(ctx, hipMalloc(&p, sizeof(T) * (size_t)count));
-    cap = count;
+    a.drop_unless_fit();
+    b.drop_unless_fit();
+    if (a.ensure() == hipSuccess && b.ensure() == hipSuccess) return 0;
+    (void)hipGetLastError();  // the next launch would take it for its own
+    a.drop();
+    b.drop();
+    PRT_TRY(ctx, a.ensure());
+    PRT_TRY(ctx, b.ensure());
     return 0;
 }
 
@@ -464,17 +493,19 @@ int prt_hip_scene_upload(prt_hip_ctx* ctx, const int32_t* idx3, int64_t tri_coun
     sc.d_normals = nullptr;
     sc.d_texcoords = nullptr;
     sc.bvh_ready = false;
-    sc.tri_count = tri_count;
-    sc.vertex_count = vertex_count;
+    sc.tri_count = sc.vertex_count = 0;  // until all of the scene is there
     free_ptr(ctx->d_albedo_own);
     ctx->d_albedo_own = nullptr;
     ctx->d_albedo = nullptr;
-    if (ensure_room(ctx, sc.d_idx, sc.idx_cap, 3 * tri_count) || ensure_room(ctx, sc.d_pos, sc.pos_cap, 3 * vertex_count))
+    if (ensure_room(ctx, Kept<int32_t>{sc.d_idx, sc.idx_cap, 3 * tri_count},
+                    Kept<float>{sc.d_pos, sc.pos_cap, 3 * vertex_count}))
         return 1;
     if (tri_count) {
         PRT_TRY(ctx, ctx->copy.to_device(sc.d_idx, idx3, 12 * tri_count, ctx->stream));
         PRT_TRY(ctx, ctx->copy.to_device(sc.d_pos, pos3, 12 * vertex_count, ctx->stream));
     }
+    sc.tri_count = tri_count;
+    sc.vertex_count = vertex_count;
     return 0;
 }
 
@@ -1252,14 +1283,9 @@ int prt_hip_batch_set_jobs(prt_hip_ctx* ctx, const prt_batch_job* jobs, int n_jo
     ctx->d_batch_jobs = reinterpret_cast<BatchJobDevice*>(d_tables);
     ctx->d_batch_work_begin = reinterpret_cast<uint32_t*>(d_tables + at_work);
     ctx->d_batch_pixel_begin = reinterpret_cast<uint64_t*>(d_tables + at_pixel);
-    int64_t cap = (int64_t)ctx->batch_samples_cap;
-    int rc = ensure_room(ctx, ctx->d_batch_samples, cap, (int64_t)samples);
-    ctx->batch_samples_cap = (uint64_t)cap;
-    if (rc) return rc;
-    cap = (int64_t)ctx->batch_accum_cap;
-    rc = ensure_room(ctx, ctx->d_batch_accum, cap, (int64_t)pixels);
-    ctx->batch_accum_cap = (uint64_t)cap;
-    if (rc) return rc;
+    if (ensure_room(ctx, Kept<float>{ctx->d_batch_samples, ctx->batch_samples_cap, (int64_t)samples},
+                    Kept<float4>{ctx->d_batch_accum, ctx->batch_accum_cap, (int64_t)pixels}))
+        return 1;
     PRT_TRY(ctx, hipMemsetAsync(ctx->d_batch_accum, 0, sizeof(float4) * pixels, ctx->stream));
     PRT_TRY(ctx, ctx->copy.to_device(d_tables, tables.data(), tables.size(), ctx->stream));
     ctx->batch_rendered = false;

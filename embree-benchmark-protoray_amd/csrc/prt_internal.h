@@ -194,7 +194,7 @@ struct prt_hip_ctx {
     float* d_batch_samples = nullptr;
     float4* d_batch_accum = nullptr;
     uint64_t batch_samples_len = 0, batch_pixels = 0;
-    uint64_t batch_samples_cap = 0, batch_accum_cap = 0;  // room of the two buffers above
+    int64_t batch_samples_cap = 0, batch_accum_cap = 0;  // room of the two buffers above
     uint32_t batch_total_work = 0;
     prt::BatchTuning batch_tuning;
     hipGraph_t batch_graph = nullptr;

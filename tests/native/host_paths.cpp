@@ -355,6 +355,45 @@ void no_room_for_the_lookahead()
         }
 }
 
+// Memory that a job set or a scene needs and the one before it gives up is there
+// for it: a device that holds either holds one after the other.
+void replaced_buffers()
+{
+    Context c;
+    int scene = -1;
+    EXPECT(prt_hip_batch_scene_add(c, kIdx, 1, kPos, 3, nullptr, &scene) == 0);
+    prt_batch_job wide{}, deep{};
+    wide.camera.focal_distance = deep.camera.focal_distance = 1.0f;
+    wide.scene = deep.scene = scene;
+    wide.width = wide.height = 2048;   // 67 MB of accumulators, 17 MB of samples
+    wide.spp = 1;
+    deep.width = deep.height = 1024;   // 17 and 67
+    deep.spp = 16;
+    const size_t before = fake::state().device_bytes;
+    fake::state().device_limit = before + ((size_t)90 << 20);
+    for (int k = 0; k < 4; ++k) {
+        const bool ok = prt_hip_batch_set_jobs(c, k & 1 ? &deep : &wide, 1) == 0;
+        if (!ok) std::printf("set %d: %s\n", k, prt_hip_last_error(c));
+        EXPECT(ok);
+    }
+    fake::state().device_limit = ~size_t(0);
+    EXPECT(prt_hip_batch_reset(c) == 0);
+
+    // 1 M triangles of 4 vertices, then 40 k of 3 M vertices, in turn
+    std::vector<int32_t> idx(3000000, 1);
+    std::vector<float> pos(9000000, 0.5f);
+    fake::state().device_limit = fake::state().device_bytes + ((size_t)40 << 20);
+    for (int k = 0; k < 4; ++k) {
+        EXPECT(prt_hip_scene_upload(c, idx.data(), k & 1 ? 40000 : 1000000, pos.data(), k & 1 ? 3000000 : 4) == 0);
+        EXPECT(prt_hip_bvh_build(c, nullptr) == 0);
+    }
+    // a scene that finds no room leaves none behind
+    fake::state().device_limit = fake::state().device_bytes;
+    EXPECT(prt_hip_scene_upload(c, idx.data(), 1000000, pos.data(), 3000000) != 0);
+    EXPECT(c.ctx->scene.tri_count == 0);
+    fake::state().device_limit = ~size_t(0);
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -367,6 +406,7 @@ const struct {
     {"copy_threads", copy_threads},
     {"work_deal", work_deal},
     {"no_room_for_the_lookahead", no_room_for_the_lookahead},
+    {"replaced_buffers", replaced_buffers},
 };
 
 }  // namespace

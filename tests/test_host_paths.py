@@ -30,6 +30,7 @@ def exe(tmp_path_factory):
     "copy_threads",
     "work_deal",
     "no_room_for_the_lookahead",
+    "replaced_buffers",
 ])
 def test_host_path(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
