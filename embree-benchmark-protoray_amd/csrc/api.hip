@@ -59,6 +59,43 @@ int check_hip(prt_hip_ctx* ctx, hipError_t e, const char* what)
     return set_error(ctx, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+static void drop_look_buffers(prt_hip_ctx* ctx)
+{
+    if (ctx->d_look_side) (void)hipFree(ctx->d_look_side);
+    if (ctx->d_look) (void)hipFree(ctx->d_look);
+    ctx->d_look_side = nullptr;
+    ctx->d_look = nullptr;
+    ctx->look_side_len = 0;
+    ctx->look_q_words = 0;
+    ctx->look_prev_spec = false;  // what the previous call left is gone
+}
+
+static void drop_scratch(prt_hip_ctx* ctx)
+{
+    if (ctx->d_build) (void)hipFree(ctx->d_build);
+    if (ctx->d_path_hits) (void)hipFree(ctx->d_path_hits);
+    ctx->d_build = nullptr;
+    ctx->d_path_hits = nullptr;
+    ctx->build_bytes = 0;
+    ctx->path_hits_cap = 0;
+}
+
+hipError_t device_alloc_bytes(prt_hip_ctx* ctx, void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    // no kernel that uses these runs past its call
+    drop_look_buffers(ctx);
+    drop_scratch(ctx);
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 }  // namespace prt
 
 using namespace prt;
@@ -135,12 +172,11 @@ struct Kept {
         if (!p || room() > cap || cap > std::max<int64_t>(4 * room(), 1 << 20)) drop();
     }
     int64_t room() const { return std::max<int64_t>(count, 16); }
-    hipError_t ensure()
+    hipError_t ensure(prt_hip_ctx* ctx)
     {
         if (p) return hipSuccess;
-        const hipError_t e = hipMalloc(&p, sizeof(T) * (size_t)room());
+        const hipError_t e = device_alloc(ctx, &p, sizeof(T) * (size_t)room());
         if (e == hipSuccess) cap = room();
-        else p = nullptr;
         return e;
     }
 };
@@ -153,12 +189,11 @@ int ensure_room(prt_hip_ctx* ctx, Kept<A> a, Kept<B> b)
 {
     a.drop_unless_fit();
     b.drop_unless_fit();
-    if (a.ensure() == hipSuccess && b.ensure() == hipSuccess) return 0;
-    (void)hipGetLastError();  // the next launch would take it for its own
+    if (a.ensure(ctx) == hipSuccess && b.ensure(ctx) == hipSuccess) return 0;
     a.drop();
     b.drop();
-    PRT_TRY(ctx, a.ensure());
-    PRT_TRY(ctx, b.ensure());
+    PRT_TRY(ctx, a.ensure(ctx));
+    PRT_TRY(ctx, b.ensure(ctx));
     return 0;
 }
 
@@ -198,11 +233,11 @@ int set_attributes(prt_hip_ctx* ctx, SceneBuffers& sb, const float* normals3, co
     sb.d_texcoords = nullptr;
     const int64_t nv = sb.vertex_count;
     if (normals3 && nv > 0) {
-        PRT_TRY(ctx, hipMalloc(&sb.d_normals, 12 * nv));
+        PRT_TRY(ctx, device_alloc(ctx, &sb.d_normals, 12 * nv));
         PRT_TRY(ctx, ctx->copy.to_device(sb.d_normals, normals3, 12 * nv, ctx->stream));
     }
     if (texcoords2 && nv > 0) {
-        PRT_TRY(ctx, hipMalloc(&sb.d_texcoords, 8 * nv));
+        PRT_TRY(ctx, device_alloc(ctx, &sb.d_texcoords, 8 * nv));
         PRT_TRY(ctx, ctx->copy.to_device(sb.d_texcoords, texcoords2, 8 * nv, ctx->stream));
     }
     PRT_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -224,11 +259,11 @@ int ensure_queues(prt_hip_ctx* ctx, int64_t entries)
     ctx->d_hits = nullptr;
     ctx->queue_cap = 0;
     for (int b = 0; b < 2; ++b) {
-        PRT_TRY(ctx, hipMalloc(&ctx->d_rays[b], sizeof(float4) * 2 * entries));
-        PRT_TRY(ctx, hipMalloc(&ctx->d_pix[b], sizeof(int32_t) * entries));
-        PRT_TRY(ctx, hipMalloc(&ctx->d_rng[b], sizeof(uint32_t) * entries));
+        PRT_TRY(ctx, device_alloc(ctx, &ctx->d_rays[b], sizeof(float4) * 2 * entries));
+        PRT_TRY(ctx, device_alloc(ctx, &ctx->d_pix[b], sizeof(int32_t) * entries));
+        PRT_TRY(ctx, device_alloc(ctx, &ctx->d_rng[b], sizeof(uint32_t) * entries));
     }
-    PRT_TRY(ctx, hipMalloc(&ctx->d_hits, sizeof(float4) * entries));
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_hits, sizeof(float4) * entries));
     ctx->queue_cap = entries;
     return 0;
 }
@@ -274,8 +309,8 @@ int ensure_io(prt_hip_ctx* ctx, int64_t n)
     ctx->d_io_rays = nullptr;
     ctx->d_io_hits = nullptr;
     ctx->io_cap = 0;
-    PRT_TRY(ctx, hipMalloc(&ctx->d_io_rays, sizeof(prt_ray) * n));
-    PRT_TRY(ctx, hipMalloc(&ctx->d_io_hits, sizeof(prt_hit) * n));
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_io_rays, sizeof(prt_ray) * n));
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_io_hits, sizeof(prt_hit) * n));
     ctx->io_cap = n;
     return 0;
 }
@@ -722,8 +757,8 @@ int prt_hip_frame_init(prt_hip_ctx* ctx, int width, int height)
     ctx->look_refused = false;
     ctx->width = width;
     ctx->height = height;
-    PRT_TRY(ctx, hipMalloc(&ctx->d_accum, sizeof(float4) * (int64_t)width * height));
-    PRT_TRY(ctx, hipMalloc(&ctx->d_bgr8, sizeof(int32_t) * (int64_t)width * height));
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_accum, sizeof(float4) * (int64_t)width * height));
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_bgr8, sizeof(int32_t) * (int64_t)width * height));
     if (ensure_queues(ctx, frame_entries(ctx))) return 1;
     return prt_hip_frame_clear(ctx);
 }
@@ -790,12 +825,19 @@ bool ensure_look_resources(prt_hip_ctx* ctx, uint32_t entries, int item)
     const int64_t side_len = pixels * kLookLevels;
     const uint32_t lanes = (uint32_t)diffuse_grid(ctx, entries) * (uint32_t)kTraceBlock;
     bool fresh = false;
+    // the scratch of builds and of the adjoint gives way, these buffers not to each other
+    auto alloc = [&](void** p, size_t bytes) {
+        if (hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
+        (void)hipGetLastError();  // the next launch would take it for its own
+        drop_scratch(ctx);
+        return hipMalloc(p, bytes);
+    };
     hipError_t e = hipSuccess;
     if (side_len != ctx->look_side_len) {
         free_ptr(ctx->d_look_side);
         ctx->d_look_side = nullptr;
         ctx->look_side_len = 0;
-        e = hipMalloc(&ctx->d_look_side, sizeof(uint2) * side_len);
+        e = alloc(reinterpret_cast<void**>(&ctx->d_look_side), sizeof(uint2) * side_len);
         if (e == hipSuccess) e = hipMemsetAsync(ctx->d_look_side, 0, sizeof(uint2) * side_len, ctx->stream);
         ctx->look_side_len = side_len;
         fresh = true;
@@ -808,7 +850,7 @@ bool ensure_look_resources(prt_hip_ctx* ctx, uint32_t entries, int item)
         constexpr size_t kStateBytes = (sizeof(LookState) + 255) & ~(size_t)255;
         const size_t flag_bytes = sizeof(uint32_t) * kLookFlagStride * (size_t)ctx->trace_grid;
         const size_t q_bytes = sizeof(uint4) * (size_t)words;
-        e = hipMalloc(&ctx->d_look, kStateBytes + flag_bytes + 2 * kLookLevels * q_bytes);
+        e = alloc(reinterpret_cast<void**>(&ctx->d_look), kStateBytes + flag_bytes + 2 * kLookLevels * q_bytes);
         if (e == hipSuccess) {
             e = hipMemsetAsync(ctx->d_look, 0, kStateBytes + flag_bytes, ctx->stream);
             char* at = reinterpret_cast<char*>(ctx->d_look) + kStateBytes;
@@ -824,13 +866,8 @@ bool ensure_look_resources(prt_hip_ctx* ctx, uint32_t entries, int item)
         fresh = true;
     }
     if (e != hipSuccess) {
-        (void)hipGetLastError();  // the next launch would take it for its own
-        free_ptr(ctx->d_look_side);
-        free_ptr(ctx->d_look);
-        ctx->d_look_side = nullptr;
-        ctx->d_look = nullptr;
-        ctx->look_side_len = 0;
-        ctx->look_q_words = 0;
+        (void)hipGetLastError();
+        drop_look_buffers(ctx);
         ctx->look_refused = true;
         return false;
     }
@@ -1174,8 +1211,8 @@ int prt_hip_batch_scene_add(prt_hip_ctx* ctx, const int32_t* idx3, int64_t tri_c
     SceneBuffers sb;
     sb.tri_count = tri_count;
     sb.vertex_count = vertex_count;
-    hipError_t e = hipMalloc(&sb.d_idx, 12 * tri_count);
-    if (e == hipSuccess) e = hipMalloc(&sb.d_pos, 12 * vertex_count);
+    hipError_t e = device_alloc(ctx, &sb.d_idx, 12 * tri_count);
+    if (e == hipSuccess) e = device_alloc(ctx, &sb.d_pos, 12 * vertex_count);
     if (e == hipSuccess) e = ctx->copy.to_device(sb.d_idx, idx3, 12 * tri_count, ctx->stream);
     if (e == hipSuccess) e = ctx->copy.to_device(sb.d_pos, pos3, 12 * vertex_count, ctx->stream);
     if (e != hipSuccess) {
@@ -1192,7 +1229,7 @@ int prt_hip_batch_scene_add(prt_hip_ctx* ctx, const int32_t* idx3, int64_t tri_c
     ctx->d_batch_scenes = nullptr;
     std::vector<SceneDevice> table;
     for (const SceneBuffers& b : ctx->batch_scenes) table.push_back(b.device());
-    PRT_TRY(ctx, hipMalloc(&ctx->d_batch_scenes, sizeof(SceneDevice) * table.size()));
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_batch_scenes, sizeof(SceneDevice) * table.size()));
     PRT_TRY(ctx, hipMemcpy(ctx->d_batch_scenes, table.data(), sizeof(SceneDevice) * table.size(),
                            hipMemcpyHostToDevice));
     *out_scene = (int32_t)ctx->batch_scenes.size() - 1;
@@ -1279,7 +1316,7 @@ int prt_hip_batch_set_jobs(prt_hip_ctx* ctx, const prt_batch_job* jobs, int n_jo
     std::memcpy(tables.data() + at_work, work_begin.data(), sizeof(uint32_t) * (n_jobs + 1));
     std::memcpy(tables.data() + at_pixel, pixel_begin.data(), sizeof(uint64_t) * (n_jobs + 1));
     char* d_tables = nullptr;
-    PRT_TRY(ctx, hipMalloc(&d_tables, tables.size()));
+    PRT_TRY(ctx, device_alloc(ctx, &d_tables, tables.size()));
     ctx->d_batch_jobs = reinterpret_cast<BatchJobDevice*>(d_tables);
     ctx->d_batch_work_begin = reinterpret_cast<uint32_t*>(d_tables + at_work);
     ctx->d_batch_pixel_begin = reinterpret_cast<uint64_t*>(d_tables + at_pixel);
@@ -1526,7 +1563,7 @@ int prt_hip_set_albedo_host(prt_hip_ctx* ctx, const float* rgb)
     if (!rgb || ctx->scene.tri_count <= 0) return set_error(ctx, "set_albedo: no scene or null array");
     free_ptr(ctx->d_albedo_own);
     ctx->d_albedo_own = nullptr;
-    PRT_TRY(ctx, hipMalloc(&ctx->d_albedo_own, sizeof(float) * 3 * ctx->scene.tri_count));
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_albedo_own, sizeof(float) * 3 * ctx->scene.tri_count));
     PRT_TRY(ctx, ctx->copy.to_device(ctx->d_albedo_own, rgb, sizeof(float) * 3 * ctx->scene.tri_count, ctx->stream));
     ctx->d_albedo = ctx->d_albedo_own;
     return 0;
@@ -1559,7 +1596,7 @@ int prt_hip_render_albedo_image(prt_hip_ctx* ctx, int pass0, int spp, int max_de
         free_ptr(ctx->d_rgb_planes);
         ctx->d_rgb_planes = nullptr;
         ctx->rgb_planes_cap = 0;
-        PRT_TRY(ctx, hipMalloc(&ctx->d_rgb_planes, (size_t)chunk * plane_bytes));
+        PRT_TRY(ctx, device_alloc(ctx, &ctx->d_rgb_planes, (size_t)chunk * plane_bytes));
         ctx->rgb_planes_cap = (int64_t)chunk * pixels;
     }
     PRT_TRY(ctx, hipMemsetAsync(ctx->d_accum, 0, sizeof(float4) * pixels, ctx->stream));
@@ -1586,7 +1623,7 @@ int prt_hip_render_albedo_image_host(prt_hip_ctx* ctx, int pass0, int spp, int m
     if (!image) return set_error(ctx, "render_albedo_image: null image");
     const int64_t n = (int64_t)ctx->width * ctx->height * 3;
     float* d = nullptr;
-    PRT_TRY(ctx, hipMalloc(&d, sizeof(float) * n));
+    PRT_TRY(ctx, device_alloc(ctx, &d, sizeof(float) * n));
     int rc = prt_hip_render_albedo_image(ctx, pass0, spp, max_depth, d, out);
     if (rc == 0) {
         hipError_t e = ctx->copy.to_host(image, d, sizeof(float) * n, ctx->stream);
@@ -1641,8 +1678,8 @@ int prt_hip_adjoint_albedo_host(prt_hip_ctx* ctx, int pass0, int spp, int max_de
     if (!dldi || !grad) return set_error(ctx, "adjoint_albedo: null array");
     const int64_t ni = (int64_t)ctx->width * ctx->height * 3, ng = ctx->scene.tri_count * 3;
     float *di = nullptr, *dg = nullptr;
-    hipError_t e = hipMalloc(&di, sizeof(float) * ni);
-    if (e == hipSuccess) e = hipMalloc(&dg, sizeof(float) * ng);
+    hipError_t e = device_alloc(ctx, &di, sizeof(float) * ni);
+    if (e == hipSuccess) e = device_alloc(ctx, &dg, sizeof(float) * ng);
     if (e == hipSuccess) e = ctx->copy.to_device(di, dldi, sizeof(float) * ni, ctx->stream);
     if (e == hipSuccess) e = ctx->copy.to_device(dg, grad, sizeof(float) * ng, ctx->stream);
     int rc = e == hipSuccess ? prt_hip_adjoint_albedo(ctx, pass0, spp, max_depth, di, dg, out)
@@ -1683,8 +1720,8 @@ int prt_hip_debug_raygen(prt_hip_ctx* ctx, int pass, prt_ray* rays, uint32_t* st
     PRT_TRY(ctx, launch_raygen(ctx, pass, ctx->d_rays[0], ctx->d_pix[0], ctx->d_rng[0]));
     prt_ray* d_out = nullptr;
     uint32_t* d_states = nullptr;
-    PRT_TRY(ctx, hipMalloc(&d_out, sizeof(prt_ray) * np));
-    PRT_TRY(ctx, hipMalloc(&d_states, sizeof(uint32_t) * np));
+    PRT_TRY(ctx, device_alloc(ctx, &d_out, sizeof(prt_ray) * np));
+    PRT_TRY(ctx, device_alloc(ctx, &d_states, sizeof(uint32_t) * np));
     hipError_t e = launch_unpack_rays(ctx->d_rays[0], ctx->d_pix[0], ctx->d_rng[0], n, ctx->width,
                                       ctx->height, d_out, d_states, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(rays, d_out, sizeof(prt_ray) * np, hipMemcpyDeviceToHost, ctx->stream);

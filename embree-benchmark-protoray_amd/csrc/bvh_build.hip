@@ -1067,9 +1067,9 @@ int build_bvh8(prt_hip_ctx* ctx, SceneBuffers& sb, prt_build_stats* stats)
         sb.d_tris = nullptr;
         sb.d_prim_ids = nullptr;
         sb.bvh_cap = 0;
-        PRT_TRY(ctx, hipMalloc(&sb.d_nodes, sizeof(Bvh8Node) * max_nodes));
-        PRT_TRY(ctx, hipMalloc(&sb.d_tris, sizeof(float) * 9 * n));
-        PRT_TRY(ctx, hipMalloc(&sb.d_prim_ids, sizeof(int32_t) * n));
+        PRT_TRY(ctx, device_alloc(ctx, &sb.d_nodes, sizeof(Bvh8Node) * max_nodes));
+        PRT_TRY(ctx, device_alloc(ctx, &sb.d_tris, sizeof(float) * 9 * n));
+        PRT_TRY(ctx, device_alloc(ctx, &sb.d_prim_ids, sizeof(int32_t) * n));
         sb.bvh_cap = n;
     }
 
@@ -1080,7 +1080,7 @@ int build_bvh8(prt_hip_ctx* ctx, SceneBuffers& sb, prt_build_stats* stats)
         if (ctx->d_build) (void)hipFree(ctx->d_build);
         ctx->d_build = nullptr;
         ctx->build_bytes = 0;
-        PRT_TRY(ctx, hipMalloc(&ctx->d_build, arena.used));
+        PRT_TRY(ctx, device_alloc(ctx, &ctx->d_build, arena.used));
         ctx->build_bytes = arena.used;
     }
     arena = Arena{static_cast<char*>(ctx->d_build), 0};

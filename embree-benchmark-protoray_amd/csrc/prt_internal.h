@@ -424,6 +424,20 @@ hipError_t launch_unpack_rays(const float4* rays, const int32_t* pix, const uint
 int set_error(prt_hip_ctx* ctx, const std::string& msg);
 int check_hip(prt_hip_ctx* ctx, hipError_t e, const char* what);
 
+// Device memory.  Where there is no room, the context gives back what it keeps
+// between calls but could lay out again (build scratch, the adjoint's hit record,
+// the lookahead's buffers), and it is tried once more.  A failure is only
+// returned: it is not left behind for the next launch's check.
+hipError_t device_alloc_bytes(prt_hip_ctx* ctx, void** p, size_t bytes);
+template <class T>
+hipError_t device_alloc(prt_hip_ctx* ctx, T** p, size_t bytes)
+{
+    void* m = nullptr;
+    const hipError_t e = device_alloc_bytes(ctx, &m, bytes);
+    *p = static_cast<T*>(m);
+    return e;
+}
+
 }  // namespace prt
 
 #define PRT_TRY(ctx, expr)                                              \

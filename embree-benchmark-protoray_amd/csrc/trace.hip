@@ -1679,7 +1679,7 @@ int ensure_trace_resources(prt_hip_ctx* ctx)
         if (ctx->d_spill) { (void)hipFree(ctx->d_spill); ctx->d_spill = nullptr; }
         ctx->spill_bytes = 0;
         ctx->stack_entries = 0;
-        PRT_TRY(ctx, hipMalloc(&ctx->d_spill, bytes));
+        PRT_TRY(ctx, device_alloc(ctx, &ctx->d_spill, bytes));
         ctx->spill_bytes = bytes;
         ctx->stack_entries = need;
     }

@@ -4,6 +4,7 @@
 //   host_paths NAME   runs one check; prints what failed and returns 1
 #include <cstdio>
 #include <filesystem>
+#include <functional>
 
 #include "../../embree-benchmark-protoray_amd/csrc/api.hip"
 #include "../../embree-benchmark-protoray_amd/csrc/host_copy.hip"
@@ -394,6 +395,85 @@ void replaced_buffers()
     fake::state().device_limit = ~size_t(0);
 }
 
+// What a context keeps between calls (build scratch, the adjoint's hit record,
+// the lookahead's buffers) gives way to an allocation that finds no room.
+void kept_memory()
+{
+    constexpr size_t kMb = (size_t)1 << 20;
+    Context c;
+    with_scene(c);
+    prt_camera cam{};
+    cam.focal_distance = 1.0f;
+    EXPECT(prt_hip_camera_set(c, &cam) == 0);
+    int scene = -1;
+    EXPECT(prt_hip_batch_scene_add(c, kIdx, 1, kPos, 3, nullptr, &scene) == 0);
+    std::vector<float> values(9000000, 0.5f), image(3 * 512 * 512);
+    std::vector<int32_t> idx(3000000, 1);
+    std::vector<prt_ray> rays(1000000);
+    std::vector<prt_hit> hits(1000000);
+    prt_batch_job job{};
+    job.camera.focal_distance = 1.0f;
+    job.scene = scene;
+    job.width = job.height = 1024;
+    job.spp = 8;
+    const std::function<int()> calls[] = {
+        [&] { return prt_hip_frame_init(c, 1024, 1024); },
+        [&] { return prt_hip_intersect_closest(c, rays.data(), hits.data(), 1000000); },
+        [&] { return prt_hip_batch_set_jobs(c, &job, 1); },
+        [&] { return prt_hip_batch_scene_add(c, idx.data(), 1000000, values.data(), 3000000, nullptr, &scene); },
+        [&] { return prt_hip_scene_upload(c, idx.data(), 1000000, values.data(), 3000000); },
+        [&] { return prt_hip_scene_attributes(c, values.data(), values.data()); },
+        [&] { return prt_hip_set_albedo_host(c, values.data()); },
+        [&] { return prt_hip_bvh_build(c, nullptr) || prt_hip_render_albedo_image_host(c, 0, 16, 6, image.data(), nullptr); },
+        [&] { return prt_hip_adjoint_albedo_host(c, 0, 1, 65, image.data(), values.data(), nullptr); },
+    };
+    for (const auto& call : calls) {
+        auto room = [&](int64_t left) {   // a device with so much left, and all kept memory laid out
+            fake::state().device_limit = ~size_t(0);
+            EXPECT(prt_hip_bvh_build(c, nullptr) == 0);
+            std::vector<float> rgb(3 * (size_t)c.ctx->scene.tri_count, 0.5f), image(3 * 512 * 512);
+            EXPECT(prt_hip_set_albedo_host(c, rgb.data()) == 0);
+            if (c.ctx->width != 512) EXPECT(prt_hip_frame_init(c, 512, 512) == 0);
+            EXPECT(prt_hip_frame_clear(c) == 0);
+            for (int k = 0; k < 6; ++k) EXPECT(prt_hip_render(c, PRT_RENDERER_DIFFUSE2, 6, 0.8f, nullptr) == 0);
+            EXPECT(g_paths.look != nullptr);
+            EXPECT(prt_hip_adjoint_albedo_host(c, 0, 1, 6, image.data(), rgb.data(), nullptr) == 0);
+            EXPECT(c.ctx->d_path_hits != nullptr && c.ctx->d_look != nullptr);
+            if (!c.ctx->d_build) EXPECT(hipMalloc(&c.ctx->d_build, c.ctx->build_bytes = 200 * kMb) == hipSuccess);
+            fake::state().device_limit = fake::state().device_bytes + left;
+        };
+        room(0);
+        const int refused = call();
+        if (refused) std::printf("call %d: %s\n", (int)(&call - calls), prt_hip_last_error(c));
+        EXPECT(refused == 0);
+        EXPECT(hipGetLastError() == hipSuccess);
+        // the frames go on, with the lookahead from its beginning
+        fake::state().device_limit = ~size_t(0);
+        if (!c.ctx->scene.bvh_ready) EXPECT(prt_hip_bvh_build(c, nullptr) == 0);
+        EXPECT(prt_hip_frame_clear(c) == 0);
+        int runs = 0;
+        for (int k = 0; k < 12; ++k) {
+            EXPECT(prt_hip_render(c, PRT_RENDERER_DIFFUSE2, 6, 0.8f, nullptr) == 0);
+            if (g_paths.look) EXPECT(g_look_valid == (runs++ > 0));
+        }
+        EXPECT(runs >= 3);
+    }
+    // the lookahead's own buffers take the scratch's room
+    EXPECT(prt_hip_frame_init(c, 512, 512) == 0);
+    for (int k = 0; k < 2; ++k) EXPECT(prt_hip_render(c, PRT_RENDERER_DIFFUSE2, 6, 0.8f, nullptr) == 0);
+    EXPECT(prt_hip_frame_init(c, 640, 480) == 0);
+    if (!c.ctx->d_build) EXPECT(hipMalloc(&c.ctx->d_build, c.ctx->build_bytes = 200 * kMb) == hipSuccess);
+    fake::state().device_limit = fake::state().device_bytes;
+    for (int k = 0; k < 6; ++k) EXPECT(prt_hip_render(c, PRT_RENDERER_DIFFUSE2, 6, 0.8f, nullptr) == 0);
+    EXPECT(g_paths.look != nullptr && c.ctx->d_build == nullptr);
+    // refused all the same, and nothing of it left to the next call
+    fake::state().device_limit = fake::state().device_bytes;
+    EXPECT(prt_hip_frame_init(c, 16384, 16384) != 0);
+    EXPECT(std::string(prt_hip_last_error(c)).find("out of memory") != std::string::npos);
+    EXPECT(hipGetLastError() == hipSuccess);
+    fake::state().device_limit = ~size_t(0);
+}
+
 const struct {
     const char* name;
     void (*run)();
@@ -407,6 +487,7 @@ const struct {
     {"work_deal", work_deal},
     {"no_room_for_the_lookahead", no_room_for_the_lookahead},
     {"replaced_buffers", replaced_buffers},
+    {"kept_memory", kept_memory},
 };
 
 }  // namespace

@@ -31,6 +31,7 @@ def exe(tmp_path_factory):
     "work_deal",
     "no_room_for_the_lookahead",
     "replaced_buffers",
+    "kept_memory",
 ])
 def test_host_path(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
