@@ -73,7 +73,11 @@ hipError_t launch_look_call_begin(prt_hip_ctx*, bool valid, uint32_t)
     return hipGetLastError();
 }
 hipError_t launch_paths_rgb(prt_hip_ctx*, const PathLaunch&, bool) { return hipSuccess; }
-hipError_t launch_adjoint(prt_hip_ctx*, const PathLaunch&, bool) { return hipSuccess; }
+hipError_t launch_adjoint(prt_hip_ctx*, const PathLaunch& p, bool)
+{
+    g_paths = p;
+    return hipGetLastError();
+}
 const BatchKernelConfig kBatchVariants[kBatchVariantCount] = {{256, 16}, {256, 8}, {128, 16}, {128, 8}};
 hipError_t launch_batch(prt_hip_ctx*, const BatchLaunch&, const BatchTuning&, bool, int* max_blocks_per_cu)
 {
@@ -359,6 +363,33 @@ void no_room_for_the_lookahead()
         }
 }
 
+// The adjoint runs where its hit record finds no room (its paths are traced again
+// instead), with the record again once there is, and never beyond the depth that
+// is recorded.
+void no_room_for_the_hit_record()
+{
+    Context c;
+    with_scene(c);
+    prt_camera cam{};
+    cam.focal_distance = 1.0f;
+    EXPECT(prt_hip_camera_set(c, &cam) == 0);
+    EXPECT(prt_hip_frame_init(c, 64, 64) == 0);
+    const float rgb[3] = {0.5f, 0.5f, 0.5f};
+    EXPECT(prt_hip_set_albedo_host(c, rgb) == 0);
+    std::vector<float> dldi(3 * 64 * 64, 1.0f), grad(3, 0.0f);
+    const int64_t lanes = (int64_t)c.ctx->trace_grid * kTraceBlock;
+    for (int depth : {0, 1, 6, 64, 65, 6}) {
+        fake::state().device_limit = fake::state().device_bytes;
+        EXPECT(prt_hip_adjoint_albedo(c, 0, 1, depth, dldi.data(), grad.data(), nullptr) == 0);
+        const bool kept = c.ctx->path_hits_cap >= lanes * std::max(1, depth);
+        EXPECT((g_paths.path_hits != nullptr) == (kept && depth <= 64));
+        fake::state().device_limit = ~size_t(0);
+        EXPECT(prt_hip_adjoint_albedo(c, 0, 1, depth, dldi.data(), grad.data(), nullptr) == 0);
+        EXPECT((g_paths.path_hits != nullptr) == (depth <= 64));
+        EXPECT(depth > 64 || (g_paths.path_hits_stride == lanes && c.ctx->path_hits_cap >= lanes * depth));
+    }
+}
+
 // Memory that a job set or a scene needs and the one before it gives up is there
 // for it: a device that holds either holds one after the other.
 void replaced_buffers()
@@ -489,6 +520,7 @@ const struct {
     {"copy_threads", copy_threads},
     {"work_deal", work_deal},
     {"no_room_for_the_lookahead", no_room_for_the_lookahead},
+    {"no_room_for_the_hit_record", no_room_for_the_hit_record},
     {"replaced_buffers", replaced_buffers},
     {"kept_memory", kept_memory},
 };

@@ -30,6 +30,7 @@ def exe(tmp_path_factory):
     "copy_threads",
     "work_deal",
     "no_room_for_the_lookahead",
+    "no_room_for_the_hit_record",
     "replaced_buffers",
     "kept_memory",
 ])
