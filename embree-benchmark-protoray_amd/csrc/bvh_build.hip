@@ -351,10 +351,11 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint64_t* kin, c
 
 // All passes in one workgroup, which spares a small build 24 launches.  The same
 // stable passes: wave w owns the w-th part of the keys, ranks them as
-// k_radix_scatter does, and the keys move in LDS.  Build time in launches / in one
-// workgroup, us: 100 triangles 137 / 93, 1000 175 / 127, 2000 218 / 170, 4000
-// 238 / 201, 6000 255 / 227, 8202 265 / 253, 10000 268 / 262, 12288 274 / 279: a
-// pass of one workgroup takes 1 us and 1 us per 1000 keys.
+// k_radix_scatter does, and the keys move in LDS.  8192 keys are what its registers
+// and LDS hold, and where the gain has shrunk: a pass of one workgroup takes 1 us
+// and 1 us per 1000 keys.  Build time in launches / in one workgroup, us: 100
+// triangles 162 / 99, 1000 189 / 127, 2000 243 / 181, 4000 262 / 204, 6000 269 /
+// 227, 8192 281 / 249.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallItems = 8;  // most keys per thread
 constexpr int kSmallSort = kSmallThreads * kSmallItems;

@@ -152,7 +152,8 @@ __global__ __launch_bounds__(kBlock) void k_look_call_begin(uint32_t* work, uint
 
 // One bounce of the diffuse integrator for every queued ray: misses add the
 // path throughput, hits at the final depth add 0, other hits append the
-// bounced ray to the next queue (one atomic per wave, slots by lane prefix).
+// bounced ray to the next queue (one atomic per block, slots by wave and lane
+// prefix).
 __global__ __launch_bounds__(kBlock) void k_shade_diffuse(const float4* rays_in, const float4* hits,
                                                           const int32_t* pix_in, const uint32_t* rng_in,
                                                           const uint32_t* count_ptr, float4* rays_out,

@@ -273,7 +273,8 @@ int prt_hip_set_tail(prt_hip_ctx* ctx, int mode);
  * drops it).  The first call after any change (diffuse2: the first two; frames
  * of more than 640 k path slots: the first seven) renders as without the
  * lookahead.  The accumulator after each call and its ray count are those of rendering the
- * frames one by one.  Off for the primary and Fast renderers, the wavefront
+ * frames one by one.  Where its buffers find no room, frames render without it
+ * until the next prt_hip_frame_init or prt_hip_set_lookahead.  Off for the primary and Fast renderers, the wavefront
  * pipeline and under PRT_PROFILE_COUNTERS. */
 int prt_hip_set_lookahead(prt_hip_ctx* ctx, int enable);
 
@@ -308,7 +309,10 @@ int prt_hip_render_albedo_image_host(prt_hip_ctx* ctx, int pass0, int spp, int m
  * replay reads the hits that the trace recorded (one triangle index per bounce
  * of the paths in flight), or, for max_depth > 64, traces the path again from
  * its sampler seed (pass, pixelId).  rays in out_stats counts the rays of the
- * traces and of the replays. */
+ * traces and of the replays, whichever way a path is replayed: a replay from the
+ * record counts, in rays and in mray, as many as it spares.  The rays of the
+ * traces alone are those of prt_hip_render_albedo_image (less the paths whose
+ * dldi is 0). */
 int prt_hip_adjoint_albedo(prt_hip_ctx* ctx, int pass0, int spp, int max_depth, const float* d_dldi,
                            float* d_grad, prt_render_stats* out_stats);
 int prt_hip_adjoint_albedo_host(prt_hip_ctx* ctx, int pass0, int spp, int max_depth, const float* dldi,
