@@ -379,8 +379,9 @@ struct DirectIo {
     };
 };
 
-// The query can go this way; lays out the pinned buffer.  Where the system gives
-// none, small queries are copied as large ones are.
+// The query can go this way.  Its buffer is the copies' ring, which is idle
+// between them; where the system gives no pinned memory, small queries are copied
+// as large ones are.
 bool query_direct(prt_hip_ctx* ctx, int64_t n)
 {
     static_assert(kDirectRays <= (int64_t)kSpreadRays, "small queries are spread");
@@ -388,18 +389,15 @@ bool query_direct(prt_hip_ctx* ctx, int64_t n)
     if (!ctx->scene.bvh_ready || !ctx->tail_coop || n > kDirectRays ||
         !spread_covers(spread_grid(ctx->num_cus, (uint64_t)n, kBlockWaves, ctx->trace_grid), kBlockWaves, (uint64_t)n))
         return false;
-    if (!ctx->h_direct && hipHostMalloc(&ctx->h_direct, sizeof(DirectIo), hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->h_direct = nullptr;
-    }
-    return ctx->h_direct != nullptr;
+    return ctx->copy.prepare();
 }
 
 // hits or any_t: closest or any hit
 int run_direct(prt_hip_ctx* ctx, const prt_ray* rays, prt_hit* hits, float* any_t, int64_t n)
 {
     if (ensure_trace_resources(ctx)) return 1;
-    DirectIo* io = static_cast<DirectIo*>(ctx->h_direct);
+    static_assert(sizeof(DirectIo) <= HostCopy::kRingBytes, "room in the ring");
+    DirectIo* io = static_cast<DirectIo*>(ctx->copy.ring());
     io->err = 0;
     std::memcpy(io->rays, rays, sizeof(prt_ray) * (size_t)n);
     TraceLaunch t{};
@@ -495,7 +493,6 @@ int prt_hip_destroy(prt_hip_ctx* ctx)
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->h_readback) (void)hipHostFree(ctx->h_readback);
-    if (ctx->h_direct) (void)hipHostFree(ctx->h_direct);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return 0;

@@ -73,10 +73,14 @@ public:
     hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
     hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t s);
     Workers& workers() { return workers_; }
-
-private:
+    // The ring, kRingBytes of pinned memory, once prepare has laid it out.  Between
+    // two copies it is the caller's.
+    void* ring() { return ring_; }
     static constexpr int kSlots = 6;
     static constexpr size_t kChunk = size_t(2) << 20;
+    static constexpr size_t kRingBytes = kSlots * kChunk;
+
+private:
     static constexpr size_t kAskBytes = size_t(64) << 10;  // a smaller copy gains less than the question costs
     struct Slot {
         void* to;
@@ -88,7 +92,7 @@ private:
     void hand(int slot, void* to, const void* from, size_t bytes);
     Workers workers_;
     Slot slots_[kSlots];
-    char* ring_ = nullptr;          // kSlots * kChunk, pinned
+    char* ring_ = nullptr;          // kRingBytes, pinned
     hipEvent_t ev_[kSlots] = {};    // last DMA of each slot
     bool refused_ = false;          // no ring: the system gave no pinned memory
 };

@@ -112,7 +112,7 @@ bool HostCopy::prepare()
 {
     if (refused_) return false;
     if (!ring_ &&
-        hipHostMalloc(reinterpret_cast<void**>(&ring_), kSlots * kChunk, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc(reinterpret_cast<void**>(&ring_), kRingBytes, hipHostMallocDefault) != hipSuccess) {
         ring_ = nullptr;
         refused_ = true;
     }

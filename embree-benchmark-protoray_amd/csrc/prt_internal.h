@@ -235,7 +235,6 @@ struct prt_hip_ctx {
     float4* d_io_rays = nullptr;
     float4* d_io_hits = nullptr;
     int64_t io_cap = 0;
-    void* h_direct = nullptr;                 // pinned rays and hits of small host queries
     prt::HostCopy copy;                       // copies from and to pageable memory
 
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

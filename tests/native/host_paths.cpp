@@ -161,6 +161,31 @@ void small_query_on_small_devices()
         }
 }
 
+// A small query needs no pinned memory beside what the context laid out when it
+// was made, and leaves the copies that use the same memory as they were.
+void small_query_memory()
+{
+    Context c;
+    with_scene(c);
+    const int pinned = fake::state().pinned_calls;
+    EXPECT(prt_hip_frame_init(c, 700, 700) == 0);
+    std::vector<float> image((size_t)4 * 700 * 700);
+    for (int64_t n : {1, 32768, 300000, 5}) {
+        std::vector<prt_ray> rays(n);
+        for (int64_t k = 0; k < n; ++k) reinterpret_cast<float*>(&rays[k])[0] = 2.0f + (float)k;
+        std::vector<prt_hit> hits(n);
+        std::vector<float> any(n);
+        EXPECT(prt_hip_intersect_closest(c, rays.data(), hits.data(), n) == 0);
+        EXPECT(prt_hip_occluded(c, rays.data(), any.data(), n) == 0);
+        for (int64_t k : {(int64_t)0, n / 2, n - 1})
+            EXPECT(reinterpret_cast<const float*>(&hits[k])[0] == 2.0f + (float)k && any[k] == 2.0f + (float)k);
+        std::fill(image.begin(), image.end(), -1.0f);
+        EXPECT(prt_hip_accum_read(c, image.data()) == 0);
+        EXPECT(*std::min_element(image.begin(), image.end()) == 0.0f && *std::max_element(image.begin(), image.end()) == 0.0f);
+    }
+    EXPECT(fake::state().pinned_calls == pinned);
+}
+
 // A count that no query accepts is refused before anything is copied.
 void bad_ray_counts()
 {
@@ -513,6 +538,7 @@ const struct {
     void (*run)();
 } kChecks[] = {
     {"small_query_on_small_devices", small_query_on_small_devices},
+    {"small_query_memory", small_query_memory},
     {"bad_ray_counts", bad_ray_counts},
     {"no_pinned_memory", no_pinned_memory},
     {"host_copies", host_copies},

@@ -23,6 +23,7 @@ def exe(tmp_path_factory):
 
 @pytest.mark.parametrize("name", [
     "small_query_on_small_devices",
+    "small_query_memory",
     "bad_ray_counts",
     "no_pinned_memory",
     "host_copies",
