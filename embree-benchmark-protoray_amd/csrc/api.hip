@@ -754,9 +754,10 @@ int prt_hip_frame_init(prt_hip_ctx* ctx, int width, int height)
     ctx->look_refused = false;
     ctx->width = width;
     ctx->height = height;
-    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_accum, sizeof(float4) * (int64_t)width * height));
-    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_bgr8, sizeof(int32_t) * (int64_t)width * height));
     if (ensure_queues(ctx, frame_entries(ctx))) return 1;
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_bgr8, sizeof(int32_t) * (int64_t)width * height));
+    // last: a frame with an accumulator has all of its buffers
+    PRT_TRY(ctx, device_alloc(ctx, &ctx->d_accum, sizeof(float4) * (int64_t)width * height));
     return prt_hip_frame_clear(ctx);
 }
 

@@ -388,6 +388,31 @@ void no_room_for_the_lookahead()
         }
 }
 
+// A frame that finds no room for one of its buffers is none: what needs it is
+// refused until there is one.
+void half_a_frame()
+{
+    Context c;
+    with_scene(c);
+    prt_camera cam{};
+    cam.focal_distance = 1.0f;
+    EXPECT(prt_hip_camera_set(c, &cam) == 0);
+    std::vector<float> image(4 * 512 * 512);
+    std::vector<int32_t> pixels(512 * 512);
+    for (size_t room : {(size_t)0, (size_t)5 << 20, (size_t)8 << 20, (size_t)20 << 20}) {  // none, image, pixels, some queues
+        fake::state().device_limit = fake::state().device_bytes + room;
+        EXPECT(prt_hip_frame_init(c, 512, 512) != 0);
+        EXPECT(prt_hip_frame_clear(c) != 0);
+        EXPECT(prt_hip_render(c, PRT_RENDERER_DIFFUSE, 6, 0.8f, nullptr) != 0);
+        EXPECT(prt_hip_accum_read(c, image.data()) != 0);
+        EXPECT(prt_hip_frame_read_bgr8(c, pixels.data()) != 0);
+        fake::state().device_limit = ~size_t(0);
+    }
+    EXPECT(prt_hip_frame_init(c, 512, 512) == 0);
+    EXPECT(prt_hip_render(c, PRT_RENDERER_DIFFUSE, 6, 0.8f, nullptr) == 0);
+    EXPECT(prt_hip_frame_read_bgr8(c, pixels.data()) == 0);
+}
+
 // The adjoint runs where its hit record finds no room (its paths are traced again
 // instead), with the record again once there is, and never beyond the depth that
 // is recorded.
@@ -547,6 +572,7 @@ const struct {
     {"work_deal", work_deal},
     {"no_room_for_the_lookahead", no_room_for_the_lookahead},
     {"no_room_for_the_hit_record", no_room_for_the_hit_record},
+    {"half_a_frame", half_a_frame},
     {"replaced_buffers", replaced_buffers},
     {"kept_memory", kept_memory},
 };

@@ -32,6 +32,7 @@ def exe(tmp_path_factory):
     "work_deal",
     "no_room_for_the_lookahead",
     "no_room_for_the_hit_record",
+    "half_a_frame",
     "replaced_buffers",
     "kept_memory",
 ])
